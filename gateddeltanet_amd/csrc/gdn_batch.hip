@@ -48,6 +48,7 @@
 #include "gdn_amd.h"
 #include "gdn_device.h"
 #include "gdn_internal.h"
+#include "gdn_scan.h"
 
 namespace gdn {
 namespace bt {
@@ -1041,154 +1042,32 @@ __global__ __launch_bounds__(kT) void k_pqk(const float *__restrict__ qkv, int n
     if (t < kQkTok && m0 + t < n) alpha_out[(m0 + t) * kNH + h] = (red2[t][0] + red2[t][1]) + (red2[t][2] + red2[t][3]);
 }
 
-// The recurrence over a segment's n_total tokens in order, chunk by chunk of
-// 64, one launch per layer, one wave per pair of state columns and no
-// workgroup barrier inside a chunk's token loop: grid (kHD / kScanWgCols,
-// kNH), four independent waves per workgroup (one per SIMD, one workgroup
-// per CU; a wave64 add holds its SIMD whatever its active lanes, so two
-// chain waves on one SIMD would take turns).  The state stays in registers
-// from the first chunk to the last, and the next chunk's k, q, v, beta,
-// decay and alpha are loaded into registers during the current token loop.
-// Lane l holds rows 4 l .. 4 l + 3 of the wave's columns c0, c0 + 1 (one
-// 16-byte LDS access per chain row piece).  Per token: every lane writes its
-// products S[j][c] * kn[j] and S[j][c] * qn[j] to the wave's LDS rows; lanes
-// 0..3 sum the chains (r of c0, r of c0 + 1, p of c0, p of c0 + 1) in row
-// order j = 0..255 (the reference's chain order, adds only); the four sums
-// and the token's v, beta, decay, alpha (held in lane m) are read across
-// the wave, and every lane forms delta, o and its updated elements.  Each
-// chunk's normalised k and q (2 x 64 x 256 FP32) are staged in LDS once.
-// Each value is formed as the decode step's k_brecur forms it.
-constexpr int kScanWgCols = 8;  // 4 waves x 2 columns
+// The recurrence over a segment's n_total tokens in token order, one launch
+// per layer: grid (kHD / kScanWgCols, kNH), scan_block with the normalised
+// q and k of k_pqk.  Each value is formed as the decode step's k_brecur forms
+// it.
+struct SegScalars {
+    const float *bd, *alpha;  // [token][16] beta, decay per head; [token][kNH]
+    int h;
+    __device__ __forceinline__ f32x4 get(int m) const {
+        return (f32x4){bd[m * 16 + 2 * h], bd[m * 16 + 2 * h + 1], alpha[m * kNH + h], 0.0f};
+    }
+};
 __global__ __launch_bounds__(kT) void k_pscan(const float *__restrict__ qkv, const float *__restrict__ qn_seg,
                                                const float *__restrict__ kn_seg, const float *__restrict__ alpha_seg,
                                                const float *__restrict__ bd_seg, int n_total, float *__restrict__ state,
                                                float *__restrict__ attn_seg) {
-    constexpr int kPad = kHD + 4;  // chain rows 16 bytes apart in bank
-    constexpr int KQ = kMaxB * 2 * (kHD / 4) / kT;  // staged 16-byte pieces per thread and chunk
-    __shared__ __attribute__((aligned(16))) float kqs[kMaxB][2][kHD];  // [token][k|q][row]
-    __shared__ __attribute__((aligned(16))) float prod[4][4 * kPad];   // [wave][chain][row]
-    const int h = blockIdx.y, t = threadIdx.x, w = t >> 6, lane = t & 63;
-    const int c0 = blockIdx.x * kScanWgCols + 2 * w;
-    const int chunks = (n_total + kMaxB - 1) / kMaxB;
-    auto chunk_len = [&](int c) { return n_total - kMaxB * c < kMaxB ? n_total - kMaxB * c : kMaxB; };
-    // chunk c's normalised k and q (piece i = t + kT j: token, k|q, 4-row
-    // group) and, in lane m, token m's v of both columns, beta, decay and
-    // alpha: loaded into registers a chunk ahead
-    f32x4 kq[KQ];
-    float v0 = 0.0f, v1 = 0.0f, beta_l = 0.0f, decay_l = 0.0f, alpha_l = 0.0f;
-    auto load_chunk = [&](int c) __attribute__((always_inline)) {
-        const int n = chunk_len(c);
-        const size_t mb = (size_t)c * kMaxB;
-#pragma unroll
-        for (int j = 0; j < KQ; ++j) {
-            const int i = t + kT * j, m = i / (2 * (kHD / 4)), rest = i - m * 2 * (kHD / 4),
-                      kind = rest / (kHD / 4), r4 = rest - kind * (kHD / 4);
-            const float *src = (kind == 0 ? kn_seg : qn_seg) + (mb + m) * kH + h * kHD + 4 * r4;
-            kq[j] = m < n ? *reinterpret_cast<const f32x4 *>(src) : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        }
-        if (lane < n) {
-            const float *vp = qkv + ((mb + lane) * 3 + 2) * kH + h * kHD + c0;
-            v0 = vp[0];
-            v1 = vp[1];
-            beta_l = bd_seg[(mb + lane) * 16 + 2 * h];
-            decay_l = bd_seg[(mb + lane) * 16 + 2 * h + 1];
-            alpha_l = alpha_seg[(mb + lane) * kNH + h];
-        }
-    };
-    float *S = state + (size_t)h * kHD * kHD + c0;
-    float sv[2][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float2 s2 = *reinterpret_cast<const float2 *>(S + (size_t)(4 * lane + i) * kHD);
-        sv[0][i] = s2.x;
-        sv[1][i] = s2.y;
-    }
-    load_chunk(0);
-    float *pw = prod[w];
-    for (int c = 0; c < chunks; ++c) {
-        const int n = chunk_len(c);
-        float *attn = attn_seg + (size_t)c * kMaxB * kH;
-#pragma unroll
-        for (int j = 0; j < KQ; ++j) {
-            const int i = t + kT * j, m = i / (2 * (kHD / 4)), rest = i - m * 2 * (kHD / 4), kind = rest / (kHD / 4),
-                      r4 = rest - kind * (kHD / 4);
-            *reinterpret_cast<f32x4 *>(&kqs[m][kind][4 * r4]) = kq[j];
-        }
-        // this chunk's per-token scalars, held through its token loop
-        const float cv0 = v0, cv1 = v1, cbeta = beta_l, cdecay = decay_l, calpha = alpha_l;
-        __syncthreads();
-        if (c + 1 < chunks) load_chunk(c + 1);
-        f32x4 k4n = *reinterpret_cast<const f32x4 *>(&kqs[0][0][4 * lane]);
-        f32x4 q4n = *reinterpret_cast<const f32x4 *>(&kqs[0][1][4 * lane]);
-        for (int m = 0; m < n; ++m) {
-            const f32x4 k4 = k4n, q4 = q4n;
-            const float kn[4] = {k4.x, k4.y, k4.z, k4.w};
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                *reinterpret_cast<f32x4 *>(pw + e * kPad + 4 * lane) =
-                    (f32x4){sv[e][0] * k4.x, sv[e][1] * k4.y, sv[e][2] * k4.z, sv[e][3] * k4.w};
-                *reinterpret_cast<f32x4 *>(pw + (2 + e) * kPad + 4 * lane) =
-                    (f32x4){sv[e][0] * q4.x, sv[e][1] * q4.y, sv[e][2] * q4.z, sv[e][3] * q4.w};
-            }
-            // the wave's own LDS writes, then its reads of other lanes' rows
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            {
-                // the next token's k and q, read while the chains run
-                const int mn = m + 1 < n ? m + 1 : m;
-                k4n = *reinterpret_cast<const f32x4 *>(&kqs[mn][0][4 * lane]);
-                q4n = *reinterpret_cast<const f32x4 *>(&kqs[mn][1][4 * lane]);
-            }
-            float acc = 0.0f;
-            if (lane < 4) {
-                const f32x4 *col = reinterpret_cast<const f32x4 *>(pw + lane * kPad);
-                f32x4 cur[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) cur[j] = col[j];
-#pragma unroll
-                for (int b = 0; b < kHD / 32; ++b) {
-                    f32x4 nxt[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) nxt[j] = (b + 1 < kHD / 32) ? col[8 * (b + 1) + j] : cur[j];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) acc = (((acc + cur[j].x) + cur[j].y) + cur[j].z) + cur[j].w;
-                    asm volatile("" : "+v"(acc) : : "memory");
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) cur[j] = nxt[j];
-                }
-            }
-            const float ra = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 0));
-            const float rb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 1));
-            const float pa = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 2));
-            const float pb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 3));
-            const float beta = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cbeta), m));
-            const float decay = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cdecay), m));
-            const float alpha = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(calpha), m));
-            const float va = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cv0), m));
-            const float vb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cv1), m));
-            const float da = beta * (va - decay * ra);
-            const float db = beta * (vb - decay * rb);
-            if (lane < 2) {
-                const float o = lane == 0 ? 0.0625f * (decay * pa + alpha * da) : 0.0625f * (decay * pb + alpha * db);
-                attn[(size_t)m * kH + h * kHD + c0 + lane] = rne_bf16(o);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                sv[0][i] = decay * sv[0][i] + kn[i] * da;
-                sv[1][i] = decay * sv[1][i] + kn[i] * db;
-            }
-            // the next token's products overwrite the rows the chains just read
-            __builtin_amdgcn_wave_barrier();
-        }
-        // every wave is done with this chunk's rows before the next are stored
-        __syncthreads();
-    }
-    float *Sw = S;
-    asm volatile("" : "+v"(Sw));
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<float2 *>(Sw + (size_t)(4 * lane + i) * kHD) = make_float2(sv[0][i], sv[1][i]);
+    __shared__ ScanLds lds;
+    const int h = blockIdx.y, c0 = blockIdx.x * kScanWgCols;
+    ScanArgs a;
+    a.k = kn_seg + h * kHD;
+    a.q = qn_seg + h * kHD;
+    a.v = qkv + 2 * kH + h * kHD + c0;
+    a.o = attn_seg + h * kHD + c0;
+    a.ldq = a.ldo = kH;
+    a.ldv = 3 * kH;
+    a.n = n_total;
+    scan_block<kBf16w, false>(a, SegScalars{bd_seg, alpha_seg, h}, state + (size_t)h * kHD * kHD + c0, lds);
 }
 
 // ---------------------------------------------------- chunked prefill (WY form)

@@ -422,6 +422,28 @@ def test_prefill_long_segment_equals_steps(n):
         m.free()
 
 
+@pytest.mark.parametrize("n", [15, 16, 17, 31, 32, 33, 48, 49])
+def test_prefill_scan_chunk_edges(n):
+    """The scan stages 16 tokens at a time in two buffers: prompts that end
+    one token before, at and after a chunk's end, with an even and an odd
+    number of chunks, equal single-stream steps bit for bit."""
+    m = g.Model.synth(num_layers=1, seed=3, std=0.02, bf16=True)
+    prompt = g.synth_tokens(n, 21, 5)
+    pre, ref = g.BatchState(m, 1), g.BatchState(m, 1)
+    try:
+        seed = pre.prefill(0, prompt)
+        for t in prompt:
+            nxt = ref.step([int(t)])
+        assert seed == int(nxt[0])
+        for a, b in zip(pre.save_stream_state(0), ref.save_stream_state(0)):
+            assert same_bits(a, b)
+        assert same_bits(pre.logits(0), ref.logits(0))
+    finally:
+        pre.free()
+        ref.free()
+        m.free()
+
+
 def test_prefill_continues_a_decoded_stream(model):
     """A prefill on a stream that has already decoded tokens continues from
     its state and conv tails: 5 steps then a 70-token prefill equal 75
