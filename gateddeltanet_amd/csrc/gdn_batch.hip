@@ -1081,7 +1081,7 @@ __global__ __launch_bounds__(kT) void k_pscan(const float *__restrict__ qkv, con
 //   Mq[m][s] = exp(G_m - G_s) (q_m . k_s)             s <= m
 //   delta_m  = beta_m (v_m - exp(G_m) S^T k_m) - sum_{s<m} L[m][s] delta_s,
 //              i.e. delta = T b with T = (I + L)^-1 (formed per chunk by
-//              k_wy_inv, chunk.py's solve of the same triangular system)
+//              k_wy_prep, chunk.py's solve of the same triangular system)
 //   o_m      = (exp(G_m) S^T q_m + sum_{s<=m} Mq[m][s] delta_s) / 16
 //   S'       = exp(G_{n-1}) S + sum_s exp(G_{n-1} - G_s) k_s delta_s^T
 // which is the per-token recurrence of the decode step unrolled over the
@@ -1090,392 +1090,480 @@ __global__ __launch_bounds__(kT) void k_pscan(const float *__restrict__ qkv, con
 // sequential chains, so this mode matches the scan within a tolerance, not
 // bit for bit; o is rounded to BF16 as the step rounds it.
 
-// L and Mq of one head for rows 16 blockIdx.y .. +15 of chunk blockIdx.z of
-// a segment of n_total tokens: grid (kNH, kMaxB / 16, chunks).
-constexpr int kKp = kHD / 4 + 1;  // padded float4 stride of a staged k/q row
+//
+// q and k are BF16 values before their normalisation, so every product with
+// them runs on the BF16 matrix cores without loss: k_m . k_s and q_m . k_s
+// as they are, with the two inverse norms as factors of the sum, and
+// products with an FP32 operand (the state, the deltas) after that operand
+// is split into three BF16 terms whose sum it is (8 + 8 + 8 significand
+// bits).  v_mfma_f32_16x16x32_bf16 forms exact products and FP32 sums at
+// 16 times the rate of v_mfma_f32_16x16x4_f32, so three (or, between two
+// split operands, six) of them still take a fifth (three eighths) of its
+// time.
 
-// The chunk's rows of one head ([token][kH] FP32, head h's 256 values),
-// held in registers between the load and the store into LDS rows of stride
-// kKp float4 (zeros from token n on).  The loads of every staged operand
-// are issued at the kernel's start, so their latencies overlap instead of
-// adding up.
-struct RowStage {
-    static constexpr int PER = kMaxB * (kHD / 4) / kT;
-    f32x4 v[PER];
-    __device__ __forceinline__ void load(const float *__restrict__ src, int h, int n) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = threadIdx.x + kT * i, m = idx / (kHD / 4), j4 = idx % (kHD / 4);
-            v[i] = m < n ? *reinterpret_cast<const f32x4 *>(src + (size_t)m * kH + h * kHD + 4 * j4)
-                         : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    }
-    __device__ __forceinline__ void store(f32x4 (*rows)[kKp]) const {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = threadIdx.x + kT * i;
-            rows[idx / (kHD / 4)][idx % (kHD / 4)] = v[i];
-        }
-    }
-};
-
-// One head's 64 x 64 matrix, stored into LDS rows of stride kMaxB + 4.
-struct MatStage {
-    static constexpr int PER = kMaxB * kMaxB / 4 / kT;
-    f32x4 v[PER];
-    __device__ __forceinline__ void load(const float *__restrict__ src) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) v[i] = reinterpret_cast<const f32x4 *>(src)[threadIdx.x + kT * i];
-    }
-    __device__ __forceinline__ void store(float (*dst)[kMaxB + 4]) const {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int q = threadIdx.x + kT * i;
-            *reinterpret_cast<f32x4 *>(&dst[q / (kMaxB / 4)][4 * (q % (kMaxB / 4))]) = v[i];
-        }
-    }
-};
-__device__ __forceinline__ float cum_log_decay(const float *__restrict__ bd, int h, int n, float *glog) {
-    // lanes 0..63 of wave 0: inclusive prefix sum of log(decay) over the chunk
-    const int lane = threadIdx.x;
-    // (a decay that underflowed to 0 is taken as 1e-30: the products it
-    // enters are 0 to FP32 either way, and G stays finite)
-    float v = lane < n ? __logf(fmaxf(bd[lane * 16 + 2 * h + 1], 1e-30f)) : 0.0f;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const float o = __shfl_up(v, d);
-        if (lane >= d) v += o;
-    }
-    glog[lane] = v;
-    return v;
+__device__ __forceinline__ f32x4 mfma_bf16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                   0, 0, 0);
 }
 
-__global__ __launch_bounds__(kT) void k_wy_gram(const float *__restrict__ qn_seg, const float *__restrict__ kn_seg,
-                                                const float *__restrict__ bd_seg, int n_total,
-                                                float *__restrict__ L_seg, float *__restrict__ M_seg) {
-    const int ch = blockIdx.z, n = n_total - kMaxB * ch < kMaxB ? n_total - kMaxB * ch : kMaxB;
-    const float *qn_all = qn_seg + (size_t)ch * kMaxB * kH, *kn_all = kn_seg + (size_t)ch * kMaxB * kH;
-    const float *bd = bd_seg + (size_t)ch * kMaxB * 16;
-    float *Lout = L_seg + (size_t)ch * kNH * kMaxB * kMaxB, *Mout = M_seg + (size_t)ch * kNH * kMaxB * kMaxB;
-    __shared__ f32x4 ks[kMaxB][kKp];
-    __shared__ f32x4 qr[16][kKp];
-    __shared__ float glog[kMaxB];
-    const int h = blockIdx.x, r0 = 16 * blockIdx.y, t = threadIdx.x, w = t >> 6, lane = t & 63;
+// x as three BF16 terms: p[0] + p[1] + p[2] = x (each rounded to nearest, the
+// differences exact), four values packed in two words.
+__device__ __forceinline__ void split3(const f32x4 x, u32x2 (&p)[3]) {
+    f32x4 r = x;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        p[i].x = cvt_pk(r.x, r.y);
+        p[i].y = cvt_pk(r.z, r.w);
+        if (i < 2) {
+            r.x = r.x - u2f(p[i].x << 16);
+            r.y = r.y - u2f(p[i].x & 0xffff0000u);
+            r.z = r.z - u2f(p[i].y << 16);
+            r.w = r.w - u2f(p[i].y & 0xffff0000u);
+        }
+    }
+}
+
+// The product of two split operands over one 32-wide k step, smallest terms
+// first (the three terms below 2^-24 of the product are left out).
+__device__ __forceinline__ f32x4 mfma_split(const u32x4 (&a)[3], const u32x4 (&b)[3], f32x4 c) {
+    c = mfma_bf16(a[2], b[0], c);
+    c = mfma_bf16(a[0], b[2], c);
+    c = mfma_bf16(a[1], b[1], c);
+    c = mfma_bf16(a[1], b[0], c);
+    c = mfma_bf16(a[0], b[1], c);
+    return mfma_bf16(a[0], b[0], c);
+}
+
+// One (chunk, head)'s operands of k_wy_seq, written by k_wy_prep: MFMA A
+// fragments (64 lanes x 8 BF16 values, 1 KB), grouped by the wave that reads
+// them.
+//   kf, qf  [wave w][16-token tile][k step t]: token 16 tile + l % 16, keys
+//           64 w + 32 t + 4 (l / 16) + {0..3, 16..19} (the keys a lane of
+//           k_wy_seq holds of the state, so the state is the B operand as
+//           it lies in registers)
+//   ktf     [w][16-key tile][t]: key 64 w + 16 tile + l % 16, tokens
+//           32 t + 8 (l / 16) .. + 7
+//   tf, mf  [w][t][term]: T and Mq, row 16 w + l % 16, columns
+//           32 t + 8 (l / 16) .. + 7, the three BF16 terms
+//   sc      [token]: exp(G_m) / |k_m|, beta_m, exp(G_m) / |q_m|,
+//           exp(G_{n-1} - G_m) / |k_m|
+//   dn      exp(G_{n-1})
+struct WyOps {
+    u32x4 kf[4][4][2][64], qf[4][4][2][64], ktf[4][4][2][64];
+    u32x4 tf[4][2][3][64], mf[4][2][3][64];
+    f32x4 sc[kMaxB];
+    float dn, pad[3];
+};
+static_assert(sizeof(WyOps) % 16 == 0, "16-byte fragments of every (chunk, head)");
+
+// The operands of one (head, chunk): grid (kNH, chunks).  q and k come as
+// the conv left them ([token][3][kH], BF16 values); each row is scaled by a
+// power of two to the size of a unit vector (exact, so the sums of raw
+// products cannot overflow where the normalised ones would not) and that
+// power is taken back in its inverse norm.  T = (I + L)^-1 is formed in 16 x
+// 16 blocks: the diagonal blocks by forward substitution (a lane per column),
+// then T[I][J] = -T[I][I] sum_{J <= K < I} L[I][K] T[K][J] by distance from
+// the diagonal on v_mfma_f32_16x16x4_f32.  One wave substituting all 64 rows
+// took 24 us a launch; with the norms (k_pqk) and the FP32 gram kernel this
+// launch replaces, 108 us per layer of a 4096-token prefill.
+constexpr int kWyRow = kHD + 8;    // padded BF16 row of a token (528 bytes)
+constexpr int kWyMat = kMaxB + 4;  // padded FP32 row of a chunk matrix
+__global__ __launch_bounds__(kT) void k_wy_prep(const float *__restrict__ qkv_seg, const float *__restrict__ bd_seg,
+                                                int n_total, WyOps *__restrict__ ops_seg) {
+    constexpr int kRows = kMaxB * kWyRow * 2, kMats = 2 * kMaxB * kWyMat * 4;
+    // q rows, later L and Mq; k rows, later T
+    __shared__ __attribute__((aligned(16))) unsigned char mem_q[kMats > kRows ? kMats : kRows];
+    __shared__ __attribute__((aligned(16))) unsigned char mem_k[kRows];
+    __shared__ double glog[kMaxB];
+    __shared__ float ikn[kMaxB], iqn[kMaxB], bet[kMaxB];
+    uint16_t(*qr)[kWyRow] = reinterpret_cast<uint16_t(*)[kWyRow]>(mem_q);
+    uint16_t(*kr)[kWyRow] = reinterpret_cast<uint16_t(*)[kWyRow]>(mem_k);
+    float(*lm)[kWyMat] = reinterpret_cast<float(*)[kWyMat]>(mem_q);
+    float(*mm)[kWyMat] = lm + kMaxB;
+    float(*tm)[kWyMat] = reinterpret_cast<float(*)[kWyMat]>(mem_k);
+    static_assert(kMaxB * kWyMat * 4 <= kRows, "T fits the k rows");
+    const int h = blockIdx.x, ch = blockIdx.y, t = threadIdx.x, w = t >> 6, lane = t & 63;
     const int li = lane & 15, kk = lane >> 4;
-    RowStage kst;
-    kst.load(kn_all, h, n);
-    {
-        // this block's 16 q rows (zeros from token n on)
-        constexpr int PER = 16 * (kHD / 4) / kT;
-        f32x4 v[PER];
+    const int n = n_total - kMaxB * ch < kMaxB ? n_total - kMaxB * ch : kMaxB;
+    const float *qkv = qkv_seg + (size_t)ch * kMaxB * 3 * kH + h * kHD + 4 * lane;
+    const float *bd = bd_seg + (size_t)ch * kMaxB * 16;
+    WyOps &ops = ops_seg[(size_t)ch * kNH + h];
+
+    // wave w: tokens 16 w .. + 15, four channels per lane; a token past the
+    // chunk's end re-reads its last one and is stored as zeros
+    f32x4 x[2][16];
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = t + kT * i, r = idx / (kHD / 4), j4 = idx % (kHD / 4);
-            v[i] = (r0 + r < n) ? *reinterpret_cast<const f32x4 *>(qn_all + (size_t)(r0 + r) * kH + h * kHD + 4 * j4)
-                                : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 16; ++i) {
+        const int m = 16 * w + i < n ? 16 * w + i : n - 1;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) x[j][i] = *reinterpret_cast<const f32x4 *>(qkv + ((size_t)m * 3 + j) * kH);
+    }
+    if (t < kMaxB) {
+        // G: inclusive prefix sum of log(decay) over the chunk (a decay that
+        // underflowed to 0 is taken as 1e-30: the products it enters are 0
+        // to FP32 either way, and G stays finite).  In FP64: the weights are
+        // exponentials of differences of G, whose FP32 rounding alone was
+        // most of this mode's distance from the scan.
+        double v = t < n ? log((double)fmaxf(bd[t * 16 + 2 * h + 1], 1e-30f)) : 0.0;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const double o = __shfl_up(v, d);
+            if (lane >= d) v += o;
         }
+        glog[t] = v;
+        bet[t] = t < n ? bd[t * 16 + 2 * h] : 0.0f;
+    }
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = t + kT * i;
-            qr[idx / (kHD / 4)][idx % (kHD / 4)] = v[i];
+    for (int i = 0; i < 16; ++i) {
+        const int m = 16 * w + i;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const f32x4 v = x[j][i];
+            // 1 / |x| in gdn_tree_reduce_256's order, as the scan has it
+            const float sq = wave_tree64((v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w));
+            const float inv = 1.0f / __builtin_sqrtf(sq + 1e-6f);
+            // 2^e of 1 / |x|; both factors normal numbers
+            uint32_t e = f2u(inv) & 0x7f800000u;
+            e = e < 0x01000000u ? 0x01000000u : e;
+            const float up = u2f(e), down = u2f(0x7f000000u - e);
+            u32x2 pk;
+            pk.x = cvt_pk(v.x * up, v.y * up);
+            pk.y = cvt_pk(v.z * up, v.w * up);
+            if (m >= n) pk = (u32x2){0u, 0u};
+            *reinterpret_cast<u32x2 *>(&(j ? kr : qr)[m][4 * lane]) = pk;
+            if (lane == 0) (j ? ikn : iqn)[m] = inv * down;
         }
     }
-    kst.store(ks);
-    if (t < 64) cum_log_decay(bd, h, n, glog);
     __syncthreads();
-    // wave w: columns s = 16 w .. +15 of rows r0 .. r0 + 15: K_m . K_s and
-    // Q_m . K_s on v_mfma_f32_16x16x4_f32 (component q of a lane's 16-byte
-    // read feeds the q-th MFMA of its group, for A and B alike)
-    f32x4 kk0 = {0.0f, 0.0f, 0.0f, 0.0f}, kk1 = kk0, qk0 = kk0, qk1 = kk0;
-#pragma unroll
-    for (int g = 0; g < kHD / 16; ++g) {
-        const f32x4 ka = ks[r0 + li][4 * g + kk];
-        const f32x4 qa = qr[li][4 * g + kk];
-        const f32x4 kb = ks[16 * w + li][4 * g + kk];
-        kk0 = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.x, kb.x, kk0, 0, 0, 0);
-        qk0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.x, kb.x, qk0, 0, 0, 0);
-        kk1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.y, kb.y, kk1, 0, 0, 0);
-        qk1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.y, kb.y, qk1, 0, 0, 0);
-        kk0 = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.z, kb.z, kk0, 0, 0, 0);
-        qk0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.z, kb.z, qk0, 0, 0, 0);
-        kk1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.w, kb.w, kk1, 0, 0, 0);
-        qk1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.w, kb.w, qk1, 0, 0, 0);
+    if (t < kMaxB) {
+        const float g = __expf((float)glog[t]);
+        ops.sc[t] = (f32x4){g * ikn[t], bet[t], g * iqn[t], __expf((float)(glog[n - 1] - glog[t])) * ikn[t]};
+        if (t == 0) ops.dn = __expf((float)glog[n - 1]);
     }
-    const f32x4 gk4 = kk0 + kk1, gq4 = qk0 + qk1;
-    const int sidx = 16 * w + li;
+    // A fragments for k_wy_seq's wave w
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int m = r0 + 4 * kk + r;
-        float lv = 0.0f, mv = 0.0f;
-        if (m < n && sidx <= m) {
-            const float ratio = __expf(glog[m] - glog[sidx]);
-            if (sidx < m) lv = bd[m * 16 + 2 * h] * ratio * gk4[r];
-            mv = ratio * gq4[r];
+    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int key = 64 * w + 32 * ks + 4 * kk;
+            const u32x2 k0 = *reinterpret_cast<const u32x2 *>(&kr[16 * mt + li][key]);
+            const u32x2 k1 = *reinterpret_cast<const u32x2 *>(&kr[16 * mt + li][key + 16]);
+            ops.kf[w][mt][ks][lane] = (u32x4){k0.x, k0.y, k1.x, k1.y};
+            const u32x2 q0 = *reinterpret_cast<const u32x2 *>(&qr[16 * mt + li][key]);
+            const u32x2 q1 = *reinterpret_cast<const u32x2 *>(&qr[16 * mt + li][key + 16]);
+            ops.qf[w][mt][ks][lane] = (u32x4){q0.x, q0.y, q1.x, q1.y};
+            uint32_t kt[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) kt[e] = kr[32 * ks + 8 * kk + e][64 * w + 16 * mt + li];
+            ops.ktf[w][mt][ks][lane] = (u32x4){kt[0] | (kt[1] << 16), kt[2] | (kt[3] << 16), kt[4] | (kt[5] << 16),
+                                               kt[6] | (kt[7] << 16)};
         }
-        Lout[((size_t)h * kMaxB + m) * kMaxB + sidx] = lv;
-        Mout[((size_t)h * kMaxB + m) * kMaxB + sidx] = mv;
+    // rows 16 w .. + 15 of K K^T and Q K^T, the tiles on or below the diagonal
+    f32x4 gk[4], gq[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) gk[s] = gq[s] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int g = 0; g < kHD / 32; ++g) {
+        const u32x4 ka = *reinterpret_cast<const u32x4 *>(&kr[16 * w + li][32 * g + 8 * kk]);
+        const u32x4 qa = *reinterpret_cast<const u32x4 *>(&qr[16 * w + li][32 * g + 8 * kk]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (s <= w) {
+                const u32x4 kb = *reinterpret_cast<const u32x4 *>(&kr[16 * s + li][32 * g + 8 * kk]);
+                gk[s] = mfma_bf16(ka, kb, gk[s]);
+                gq[s] = mfma_bf16(qa, kb, gq[s]);
+            }
     }
-}
-
-// T = (I + L)^-1 of one (head, chunk), in place of L: grid (kNH, chunks),
-// one wave.  Lane j forms column j by forward substitution in row order,
-// T[m][j] = [m == j] - sum_{s<m} L[m][s] T[s][j] (s ascending), so the
-// chunk's deltas (I + L) delta = b become one matrix product, delta = T b,
-// off the sequential path.  Rows of L from the chunk's length on are zero,
-// so T is the identity there.
-__global__ __launch_bounds__(64) void k_wy_inv(float *__restrict__ L_seg) {
-    __shared__ __attribute__((aligned(16))) float ls[kMaxB][kMaxB];
-    const int h = blockIdx.x, ch = blockIdx.y, j = threadIdx.x;
-    float *lp = L_seg + ((size_t)ch * kNH + h) * kMaxB * kMaxB;
-#pragma unroll 8
-    for (int m = 0; m < kMaxB; ++m) ls[m][j] = lp[m * kMaxB + j];
-    __syncthreads();
-    // every row runs over all 64 columns (constant bounds, so the column
-    // stays in registers): L[m][s] is exactly zero for s >= m and tc[s] is
-    // still zero there, so those terms add exact zeros after the real ones
-    float tc[kMaxB];
+    __syncthreads();  // q and k rows read; L, Mq and T take their place
 #pragma unroll
-    for (int m = 0; m < kMaxB; ++m) tc[m] = 0.0f;
-#pragma unroll
-    for (int m = 0; m < kMaxB; ++m) {
-        float acc = m == j ? 1.0f : 0.0f;
-#pragma unroll
-        for (int s4 = 0; s4 < kMaxB; s4 += 4) {
-            const f32x4 lv = *reinterpret_cast<const f32x4 *>(&ls[m][s4]);
-            acc = __builtin_fmaf(-lv.x, tc[s4], acc);
-            acc = __builtin_fmaf(-lv.y, tc[s4 + 1], acc);
-            acc = __builtin_fmaf(-lv.z, tc[s4 + 2], acc);
-            acc = __builtin_fmaf(-lv.w, tc[s4 + 3], acc);
-        }
-        tc[m] = acc;
-    }
-#pragma unroll
-    for (int m = 0; m < kMaxB; ++m) lp[m * kMaxB + j] = tc[m];
-}
-
-// One head's recurrence over a segment's chunks for 16 state columns: grid
-// (kHD / kWyCols, kNH), 256 threads, the state tile held in LDS from the
-// first chunk to the last and each chunk's operands loaded into registers
-// while the previous chunk computes.  The matrix products run on
-// v_mfma_f32_16x16x4_f32 (FP32 operands and sums; this form is held to a
-// tolerance, not to the step's rounding): Q S and K S (wave w: rows 16 w ..
-// +15 of the chunk, all 256 keys), the deltas T b and o (wave w: rows 16 w
-// .. +15) and the state update (wave w: state rows 64 w .. +63).  An MFMA takes A[i][k] from lane i + 16 k and
-// B[k][j] from lane j + 16 k and leaves D[4 (l / 16) + r][l % 16] in
-// component r of lane l.  A lane reads 4 consecutive k values of its row
-// (or column) in one 16-byte LDS read and feeds them to 4 MFMAs, component
-// q to the q-th, so MFMA q of a group sums the k = 4 (4 g + kk) + q; A and B
-// use the same assignment.
-constexpr int kWyCols = 16;
-constexpr int kS0p = kHD + 4;    // padded key stride of the transposed state tile
-constexpr int kDtp = kMaxB + 4;  // padded token stride of the transposed deltas
-
-__global__ __launch_bounds__(kT) void k_wy_seq(const float *__restrict__ qkv, const float *__restrict__ qn_seg,
-                                               const float *__restrict__ kn_seg, const float *__restrict__ bd_seg,
-                                               const float *__restrict__ T_seg, const float *__restrict__ M_seg,
-                                               int n_total, float *__restrict__ state, float *__restrict__ attn) {
-    __shared__ f32x4 rows[kMaxB][kKp];                                   // Q, then K
-    __shared__ __attribute__((aligned(16))) float s0t[kWyCols][kS0p];    // state tile, [column][key]
-    __shared__ __attribute__((aligned(16))) float lm[kMaxB][kMaxB + 4];  // T, then Mq
-    __shared__ float qs[kMaxB][kWyCols + 1];                             // S^T q
-    __shared__ __attribute__((aligned(16))) float bt[kWyCols][kDtp];     // b, [column][token]
-    __shared__ __attribute__((aligned(16))) float dlt[kWyCols][kDtp];    // delta, [column][token]
-    __shared__ __attribute__((aligned(16))) float dft[kWyCols][kDtp];    // exp(G_{n-1} - G_s) delta_s
-    __shared__ float glog[kMaxB], fdec[kMaxB];
-    const int h = blockIdx.y, c0 = blockIdx.x * kWyCols, t = threadIdx.x, w = t >> 6, lane = t & 63;
-    const int li = lane & 15, kk = lane >> 4;  // MFMA operand row/column, k quarter
-    const int chunks = (n_total + kMaxB - 1) / kMaxB;
-    const size_t mat = (size_t)kNH * kMaxB * kMaxB;  // one chunk's L (or Mq), every head
-    float *S = state + (size_t)h * kHD * kHD + c0;
-    auto chunk_len = [&](int c) { return n_total - kMaxB * c < kMaxB ? n_total - kMaxB * c : kMaxB; };
-    // the operands of chunk c into registers (issued a chunk ahead)
-    RowStage qst, kst;
-    MatStage lst, mst;
-    float vv[4], beta[4], dec = 1.0f;
-    auto load_vb = [&](int c) __attribute__((always_inline)) {
-        const int n = chunk_len(c);
-        const size_t m0 = (size_t)c * kMaxB;
-        // v and beta of this lane's D elements of K S: rows 16 w + 4 kk + r, column li
+    for (int s = 0; s < 4; ++s) {
+        const int c = 16 * s + li;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = 16 * w + 4 * kk + r;
-            vv[r] = m < n ? qkv[((m0 + m) * 3 + 2) * kH + h * kHD + c0 + li] : 0.0f;
-            beta[r] = m < n ? bd_seg[(m0 + m) * 16 + 2 * h] : 0.0f;
-        }
-        dec = lane < n ? bd_seg[(m0 + lane) * 16 + 2 * h + 1] : 1.0f;
-    };
-    qst.load(qn_seg, h, chunk_len(0));
-    lst.load(T_seg + (size_t)h * kMaxB * kMaxB);
-    kst.load(kn_seg, h, chunk_len(0));
-    mst.load(M_seg + (size_t)h * kMaxB * kMaxB);
-    load_vb(0);
-    {
-        const f32x4 *src = reinterpret_cast<const f32x4 *>(S + (size_t)t * kHD);
-        f32x4 v[kWyCols / 4];
-#pragma unroll
-        for (int i = 0; i < kWyCols / 4; ++i) v[i] = src[i];
-#pragma unroll
-        for (int i = 0; i < kWyCols / 4; ++i) {
-            s0t[4 * i][t] = v[i].x;
-            s0t[4 * i + 1][t] = v[i].y;
-            s0t[4 * i + 2][t] = v[i].z;
-            s0t[4 * i + 3][t] = v[i].w;
+            float lv = 0.0f, mv = 0.0f;
+            if (m < n && c <= m) {
+                const float ratio = __expf((float)(glog[m] - glog[c])) * ikn[c];
+                if (c < m) lv = bet[m] * (ratio * ikn[m]) * gk[s][r];
+                mv = (ratio * iqn[m]) * gq[s][r];
+            }
+            lm[m][c] = lv;
+            mm[m][c] = mv;
+            tm[m][c] = 0.0f;
         }
     }
-
-    // X S for the staged rows X (Q, then K): rows 16 w .. +15, 256 keys
-    const auto xs_mfma = [&]() __attribute__((always_inline)) {
-        f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
+    __syncthreads();
+    auto write_terms = [&](const float(*src)[kWyMat], u32x4(&dst)[4][2][3][64], int tile) {
 #pragma unroll
-        for (int g = 0; g < kHD / 16; ++g) {
-            const f32x4 xa = rows[16 * w + li][4 * g + kk];
-            const f32x4 xb = *reinterpret_cast<const f32x4 *>(&s0t[li][16 * g + 4 * kk]);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.x, xb.x, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.y, xb.y, acc1, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.z, xb.z, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.w, xb.w, acc1, 0, 0, 0);
+        for (int ks = 0; ks < 2; ++ks) {
+            u32x2 a[3], b[3];
+            split3(*reinterpret_cast<const f32x4 *>(&src[16 * tile + li][32 * ks + 8 * kk]), a);
+            split3(*reinterpret_cast<const f32x4 *>(&src[16 * tile + li][32 * ks + 8 * kk + 4]), b);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) dst[tile][ks][p][lane] = (u32x4){a[p].x, a[p].y, b[p].x, b[p].y};
         }
-        return acc0 + acc1;
     };
-
-    for (int c = 0; c < chunks; ++c) {
-        const int n = chunk_len(c);
-        const bool more = c + 1 < chunks;
-        const size_t m0 = (size_t)c * kMaxB, m1 = m0 + kMaxB;
-        qst.store(rows);
-        lst.store(lm);
-        if (more) {
-            qst.load(qn_seg + m1 * kH, h, chunk_len(c + 1));
-            lst.load(T_seg + (c + 1) * mat + (size_t)h * kMaxB * kMaxB);
-        }
-        if (t < 64) {
-            // inclusive prefix sum of log(decay) over the chunk (a decay that
-            // underflowed to 0 is taken as 1e-30: the products it enters are 0
-            // to FP32 either way, and G stays finite)
-            float v = lane < n ? __logf(fmaxf(dec, 1e-30f)) : 0.0f;
+    if (w == 0) {
+        // lane 16 B + j: column j of the inverse of diagonal block B
+        const int b0 = 16 * kk;
+        float tc[16];
 #pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const float o = __shfl_up(v, d);
-                if (lane >= d) v += o;
+        for (int m = 0; m < 16; ++m) {
+            float acc = m == li ? 1.0f : 0.0f;
+#pragma unroll
+            for (int s4 = 0; s4 < (m + 3) / 4; ++s4) {
+                const f32x4 lv = *reinterpret_cast<const f32x4 *>(&lm[b0 + m][b0 + 4 * s4]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (4 * s4 + e < m) acc = __builtin_fmaf(lv[e], -tc[4 * s4 + e], acc);
             }
-            glog[lane] = v;
+            tc[m] = acc;
         }
-        __syncthreads();
-        if (t < kMaxB) fdec[t] = __expf(glog[n - 1] - glog[t]);
-
-        // S^T q for every token
-        {
-            const f32x4 d = xs_mfma();
 #pragma unroll
-            for (int r = 0; r < 4; ++r) qs[16 * w + 4 * kk + r][li] = d[r];
-        }
-        __syncthreads();
-        kst.store(rows);
-        if (more) kst.load(kn_seg + m1 * kH, h, chunk_len(c + 1));
-        __syncthreads();
-        // S^T k for every token, then b_m = beta_m (v_m - exp(G_m) S^T k_m)
-        {
-            const f32x4 d = xs_mfma();
-            f32x4 b;
+        for (int m = 0; m < 16; ++m) tm[b0 + m][b0 + li] = tc[m];
+    } else {
+        write_terms(mm, ops.mf, w);
+        if (w == 1) write_terms(mm, ops.mf, 0);
+    }
+    __syncthreads();
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = 16 * w + 4 * kk + r;
-                b[r] = m < n ? beta[r] * (vv[r] - __expf(glog[m]) * d[r]) : 0.0f;
+    for (int d = 1; d < 4; ++d) {
+        if (w + d < 4) {
+            const int I = w + d, J = w;
+            f32x4 y = {0.0f, 0.0f, 0.0f, 0.0f}, z = y;
+            for (int K = J; K < I; ++K) {
+                const f32x4 a = *reinterpret_cast<const f32x4 *>(&lm[16 * I + li][16 * K + 4 * kk]);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], tm[16 * K + 4 * kk + q][16 * J + li], y, 0, 0, 0);
             }
-            *reinterpret_cast<f32x4 *>(&bt[li][16 * w + 4 * kk]) = b;
+            // y's rows 4 kk + r are the B operand's k = 4 kk + q as they lie
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(&tm[16 * I + li][16 * I + 4 * kk]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) z = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], y[q], z, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) tm[16 * I + 4 * kk + r][16 * J + li] = -z[r];
         }
-        __syncthreads();
-        if (more) load_vb(c + 1);
-
-        // delta = T b: rows 16 w .. +15 (zero from row n on, where b is
-        // zero and T the identity), transposed for the MFMA B operands and
-        // scaled by their decay for the state update
-        {
-            f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
-#pragma unroll
-            for (int g = 0; g < kMaxB / 16; ++g) {
-                const f32x4 xa = *reinterpret_cast<const f32x4 *>(&lm[16 * w + li][16 * g + 4 * kk]);
-                const f32x4 xb = *reinterpret_cast<const f32x4 *>(&bt[li][16 * g + 4 * kk]);
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.x, xb.x, acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.y, xb.y, acc1, 0, 0, 0);
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.z, xb.z, acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.w, xb.w, acc1, 0, 0, 0);
-            }
-            const f32x4 d = acc0 + acc1;
-            const int m = 16 * w + 4 * kk;
-            *reinterpret_cast<f32x4 *>(&dlt[li][m]) = d;
-            *reinterpret_cast<f32x4 *>(&dft[li][m]) =
-                (f32x4){fdec[m] * d[0], fdec[m + 1] * d[1], fdec[m + 2] * d[2], fdec[m + 3] * d[3]};
-        }
-        __syncthreads();
-        mst.store(lm);
-        if (more) mst.load(M_seg + (c + 1) * mat + (size_t)h * kMaxB * kMaxB);
-        __syncthreads();
-
-        // o_m = (exp(G_m) S^T q_m + sum_{s<=m} Mq[m][s] delta_s) / 16,
-        // rounded: rows 16 w .. +15
-        {
-            f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
-#pragma unroll
-            for (int g = 0; g < kMaxB / 16; ++g) {
-                const f32x4 xa = *reinterpret_cast<const f32x4 *>(&lm[16 * w + li][16 * g + 4 * kk]);
-                const f32x4 xb = *reinterpret_cast<const f32x4 *>(&dlt[li][16 * g + 4 * kk]);
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.x, xb.x, acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.y, xb.y, acc1, 0, 0, 0);
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.z, xb.z, acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.w, xb.w, acc1, 0, 0, 0);
-            }
-            const f32x4 d = acc0 + acc1;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = 16 * w + 4 * kk + r;
-                if (m < n) {
-                    const float o = __expf(glog[m]) * qs[m][li] + d[r];
-                    attn[(m0 + m) * kH + h * kHD + c0 + li] = rne_bf16(0.0625f * o);
-                }
-            }
-        }
-
-        // S' = exp(G_{n-1}) S + sum_s exp(G_{n-1} - G_s) k_s delta_s^T:
-        // state rows 64 w .. +63 as four 16-row tiles; A[j][s] = k_s[j]
-        // (token rows of the staged K), B[s][c] = exp(G_{n-1} - G_s)
-        // delta_s[c].  Each element is read and rewritten in place by the
-        // lane that owns it.
-        {
-            const float dn = __expf(glog[n - 1]);
-            const float *krow = reinterpret_cast<const float *>(&rows[0][0]);
-#pragma unroll
-            for (int tile = 0; tile < 4; ++tile) {
-                const int j0 = 64 * w + 16 * tile;
-                f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
-#pragma unroll
-                for (int g = 0; g < kMaxB / 16; ++g) {
-                    const int sb = 16 * g + 4 * kk;  // this lane's 4 tokens
-                    const f32x4 xb = *reinterpret_cast<const f32x4 *>(&dft[li][sb]);
-                    const float a0 = krow[(sb + 0) * (4 * kKp) + j0 + li];
-                    const float a1 = krow[(sb + 1) * (4 * kKp) + j0 + li];
-                    const float a2 = krow[(sb + 2) * (4 * kKp) + j0 + li];
-                    const float a3 = krow[(sb + 3) * (4 * kKp) + j0 + li];
-                    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, xb.x, acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, xb.y, acc1, 0, 0, 0);
-                    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, xb.z, acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a3, xb.w, acc1, 0, 0, 0);
-                }
-                const f32x4 d = acc0 + acc1;
-                f32x4 *sp = reinterpret_cast<f32x4 *>(&s0t[li][j0 + 4 * kk]);
-                const f32x4 sv = *sp;
-                *sp = (f32x4){__builtin_fmaf(dn, sv[0], d[0]), __builtin_fmaf(dn, sv[1], d[1]),
-                              __builtin_fmaf(dn, sv[2], d[2]), __builtin_fmaf(dn, sv[3], d[3])};
-            }
-        }
-        // the next chunk overwrites rows, lm and the deltas
         __syncthreads();
     }
-    {
-        f32x4 *dst = reinterpret_cast<f32x4 *>(S + (size_t)t * kHD);
+    write_terms(tm, ops.tf, w);
+}
+
+// One head's recurrence over a segment's chunks for 16 state columns: grid
+// 8 x 16 workgroups of eight waves, workgroup b on head b % 8 (so an XCD's L2
+// serves one head's operands to its sixteen workgroups).
+// Waves 0..3, the sequential path: wave w holds state rows 64 w .. + 63 in
+// registers from the first chunk to the last, as the accumulator tiles of
+// its updates (lane l: rows 16 tile + 4 (l / 16) + r, column l % 16).  Per
+// chunk: its keys' share of K S for all 64 tokens, summed over the waves
+// through LDS; b = beta (v - exp(G) S^T k) for its 16 tokens; delta = T b;
+// S' = exp(G_{n-1}) S + sum_s k_s (exp(G_{n-1} - G_s) delta_s)^T on its rows.
+// Waves 4..7, beside them: the same keys' share of Q S (the state's terms
+// through LDS) and o for 16 tokens.
+// Three barriers a chunk.  Every operand but b, delta, the terms and the
+// partial sums comes straight from global memory into registers, a chunk
+// ahead.  What bounds it, from cycle stamps of each phase: the latencies of
+// the sequential path's three dependent products and their barriers (about
+// 4200 cycles a chunk), and the issue of the operand loads (about 1700: 128 KB
+// per CU and chunk against a SIMD's limit of some 16 loads in flight); with
+// the Q products, or two thirds of the state products, left out it ran only
+// 10 % shorter.  At 4096 tokens a launch takes 180 us (2.8 us a chunk), 192
+// with the o path on the same four waves, and 520 (8.0) in FP32 MFMAs with the
+// state and operands through LDS and seven barriers a chunk.
+constexpr int kWyCols = 16;
+constexpr int kWyTok = kMaxB + 8;  // padded token stride of b and delta (BF16)
+constexpr int kWyWaves = 8;
+
+struct WyLds {
+    f32x4 ksp[4][4][64], qsp[4][4][64];  // [wave][token tile][lane]
+    u32x4 sb[4][3][2][64];               // the state's terms: [wave][term][k step][lane]
+    uint16_t bt[3][kWyCols][kWyTok];     // b's terms, [column][token]
+    uint16_t dt[3][kWyCols][kWyTok];     // delta's
+    uint16_t ft[3][kWyCols][kWyTok];     // the scaled delta's
+};
+
+// part[i], component r: token 16 i + 4 (lane / 16) + r, column lane % 16
+__device__ __forceinline__ void wy_state_product(const u32x4 (&xf)[4][2], const u32x4 (&sb)[3][2], f32x4 (&part)[4]) {
 #pragma unroll
-        for (int i = 0; i < kWyCols / 4; ++i)
-            dst[i] = (f32x4){s0t[4 * i][t], s0t[4 * i + 1][t], s0t[4 * i + 2][t], s0t[4 * i + 3][t]};
+    for (int i = 0; i < 4; ++i) part[i] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part[i] = mfma_bf16(xf[i][ks], sb[p][ks], part[i]);
+}
+__device__ __forceinline__ void wy_read_terms(const uint16_t (&src)[3][kWyCols][kWyTok], int li, int kk,
+                                              u32x4 (&b)[2][3]) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+        b[i / 3][i % 3] = *reinterpret_cast<const u32x4 *>(&src[i % 3][li][32 * (i / 3) + 8 * kk]);
+}
+__device__ __forceinline__ void wy_write_terms(uint16_t (&dst)[3][kWyCols][kWyTok], int li, int tok, const f32x4 v) {
+    u32x2 p[3];
+    split3(v, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2 *>(&dst[i][li][tok]) = p[i];
+}
+__device__ __forceinline__ f32x4 wy_sum4(const f32x4 (&part)[4][4][64], int tile, int lane) {
+    return (part[0][tile][lane] + part[1][tile][lane]) + (part[2][tile][lane] + part[3][tile][lane]);
+}
+__device__ __forceinline__ void wy_load8(const u32x4 (&src)[4][2][64], int lane, u32x4 (&dst)[4][2]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[i >> 1][i & 1] = src[i >> 1][i & 1][lane];
+}
+__device__ __forceinline__ void wy_load6(const u32x4 (&src)[2][3][64], int lane, u32x4 (&dst)[2][3]) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) dst[i / 3][i % 3] = src[i / 3][i % 3][lane];
+}
+
+__global__ __launch_bounds__(kWyWaves * 64) void k_wy_seq(const float *__restrict__ qkv,
+                                                          const WyOps *__restrict__ ops_seg, int n_total,
+                                                          float *__restrict__ state, float *__restrict__ attn) {
+    __shared__ __attribute__((aligned(16))) WyLds lds;
+    const int h = blockIdx.x & 7, c0 = (blockIdx.x >> 3) * kWyCols;
+    const int t = threadIdx.x, w = (t >> 6) & 3, lane = t & 63, li = lane & 15, kk = lane >> 4;
+    const int tok = 16 * w + 4 * kk;  // this lane's four tokens of a chunk
+    const int chunks = (n_total + kMaxB - 1) / kMaxB;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto ops = [&](int c) -> const WyOps & { return ops_seg[(size_t)c * kNH + h]; };
+
+    if (t < 256) {
+        float *S = state + (size_t)h * kHD * kHD + (size_t)(64 * w + 4 * kk) * kHD + c0 + li;
+        const float *vp = qkv + 2 * kH + h * kHD + c0 + li;
+        u32x4 kf[4][2], ktf[4][2], tf[2][3];
+        f32x4 scn[4], st[4];
+        float vn[4], dnn;
+        auto load_sv = [&](int c) __attribute__((always_inline)) {
+            dnn = vector_load(&ops(c).dn);  // a scalar load's wait would also wait for LDS, and LDS's for it
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = kMaxB * c + tok + r;
+                scn[r] = ops(c).sc[tok + r];
+                vn[r] = vp[(size_t)(m < n_total ? m : n_total - 1) * 3 * kH];
+            }
+        };
+        load_sv(0);
+        wy_load8(ops(0).kf[w], lane, kf);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) st[i][r] = S[(size_t)(16 * i + r) * kHD];
+        wy_load6(ops(0).tf[w], lane, tf);
+        wy_load8(ops(0).ktf[w], lane, ktf);
+        for (int c = 0; c < chunks; ++c) {
+            // the next chunk's operands (the last chunk re-reads its own, unused)
+            const int cn = c + 1 < chunks ? c + 1 : c;
+            f32x4 sc[4], part[4];
+            float vv[4];
+            const float dn = dnn;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                sc[r] = scn[r];
+                vv[r] = vn[r];
+            }
+            load_sv(cn);
+            u32x4 sb[3][2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                u32x2 a[3], b[3];
+                split3(st[2 * ks], a);
+                split3(st[2 * ks + 1], b);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) sb[p][ks] = (u32x4){a[p].x, a[p].y, b[p].x, b[p].y};
+            }
+            wy_state_product(kf, sb, part);
+#pragma unroll
+            for (int i = 0; i < 6; ++i) lds.sb[w][i >> 1][i & 1][lane] = sb[i >> 1][i & 1];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lds.ksp[w][i][lane] = part[i];
+            wy_load8(ops(cn).kf[w], lane, kf);
+            __syncthreads();
+            {
+                const f32x4 d = wy_sum4(lds.ksp, w, lane);
+                f32x4 b;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) b[r] = sc[r].y * (vv[r] - sc[r].x * d[r]);
+                wy_write_terms(lds.bt, li, tok, b);
+            }
+            __syncthreads();
+            // delta = T b (T is the identity and b zero from the chunk's
+            // length on; T is zero above the diagonal, so the first two
+            // waves' second k step is)
+            {
+                u32x4 b[2][3];
+                wy_read_terms(lds.bt, li, kk, b);
+                f32x4 d = mfma_split(tf[0], b[0], zero);
+                if (w >= 2) d = mfma_split(tf[1], b[1], zero) + d;
+                wy_write_terms(lds.ft, li, tok,
+                               (f32x4){sc[0].w * d[0], sc[1].w * d[1], sc[2].w * d[2], sc[3].w * d[3]});
+                wy_write_terms(lds.dt, li, tok, d);
+                wy_load6(ops(cn).tf[w], lane, tf);
+            }
+            __syncthreads();
+            u32x4 f[2][3];
+            wy_read_terms(lds.ft, li, kk, f);
+            f32x4 up[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) up[i] = zero;
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) up[i] = mfma_bf16(ktf[i][ks], f[ks][p], up[i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) st[i][r] = __builtin_fmaf(dn, st[i][r], up[i][r]);
+            wy_load8(ops(cn).ktf[w], lane, ktf);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[(size_t)(16 * i + r) * kHD] = st[i][r];
+    } else {
+        float *op = attn + h * kHD + c0 + li;
+        u32x4 qf[4][2], mf[2][3];
+        float cq[4], cqn[4];
+        auto load_cq = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) cqn[r] = ops(c).sc[tok + r].z;
+        };
+        load_cq(0);
+        wy_load8(ops(0).qf[w], lane, qf);
+        wy_load6(ops(0).mf[w], lane, mf);
+        for (int c = 0; c < chunks; ++c) {
+            const int cn = c + 1 < chunks ? c + 1 : c;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) cq[r] = cqn[r];
+            load_cq(cn);
+            __syncthreads();
+            {
+                u32x4 sb[3][2];
+                f32x4 part[4];
+#pragma unroll
+                for (int i = 0; i < 6; ++i) sb[i >> 1][i & 1] = lds.sb[w][i >> 1][i & 1][lane];
+                wy_state_product(qf, sb, part);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) lds.qsp[w][i][lane] = part[i];
+                wy_load8(ops(cn).qf[w], lane, qf);
+            }
+            __syncthreads();
+            __syncthreads();
+            // o_m = (exp(G_m) S^T q_m + sum_{s<=m} Mq[m][s] delta_s) / 16, rounded
+            u32x4 b[2][3];
+            wy_read_terms(lds.dt, li, kk, b);
+            f32x4 d = mfma_split(mf[0], b[0], zero);
+            if (w >= 2) d = mfma_split(mf[1], b[1], zero) + d;
+            const f32x4 q = wy_sum4(lds.qsp, w, lane);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = kMaxB * c + tok + r;
+                if (m < n_total) op[(size_t)m * kH] = rne_bf16(0.0625f * (cq[r] * q[r] + d[r]));
+            }
+            wy_load6(ops(cn).mf[w], lane, mf);
+        }
     }
 }
 
@@ -1896,8 +1984,8 @@ struct GDNBatchEngine {
     int seg_tokens = kSegDefault, seg_cap = 0;
     void *seg_mem = nullptr;
     float *s_h = nullptr, *s_y = nullptr, *s_qkv = nullptr, *s_gate = nullptr, *s_sgate = nullptr, *s_bd = nullptr,
-          *s_attn = nullptr, *s_qn = nullptr, *s_kn = nullptr, *s_alpha = nullptr, *s_wyl = nullptr,
-          *s_wym = nullptr, *s_xn = nullptr;
+          *s_attn = nullptr, *s_qn = nullptr, *s_kn = nullptr, *s_alpha = nullptr, *s_xn = nullptr;
+    WyOps *s_wy = nullptr;
     uint16_t *s_xh = nullptr, *s_xo = nullptr, *s_xd = nullptr;
     int *s_tok = nullptr;
     hipGraph_t graph = nullptr;
@@ -2249,8 +2337,9 @@ int seg_alloc(GDNBatchEngine *e) {
     e->seg_mem = nullptr;
     e->seg_cap = 0;
     const size_t T = (size_t)e->seg_tokens, chunks = T / kMaxB;
-    const size_t floats = T * (2 * kH + 4 * kH + 3 * kH + kH + kH + 16 + kH + kH + kH + kNH + kH) +
-                          2 * chunks * kNH * kMaxB * kMaxB;
+    // normalised q and k (scan) or k_wy_seq's operands (chunked)
+    const size_t qk = std::max(T * 2 * kH, chunks * kNH * sizeof(WyOps) / sizeof(float));
+    const size_t floats = T * (2 * kH + 4 * kH + 3 * kH + kH + kH + 16 + kH + kNH + kH) + qk;
     const size_t halves = T * (kH + kH + kI);
     const size_t bytes = floats * 4 + halves * 2 + T * sizeof(int);
     GDN_HIP(hipMalloc(&e->seg_mem, bytes));
@@ -2267,12 +2356,12 @@ int seg_alloc(GDNBatchEngine *e) {
     e->s_sgate = p; p += T * kH;
     e->s_bd = p; p += T * 16;
     e->s_attn = p; p += T * kH;
-    e->s_qn = p; p += T * kH;
-    e->s_kn = p; p += T * kH;
+    e->s_qn = p;
+    e->s_kn = p + T * kH;
+    e->s_wy = reinterpret_cast<WyOps *>(p);
+    p += qk;
     e->s_alpha = p; p += T * kNH;
     e->s_xn = p; p += T * kH;
-    e->s_wyl = p; p += chunks * kNH * kMaxB * kMaxB;
-    e->s_wym = p; p += chunks * kNH * kMaxB * kMaxB;
     uint16_t *q = reinterpret_cast<uint16_t *>(p);
     e->s_xh = q; q += T * kH;
     e->s_xo = q; q += T * kH;
@@ -2308,8 +2397,8 @@ BNorm seg_norm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_ou
 // streams (k_pgemm / k_pgu in place of the step's GEMMs, k_bnorm + k_pab in
 // place of the split a/b norm; same sums), the conv across the segment
 // (k_pconv), and the recurrence chunk by chunk of 64 tokens, in token order
-// (k_pqk, k_pscan) or in the WY form (k_wy_gram and k_wy_inv over every
-// chunk at once, then k_wy_seq over the chunks in order).
+// (k_pqk, k_pscan) or in the WY form (k_wy_prep over every chunk at once,
+// then k_wy_seq over the chunks in order).
 // k_pgemm_a (the faster kernel once its grid fills the CUs) or k_pgemm (twice
 // the workgroups at the same size, so the better one on short segments):
 // the same sums either way.
@@ -2343,19 +2432,16 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
                                e->w_qkvg[l], xh, e->s_y, 4 * kH);
         hipLaunchKernelGGL(k_pconv, dim3(4 * kH / 64, blocks), dim3(kConvT), 0, s, e->s_y, n, tl,
                            b_aux(e, l) + kAuxConv, e->s_qkv, e->s_gate, e->s_sgate);
-        hipLaunchKernelGGL(k_pqk, dim3(kNH, (n + kQkTok - 1) / kQkTok), dim3(kT), 0, s, e->s_qkv, n, e->s_qn,
-                           e->s_kn, e->s_alpha);
-        if (e->prefill_mode == GDN_PREFILL_CHUNKED)
-            hipLaunchKernelGGL(k_wy_gram, dim3(kNH, kMaxB / 16, blocks), dim3(kT), 0, s, e->s_qn, e->s_kn, e->s_bd,
-                               n, e->s_wyl, e->s_wym);
-        if (e->prefill_mode == GDN_PREFILL_CHUNKED)
-            hipLaunchKernelGGL(k_wy_inv, dim3(kNH, blocks), dim3(64), 0, s, e->s_wyl);
-        if (e->prefill_mode == GDN_PREFILL_CHUNKED)
-            hipLaunchKernelGGL(k_wy_seq, dim3(kHD / kWyCols, kNH), dim3(kT), 0, s, e->s_qkv, e->s_qn, e->s_kn,
-                               e->s_bd, e->s_wyl, e->s_wym, n, st, e->s_attn);
-        else
+        if (e->prefill_mode == GDN_PREFILL_CHUNKED) {
+            hipLaunchKernelGGL(k_wy_prep, dim3(kNH, blocks), dim3(kT), 0, s, e->s_qkv, e->s_bd, n, e->s_wy);
+            hipLaunchKernelGGL(k_wy_seq, dim3(kNH * (kHD / kWyCols)), dim3(kWyWaves * 64), 0, s, e->s_qkv, e->s_wy, n, st,
+                               e->s_attn);
+        } else {
+            hipLaunchKernelGGL(k_pqk, dim3(kNH, (n + kQkTok - 1) / kQkTok), dim3(kT), 0, s, e->s_qkv, n, e->s_qn,
+                               e->s_kn, e->s_alpha);
             hipLaunchKernelGGL(k_pscan, dim3(kHD / kScanWgCols, kNH), dim3(kT), 0, s, e->s_qkv, e->s_qn, e->s_kn,
                                e->s_alpha, e->s_bd, n, st, e->s_attn);
+        }
         hipLaunchKernelGGL(k_bonorm<kOnTok>, dim3(kNH, (n + kOnTok - 1) / kOnTok), dim3(kT), 0, s, e->s_attn,
                            e->s_gate, e->s_sgate, b_aux(e, l) + kAuxONorm, e->eps, e->s_xo, n);
         hipLaunchKernelGGL((k_pgemm<kKtH, 4, kSplitO>), dim3(kH / 128, tiles), dim3(kPgW * 64), 0, s, e->w_o[l], xo,

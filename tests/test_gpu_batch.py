@@ -444,6 +444,30 @@ def test_prefill_scan_chunk_edges(n):
         m.free()
 
 
+@pytest.mark.parametrize("n", [1, 15, 17, 33, 63, 65, 127, 129, 192])
+def test_prefill_chunked_edges(n):
+    """The chunked recurrence at the edges of its 16-token blocks and 64-token
+    chunks (T's diagonal blocks, the zero rows from the prompt's end on): one
+    layer's state against the scan's.  Both sum the same FP32 products in
+    another order (a few roundings of 2^-24 on the way to each element); 5e-7
+    is four times the largest difference measured (1.2e-7)."""
+    m = g.Model.synth(num_layers=1, seed=4, std=0.02, bf16=True)
+    prompt = g.synth_tokens(n, 22, 6)
+    states = []
+    for mode in (g.PREFILL_SCAN, g.PREFILL_CHUNKED):
+        bs = g.BatchState(m, 1)
+        bs.set_prefill_mode(mode)
+        bs.prefill(0, prompt)
+        states.append(bs.save_stream_state(0))
+        bs.free()
+    m.free()
+    (scan, tails), (chunked, tails2) = states
+    assert same_bits(tails, tails2)
+    diff = np.linalg.norm(scan.astype(np.float64) - chunked) / np.linalg.norm(scan.astype(np.float64))
+    print(f"n {n}: state relative L2 {diff:.2e}")
+    assert diff < 5e-7
+
+
 def test_prefill_continues_a_decoded_stream(model):
     """A prefill on a stream that has already decoded tokens continues from
     its state and conv tails: 5 steps then a 70-token prefill equal 75
