@@ -404,9 +404,9 @@ int gdn_test_recurrence(int contract, uint32_t n_heads, uint32_t n_steps,
  * steps of gdn_test_recurrence on caller-owned DEVICE buffers, allocating
  * nothing.  Arguments and layouts as gdn_test_recurrence, all device
  * pointers, except S, which is in the engine's device format: [heads][256][256]
- * BF16 bits (uint16) for GDN_CONTRACT_REF, FP32 otherwise.  The per-step
- * (beta, decay) pairs live in a fixed 128 KiB device array of 16384 pairs that
- * every call on a GPU shares (steps run in chunks that fit it); n_heads above
+ * BF16 bits (uint16) for GDN_CONTRACT_REF, FP32 otherwise.  The scalars of a
+ * (step, head) live in a fixed 512 KiB device array of 16384 entries that every
+ * call on a GPU shares (steps run in chunks that fit it); n_heads above
  * 16384 is rejected.  Work is enqueued on `stream` (a hipStream_t; NULL = the
  * null stream) and not waited for.  Calls that overlap on one GPU race on the
  * shared array. */

@@ -67,12 +67,16 @@ def _to_device(hip, arr, keep):
     return p
 
 
-def _noalloc(contract, q, k, v, a, b, al, dt, S):
+def _noalloc(contract, q, k, v, a, b, al, dt, S, shift=0):
+    """shift: q and k at this many floats into their allocations."""
     hip = _hip()
     steps, heads = a.shape
     keep = []
     try:
-        ins = [_to_device(hip, np.ascontiguousarray(x, np.float32), keep) for x in (q, k, v, a, b, al, dt)]
+        pad = np.zeros(shift, np.float32)
+        ins = [_to_device(hip, np.concatenate([pad, np.ravel(x)]).astype(np.float32), keep) for x in (q, k)]
+        ins = [ctypes.c_void_p(p.value + 4 * shift) for p in ins]
+        ins += [_to_device(hip, np.ascontiguousarray(x, np.float32), keep) for x in (v, a, b, al, dt)]
         if contract == g.CONTRACT_REF:
             s_host = (S.view(np.uint32) >> 16).astype(np.uint16)
         else:
@@ -109,6 +113,44 @@ def test_noalloc_recurrence_matches_allocating_entry_point(contract):
         o, S2 = _noalloc(contract, q, k, v, a, b, al, dt, S)
         assert _same(o, o_ref), (contract, heads, steps)
         assert _same(S2, S_ref), (contract, heads, steps)
+
+
+# Step counts and head counts on both sides of the choice between one scan and
+# a launch per step (2 steps: 8 heads; 3: 96; 4), of the scan's 16-token
+# staging and of a scratch fill that leaves a chunk of one step (4 x 4097).
+@pytest.mark.parametrize("contract", [g.CONTRACT_BF16W_FP32S, g.CONTRACT_REF, g.CONTRACT_FP32])
+@pytest.mark.parametrize("heads,steps", [(1, 1), (8, 2), (9, 2), (96, 3), (97, 3), (97, 4), (3, 15), (3, 16), (3, 17),
+                                         (1, 33), (4097, 4)])
+def test_noalloc_recurrence_routes(contract, heads, steps):
+    q, k, v, a, b, al, dt, S = _inputs(7 * heads + steps, steps, heads, contract)
+    o_ref, S_ref = g.recurrence(contract, q, k, v, a, b, al, dt, S)
+    o, S2 = _noalloc(contract, q, k, v, a, b, al, dt, S)
+    assert _same(o, o_ref) and _same(S2, S_ref)
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_noalloc_recurrence_unaligned_q_and_k(shift):
+    """q and k at addresses that are not multiples of 16 bytes: the per-step
+    kernel's 4-byte loads."""
+    c = g.CONTRACT_BF16W_FP32S
+    q, k, v, a, b, al, dt, S = _inputs(5, 6, 4, c)
+    o_ref, S_ref = g.recurrence(c, q, k, v, a, b, al, dt, S)
+    o, S2 = _noalloc(c, q, k, v, a, b, al, dt, S, shift)
+    assert _same(o, o_ref) and _same(S2, S_ref)
+
+
+@pytest.mark.parametrize("contract", [g.CONTRACT_BF16W_FP32S, g.CONTRACT_REF, g.CONTRACT_FP32])
+def test_noalloc_recurrence_non_finite(contract):
+    """Infinities and NaNs in the state, q and v pass through the scan as
+    through the per-step kernel (NaNs compared as NaNs)."""
+    q, k, v, a, b, al, dt, S = _inputs(9, 20, 3, contract)
+    S[0, 5, 7], S[0, 9, 8], S[1, 200, 255] = np.inf, -np.inf, np.nan
+    q[3, 2, 17], v[4, 2, 40] = np.inf, np.nan
+    o_ref, S_ref = g.recurrence(contract, q, k, v, a, b, al, dt, S)
+    o, S2 = _noalloc(contract, q, k, v, a, b, al, dt, S)
+    assert np.isnan(o_ref).any() and not np.isnan(o_ref).all()
+    np.testing.assert_array_equal(o, o_ref)
+    np.testing.assert_array_equal(S2, S_ref)
 
 
 def test_noalloc_rejects_oversized_and_bad_arguments():
