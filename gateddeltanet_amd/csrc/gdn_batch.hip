@@ -101,7 +101,8 @@ __device__ __forceinline__ void store_x8(uint16_t *x, int m, int k, const float 
 struct BEpi {
     int n_streams;
     int n_rows;          // N: row stride of y / logits
-    float *y;            // EPI_RAW / EPI_STORE: [64][N]
+    float *y;            // EPI_RAW / EPI_STORE: [splits][y_rows][N]
+    int y_rows;          // rows of one split's plane (64 in a step)
     float *qkv;          // EPI_QKVG: [64][3][kH] after conv + SiLU
     float *gate;         // [64][kH] R(g)
     float *sgate;        // [64][kH] sigmoid(R(g))
@@ -118,7 +119,8 @@ struct BEpi {
 // keep up to four tiles of operands in flight, and the per-wave sums are
 // added in wave order through LDS; the epilogue then runs on the reduced
 // tile.  Split partial sums (EPI_RAW with S > 1) are added in split order by
-// the consumer.
+// the consumer.  With EPI_RAW the grid's z dimension is the 64-token block of
+// a prefill segment.
 template <int RT, int KT, int NW, int S, int EPI>
 __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                    BEpi ep) {
@@ -142,7 +144,8 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
     const int t = threadIdx.x, w = t >> 6, l = t & 63, sp = blockIdx.y;
     const int kt0 = sp * KTS + w;
     const u32x4 *wp = W + ((size_t)rb * KT + kt0) * (RT * 64) + l;
-    const u32x4 *xp = X + (size_t)kt0 * (4 * 64) + l;
+    const int zb = EPI == EPI_RAW ? (int)blockIdx.z : 0;
+    const u32x4 *xp = X + ((size_t)zb * KT + kt0) * (4 * 64) + l;
 
     // QKVG epilogue tasks: four consecutive channels of one stream per
     // thread and pass (4-channel group g of the workgroup's RT * 4, stream
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
                     o.z = rne_bf16(v.z);
                     o.w = rne_bf16(v.w);
                 }
-                *reinterpret_cast<f32x4 *>(ep.y + ((size_t)sp * 64 + m) * ep.n_rows + row) = o;
+                *reinterpret_cast<f32x4 *>(ep.y + ((size_t)sp * ep.y_rows + zb * 64 + m) * ep.n_rows + row) = o;
             }
         }
     } else if constexpr (EPI == EPI_QKVG) {
@@ -333,6 +336,7 @@ static_assert(kGuWgs * kGuCh == kI && kGuCh > 16 && kGuCh <= 24 && (kGuCh % 2) =
 template <int NW>
 __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                  uint16_t *__restrict__ x_next, int n_streams) {
+    // grid y: the 64-token block of a prefill segment of n_streams tokens
     constexpr int RT = 3, KT = kKtH, KTW = KT / NW, GT = NW * 64;
     static_assert(KT % NW == 0, "whole k tiles per wave");
     constexpr int D = KTW < 4 ? KTW : 4;
@@ -346,7 +350,8 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
     const bool p2 = (l & 15) < kGuTail2;
     const int o2 = 128 + (p2 ? (l >> 4) * kGuTail2 + (l & 15) : 0);
     const u32x4 *wp = W + ((size_t)rb * KT + w) * kGuTileU4;
-    const u32x4 *xp = X + (size_t)w * (4 * 64) + l;
+    const int mb = (int)blockIdx.y * kMaxB;
+    const u32x4 *xp = X + ((size_t)blockIdx.y * KT + w) * (4 * 64) + l;
     const u32x4 zero = {0u, 0u, 0u, 0u};
 
     f32x4 acc[RT][4];
@@ -409,16 +414,16 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
     // task (stream m, nq), thread 4 m + nq
     {
         const int m = t >> 2, nq = t & 3;
-        if (m < n_streams) {
+        if (mb + m < n_streams) {
             const f32x4 g = val4(0, nq, m), u = val4(1, nq, m);
             const uint32_t lo = swiglu(g.x, u.x) | (swiglu(g.y, u.y) << 16);
             const uint32_t hi = swiglu(g.z, u.z) | (swiglu(g.w, u.w) << 16);
             const int k0 = rb * kGuCh + 4 * nq;  // even: pairs never straddle an 8-column group
             if ((k0 & 3) == 0) {
-                *reinterpret_cast<uint2 *>(x_next + xt_index(m, k0, kI)) = make_uint2(lo, hi);
+                *reinterpret_cast<uint2 *>(x_next + xt_index(mb + m, k0, kI)) = make_uint2(lo, hi);
             } else {
-                *reinterpret_cast<uint32_t *>(x_next + xt_index(m, k0, kI)) = lo;
-                *reinterpret_cast<uint32_t *>(x_next + xt_index(m, k0 + 2, kI)) = hi;
+                *reinterpret_cast<uint32_t *>(x_next + xt_index(mb + m, k0, kI)) = lo;
+                *reinterpret_cast<uint32_t *>(x_next + xt_index(mb + m, k0 + 2, kI)) = hi;
             }
         }
     }
@@ -426,12 +431,12 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
     // 2 p + 6, 2 p + 7 of tile 2): task (stream m, p), thread 64 + 3 m + p
     if (t >= 64) {
         const int q = t - 64, m = q / 3, p = q - 3 * m;
-        if (m < n_streams) {
+        if (mb + m < n_streams) {
             const int rg = 2 * p, ru = 2 * p + 6;
             const f32x4 gv = val4(2, rg >> 2, m), uv = val4(2, ru >> 2, m);
             const float g0 = (rg & 3) ? gv.z : gv.x, g1 = (rg & 3) ? gv.w : gv.y;
             const float u0 = (ru & 3) ? uv.z : uv.x, u1 = (ru & 3) ? uv.w : uv.y;
-            *reinterpret_cast<uint32_t *>(x_next + xt_index(m, rb * kGuCh + 16 + 2 * p, kI)) =
+            *reinterpret_cast<uint32_t *>(x_next + xt_index(mb + m, rb * kGuCh + 16 + 2 * p, kI)) =
                 swiglu(g0, u0) | (swiglu(g1, u1) << 16);
         }
     }
@@ -484,7 +489,8 @@ __global__ __launch_bounds__(kT) void k_bargmax(const float *__restrict__ part_v
 struct BNorm {
     const float *h_in;     // [64][kH] residual stream
     float *h_out;          // h_in, or (AB, several workgroups per stream) the other residual buffer
-    const float *y;        // [splits][64][kH] partial sums: h = R(h + R(sum)) first
+    const float *y;        // [splits][y_rows][kH] partial sums: h = R(h + R(sum)) first
+    int y_rows;
     const uint16_t *emb;   // embedding rows (BF16): h = R(emb[tok[m]]) (EMBED)
     const int *tok;
     const float *w;        // norm weight [kH]
@@ -546,7 +552,7 @@ __global__ __launch_bounds__(kT) void k_bnorm(BNorm p) {
             f32x4 yp[SPLITS][2];
 #pragma unroll
             for (int sp = 0; sp < SPLITS; ++sp) {
-                const f32x4 *y4 = reinterpret_cast<const f32x4 *>(p.y + ((size_t)sp * kMaxB + m) * kH + e0);
+                const f32x4 *y4 = reinterpret_cast<const f32x4 *>(p.y + ((size_t)sp * p.y_rows + m) * kH + e0);
                 yp[sp][0] = y4[0];
                 yp[sp][1] = y4[1];
             }
@@ -1649,9 +1655,17 @@ __device__ __forceinline__ bool pg_close(int j, f32x4 (&chain)[NB], f32x4 (&part
 #endif
 constexpr int kPgW = GDN_PG_WAVES;
 
-template <int KT, int NW, int S>
+// PLANES: grid z is the split; a workgroup forms one split's sum and writes
+// it to that split's plane of y (y_rows tokens), which the consumer adds in
+// split order, as it adds the step's.  Four times the workgroups of the
+// running total, for segments whose tiles leave CUs idle.
+template <int KT, int NW, int S, bool PLANES>
 __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
-                                                     float *__restrict__ y, int n_rows) {
+                                                     float *__restrict__ y, int n_rows, int y_rows) {
+    constexpr int NT = PLANES ? KT / S : KT;  // k tiles of this workgroup
+    static_assert(NT % kPgD == 0, "whole groups of kPgD k tiles");
+    const int jb = PLANES ? (int)blockIdx.z * NT : 0;
+    if constexpr (PLANES) y += (size_t)blockIdx.z * y_rows * n_rows;
     constexpr int GT = kPgW * 64, AU = 4 * 2 * 64, BU = 2 * 4 * 64, PT = (AU + BU) / GT;
     constexpr int TG = kPgW == 4 ? 4 : 2;  // 16-token groups per wave
     constexpr int NB = 4 * TG;            // 16 x 16 blocks per wave
@@ -1692,8 +1706,8 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
     };
     u32x4 rg[kPgD][PT];
 #pragma unroll
-    for (int d = 0; d < kPgD; ++d) fetch(rg[d], pg_tile<KT, NW, S>(d));
-    for (int j0 = 0; j0 < KT; j0 += kPgD) {
+    for (int d = 0; d < kPgD; ++d) fetch(rg[d], pg_tile<KT, NW, S>(jb + d));
+    for (int j0 = 0; j0 < NT; j0 += kPgD) {
 #pragma unroll
         for (int d = 0; d < kPgD; ++d) {
             const int j = j0 + d, sb = d & 1;
@@ -1702,7 +1716,7 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
             // issued on every pass (the last passes re-read the final tile,
             // unused): a conditional load would make the compiler's wait
             // for the next stage a wait for every load in flight
-            fetch(rg[d], pg_tile<KT, NW, S>(j + kPgD < KT ? j + kPgD : KT - 1));
+            fetch(rg[d], pg_tile<KT, NW, S>(jb + (j + kPgD < NT ? j + kPgD : NT - 1)));
             __syncthreads();
             u32x4 fa[4], fb[TG];
 #pragma unroll
@@ -1718,7 +1732,8 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
                         0, 0);
             if (pg_close<KT, NW, S, NB>(j, chain, part)) {
                 // the split's sum joins the total in split order
-                const bool first = j < KT / S;
+                // (one split per workgroup with PLANES)
+                const bool first = PLANES || j < KT / S;
 #pragma unroll
                 for (int b = 0; b < NB; ++b) *out(b) = first ? part[b] : *out(b) + part[b];
             }
@@ -2187,6 +2202,7 @@ BNorm bnorm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_out, 
     p.h_in = b_resid(e, l_in);
     p.h_out = b_resid(e, l_out);
     p.y = y;
+    p.y_rows = kMaxB;
     p.w = w;
     p.x_out = x_out;
     p.eps = e->eps;
@@ -2234,6 +2250,7 @@ void launch_o(GDNBatchEngine *e, int l, hipStream_t s) {
     ep.n_streams = e->streams;
     ep.n_rows = kH;
     ep.y = e->ypart;
+    ep.y_rows = kMaxB;
     hipLaunchKernelGGL((k_bgemm<kRtO, kKtH, 4, kSplitO, EPI_RAW>), dim3(kH / (16 * kRtO), kSplitO), dim3(kT), 0, s,
                        e->w_o[l], reinterpret_cast<const u32x4 *>(e->x_o), ep);
 }
@@ -2250,6 +2267,7 @@ void launch_down(GDNBatchEngine *e, int l, hipStream_t s) {
     ep.n_streams = e->streams;
     ep.n_rows = kH;
     ep.y = e->ypart;
+    ep.y_rows = kMaxB;
     hipLaunchKernelGGL((k_bgemm<kRtDown, kKtI, 4, kSplitDown, EPI_RAW>), dim3(kH / (16 * kRtDown), kSplitDown),
                        dim3(kT), 0, s, e->w_down[l], reinterpret_cast<const u32x4 *>(e->x_d), ep);
 }
@@ -2379,6 +2397,7 @@ BNorm seg_norm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_ou
     p.h_in = e->s_h + (size_t)(l_in & 1) * e->seg_cap * kH;
     p.h_out = e->s_h + (size_t)(l_out & 1) * e->seg_cap * kH;
     p.y = y;
+    p.y_rows = e->seg_cap;
     p.w = w;
     p.x_out = x_out;
     p.eps = e->eps;
@@ -2399,13 +2418,85 @@ BNorm seg_norm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_ou
 // (k_pconv), and the recurrence chunk by chunk of 64 tokens, in token order
 // (k_pqk, k_pscan) or in the WY form (k_wy_prep over every chunk at once,
 // then k_wy_seq over the chunks in order).
-// k_pgemm_a (the faster kernel once its grid fills the CUs) or k_pgemm (twice
-// the workgroups at the same size, so the better one on short segments):
-// the same sums either way.
-bool pa_fills(int rows, int tiles) { return rows % kPaRows == 0 && (rows / kPaRows) * tiles >= 256; }
+// The prefill's projections over n tokens (X in 64-token tile blocks, padded
+// to whole 128-token tiles), on the kernel that is fastest at that size; every
+// choice forms the same sums.
+enum PRoute {
+    P_STEP,    // the decode step's kernels, a grid plane per 64-token block
+    P_PLANES,  // k_pgemm with a workgroup per split (o_proj, down)
+    P_TILE,    // k_pgemm / k_pgu, 128 tokens per workgroup
+    P_WIDE     // k_pgemm_a, once its grid (half of k_pgemm's) fills the CUs
+};
+// Where the lines lie (us per launch, step / planes / tile at 64, 256, 512,
+// 1024, 2048 tokens):
+//   q/k/v/g  12 / - / 30   28 / - / 30    49 / - / 32    91 / - / 42   174 / - / 79
+//   o_proj    5 / 11 / 34    9 / 11 / 33   15 / 12 / 34   26 / 19 / 36   49 / 38 / 44
+//   down      9 / 20 / 71   18 / 20 / 69   30 / 22 / 70   54 / 37 / 75  103 / 69 / 85
+//   gate/up  15 / - / 30   33 / - / 31    57 / - / 43   107 / - / 83   207 / - / 165
+// The step's kernels re-read the weights per 64 tokens; the tile kernels leave
+// most CUs idle on short segments (16 workgroups for o_proj and down at up to
+// 128 tokens).  Planes cost the norm after them three more reads (12 against
+// 9 us at 1024 tokens, 46 against 32 at 4096), which moves their upper line
+// down: at 4096 tokens o_proj, down and their norms take 114 + 177 against
+// 114 + 161 us.
+bool pa_fills(int rows, int n) { return rows % kPaRows == 0 && (rows / kPaRows) * ((n + kPgTok - 1) / kPgTok) >= 256; }
+PRoute route_qkvg(int rows, int n) { return n <= 256 ? P_STEP : pa_fills(rows, n) ? P_WIDE : P_TILE; }
+PRoute route_o(int n) { return n <= 256 ? P_STEP : n <= 1536 ? P_PLANES : P_TILE; }
+PRoute route_down(int rows, int n) {
+    return n <= 256 ? P_STEP : n <= 3072 ? P_PLANES : pa_fills(rows, n) ? P_WIDE : P_TILE;
+}
+PRoute route_gu(int n) { return n <= 192 ? P_STEP : P_TILE; }
+
+// A projection in 32-row blocks of KT k tiles, NW classes and S splits:
+// returns the planes of y (y_rows tokens each) that its consumer adds: S, or
+// 1 (the total).
+template <int KT, int NW, int S>
+int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int rows, int n, int y_rows,
+                  hipStream_t s) {
+    const int blocks = (n + kMaxB - 1) / kMaxB, tiles = (n + kPgTok - 1) / kPgTok;
+    if (route == P_STEP) {
+        BEpi ep{};
+        ep.n_streams = kMaxB;
+        ep.n_rows = rows;
+        ep.y = y;
+        ep.y_rows = y_rows;
+        hipLaunchKernelGGL((k_bgemm<2, KT, NW, S, EPI_RAW>), dim3(rows / 32, S, blocks), dim3(NW * 64), 0, s, w, x,
+                           ep);
+        return S;
+    }
+    if (route == P_PLANES) {
+        hipLaunchKernelGGL((k_pgemm<KT, NW, S, true>), dim3(rows / 128, tiles, S), dim3(kPgW * 64), 0, s, w, x, y,
+                           rows, y_rows);
+        return S;
+    }
+    if (route == P_WIDE)
+        hipLaunchKernelGGL((k_pgemm_a<KT, NW, S>), dim3(rows / kPaRows, tiles), dim3(kPgW * 64), 0, s, w, x, y, rows);
+    else
+        hipLaunchKernelGGL((k_pgemm<KT, NW, S, false>), dim3(rows / 128, tiles), dim3(kPgW * 64), 0, s, w, x, y, rows,
+                           0);
+    return 1;
+}
+static_assert(kRtO == 2 && kRtDown == 2, "o_proj and down in 32-row blocks");
+
+void launch_p_gu(PRoute route, const u32x4 *w, const u32x4 *x, uint16_t *x_next, int n, hipStream_t s) {
+    if (route == P_STEP)
+        hipLaunchKernelGGL(k_bgu<kGuWaves>, dim3(kGuWgs, (n + kMaxB - 1) / kMaxB), dim3(kGuWaves * 64), 0, s, w, x,
+                           x_next, n);
+    else
+        hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, (n + kPgTok - 1) / kPgTok), dim3(kPgW * 64), 0, s, w, x, x_next, n);
+}
+
+// The residual add and norm after o_proj or down.
+void launch_p_norm(const BNorm &p, int planes, int n, hipStream_t s) {
+    static_assert(kSplitO == kSplitDown, "one norm kernel for both");
+    if (planes == 1)
+        hipLaunchKernelGGL((k_bnorm<1, false, false>), dim3(n), dim3(kT), 0, s, p);
+    else
+        hipLaunchKernelGGL((k_bnorm<kSplitO, false, false>), dim3(n), dim3(kT), 0, s, p);
+}
 
 void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipStream_t s) {
-    const int blocks = (n + kMaxB - 1) / kMaxB, tiles = (n + kPgTok - 1) / kPgTok;
+    const int blocks = (n + kMaxB - 1) / kMaxB;
     const int pab_blocks = (n + kPabTok - 1) / kPabTok;
     // a norm's a/b rows and beta/decay, from its normalised copy in s_xn
     auto launch_ab = [&](int l_ab) {
@@ -2424,12 +2515,7 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
     for (int l = 0; l < e->layers; ++l) {
         float *st = b_state(e, l) + (size_t)slot * kLayerState;
         uint16_t *tl = b_tails(e, l) + (size_t)slot * kStreamTails;
-        if (pa_fills(4 * kH, tiles))
-            hipLaunchKernelGGL((k_pgemm_a<kKtH, 8, 1>), dim3(4 * kH / kPaRows, tiles), dim3(kPgW * 64), 0, s,
-                               e->w_qkvg[l], xh, e->s_y, 4 * kH);
-        else
-            hipLaunchKernelGGL((k_pgemm<kKtH, 8, 1>), dim3(4 * kH / 128, tiles), dim3(kPgW * 64), 0, s,
-                               e->w_qkvg[l], xh, e->s_y, 4 * kH);
+        launch_p_gemm<kKtH, 8, 1>(route_qkvg(4 * kH, n), e->w_qkvg[l], xh, e->s_y, 4 * kH, n, e->seg_cap, s);
         hipLaunchKernelGGL(k_pconv, dim3(4 * kH / 64, blocks), dim3(kConvT), 0, s, e->s_y, n, tl,
                            b_aux(e, l) + kAuxConv, e->s_qkv, e->s_gate, e->s_sgate);
         if (e->prefill_mode == GDN_PREFILL_CHUNKED) {
@@ -2444,26 +2530,20 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
         }
         hipLaunchKernelGGL(k_bonorm<kOnTok>, dim3(kNH, (n + kOnTok - 1) / kOnTok), dim3(kT), 0, s, e->s_attn,
                            e->s_gate, e->s_sgate, b_aux(e, l) + kAuxONorm, e->eps, e->s_xo, n);
-        hipLaunchKernelGGL((k_pgemm<kKtH, 4, kSplitO>), dim3(kH / 128, tiles), dim3(kPgW * 64), 0, s, e->w_o[l], xo,
-                           e->s_y, kH);
-        const BNorm pm = seg_norm(e, e->s_y, b_aux(e, l) + kAuxMlpNorm, e->s_xh, -1, l, l);
-        hipLaunchKernelGGL((k_bnorm<1, false, false>), dim3(n), dim3(kT), 0, s, pm);
-        hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, tiles), dim3(kPgW * 64), 0, s, e->w_gu[l], xh, e->s_xd, n);
-        if (pa_fills(kH, tiles))
-            hipLaunchKernelGGL((k_pgemm_a<kKtI, 4, kSplitDown>), dim3(kH / kPaRows, tiles), dim3(kPgW * 64), 0, s,
-                               e->w_down[l], xd, e->s_y, kH);
-        else
-            hipLaunchKernelGGL((k_pgemm<kKtI, 4, kSplitDown>), dim3(kH / 128, tiles), dim3(kPgW * 64), 0, s,
-                               e->w_down[l], xd, e->s_y, kH);
+        const int po = launch_p_gemm<kKtH, 4, kSplitO>(route_o(n), e->w_o[l], xo, e->s_y, kH, n, e->seg_cap, s);
+        launch_p_norm(seg_norm(e, e->s_y, b_aux(e, l) + kAuxMlpNorm, e->s_xh, -1, l, l), po, n, s);
+        launch_p_gu(route_gu(n), e->w_gu[l], xh, e->s_xd, n, s);
+        const int pd =
+            launch_p_gemm<kKtI, 4, kSplitDown>(route_down(kH, n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
         if (l + 1 < e->layers) {
             BNorm pa = seg_norm(e, e->s_y, b_aux(e, l + 1) + kAuxAttnNorm, e->s_xh, -1, l, l + 1);
             pa.xn_out = e->s_xn;
-            hipLaunchKernelGGL((k_bnorm<1, false, false>), dim3(n), dim3(kT), 0, s, pa);
+            launch_p_norm(pa, pd, n, s);
             launch_ab(l + 1);
         } else {
             BNorm pf = seg_norm(e, e->s_y, e->aux + (size_t)e->layers * kAuxLayer, e->s_xh, -1, l, l);
             pf.xn_out = e->s_xn;
-            hipLaunchKernelGGL((k_bnorm<1, false, false>), dim3(n), dim3(kT), 0, s, pf);
+            launch_p_norm(pf, pd, n, s);
         }
     }
     if (!last) return;
@@ -2786,6 +2866,7 @@ int gdn_test_batch_gemm(const float *W, const float *X, uint32_t N, uint32_t K, 
     ep.n_streams = kMaxB;
     ep.n_rows = (int)N;
     ep.y = dy;
+    ep.y_rows = kMaxB;
     if (k_hidden)
         hipLaunchKernelGGL((k_bgemm<kRtO, kKtH, 4, kSplitO, EPI_RAW>), dim3(N / rows, kSplitO), dim3(kT), 0, 0,
                            static_cast<const u32x4 *>(dw), static_cast<const u32x4 *>(dx), ep);
@@ -2835,26 +2916,55 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     GDN_HIP(hipMalloc(&dx, xt.size() * 2));
     GDN_HIP(hipMalloc(&dy, out_elems * 4));
     GDN_HIP(hipMalloc(&dr, out_elems * 4));
-    GDN_HIP(hipMemset(dy, 0, out_elems * 4));
     GDN_HIP(hipMemset(dr, 0, out_elems * 4));
     GDN_HIP(hipMemcpy(dw, wt.data(), wt.size() * 2, hipMemcpyHostToDevice));
     GDN_HIP(hipMemcpy(dx, xt.data(), xt.size() * 2, hipMemcpyHostToDevice));
     const u32x4 *w4 = static_cast<const u32x4 *>(dw), *x4 = static_cast<const u32x4 *>(dx);
-    const dim3 pg(N / 128, tp / kPgTok);
-    const dim3 pa(N / kPaRows, tp / kPgTok);
-    if (kind == 0 && N % kPaRows == 0)
-        hipLaunchKernelGGL((k_pgemm_a<kKtH, 8, 1>), pa, dim3(kPgW * 64), 0, 0, w4, x4, (float *)dy, (int)N);
-    if (kind == 0 && N % kPaRows != 0)
-        hipLaunchKernelGGL((k_pgemm<kKtH, 8, 1>), pg, dim3(kPgW * 64), 0, 0, w4, x4, (float *)dy, (int)N);
-    if (kind == 1)
-        hipLaunchKernelGGL((k_pgemm<kKtH, 4, kSplitO>), pg, dim3(kPgW * 64), 0, 0, w4, x4, (float *)dy, (int)N);
-    if (kind == 2 && N % kPaRows == 0)
-        hipLaunchKernelGGL((k_pgemm_a<kKtI, 4, kSplitDown>), pa, dim3(kPgW * 64), 0, 0, w4, x4, (float *)dy, (int)N);
-    if (kind == 2 && N % kPaRows != 0)
-        hipLaunchKernelGGL((k_pgemm<kKtI, 4, kSplitDown>), pg, dim3(kPgW * 64), 0, 0, w4, x4, (float *)dy, (int)N);
-    if (kind == 3)
-        hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, tp / kPgTok), dim3(kPgW * 64), 0, 0, w4, x4,
-                           static_cast<uint16_t *>(dy), (int)T);
+    // one route into out (floats of a zeroed buffer's planes added in order,
+    // or the X tiles' halves)
+    const int rows = (int)N, toks = (int)T, pad = (int)tp;
+    auto run_route = [&](PRoute route, std::vector<float> &out, std::vector<uint16_t> &tiles16) -> int {
+        GDN_HIP(hipMemset(dy, 0, out_elems * 4));
+        int planes = 1;
+        float *y = static_cast<float *>(dy);
+        if (kind == 0) planes = launch_p_gemm<kKtH, 8, 1>(route, w4, x4, y, rows, toks, pad, nullptr);
+        if (kind == 1) planes = launch_p_gemm<kKtH, 4, kSplitO>(route, w4, x4, y, rows, toks, pad, nullptr);
+        if (kind == 2) planes = launch_p_gemm<kKtI, 4, kSplitDown>(route, w4, x4, y, rows, toks, pad, nullptr);
+        if (kind == 3) launch_p_gu(route, w4, x4, static_cast<uint16_t *>(dy), toks, nullptr);
+        GDN_HIP(hipGetLastError());
+        GDN_HIP(hipDeviceSynchronize());
+        if (kind == 3) {
+            tiles16.resize((size_t)tp * kI);
+            GDN_HIP(hipMemcpy(tiles16.data(), dy, tiles16.size() * 2, hipMemcpyDeviceToHost));
+            return 0;
+        }
+        std::vector<float> a(out_elems);
+        GDN_HIP(hipMemcpy(a.data(), dy, a.size() * 4, hipMemcpyDeviceToHost));
+        out.resize((size_t)T * N);
+        for (size_t i = 0; i < out.size(); ++i) {
+            float v = a[i];
+            for (int sp = 1; sp < planes; ++sp) v = v + a[(size_t)sp * tp * N + i];
+            out[i] = v;
+        }
+        return 0;
+    };
+    // the 128-token kernels give the result; every other kernel that a
+    // segment of some length runs on has to agree with it bit for bit
+    std::vector<PRoute> routes = {kind % 2 == 0 && N % kPaRows == 0 ? P_WIDE : P_TILE, P_STEP, P_TILE};
+    if (kind == 1 || kind == 2) routes.push_back(P_PLANES);
+    std::vector<float> first, other;
+    std::vector<uint16_t> first16, other16;
+    if (run_route(routes[0], first, first16)) return -1;
+    for (size_t r = 1; r < routes.size(); ++r) {
+        if (run_route(routes[r], other, other16)) return -1;
+        const size_t bytes = kind == 3 ? first16.size() * 2 : first.size() * 4;
+        if (std::memcmp(kind == 3 ? (const void *)first16.data() : first.data(),
+                        kind == 3 ? (const void *)other16.data() : other.data(), bytes) != 0) {
+            std::fprintf(stderr, "gdn_test_prefill_gemm: kind %d, route %d differs from route %d\n", kind,
+                         (int)routes[r], (int)routes[0]);
+            return -1;
+        }
+    }
     // the step's kernels, one 64-token block at a time
     for (uint32_t b = 0; b < blocks; ++b) {
         const u32x4 *xb4 = x4 + (size_t)b * kMaxB * K / 8;
@@ -2862,6 +2972,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
         ep.n_streams = kMaxB;
         ep.n_rows = (int)N;
         ep.y = static_cast<float *>(dr) + (size_t)b * kSplitDown * kMaxB * N;
+        ep.y_rows = kMaxB;
         if (kind == 0)
             hipLaunchKernelGGL((k_bgemm<2, kKtH, 8, 1, EPI_RAW>), dim3(N / 32), dim3(8 * 64), 0, 0, w4, xb4, ep);
         if (kind == 1)
@@ -2878,8 +2989,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     GDN_HIP(hipDeviceSynchronize());
     if (kind == 3) {
         // both outputs are X tiles of width kI: untile the first T tokens
-        std::vector<uint16_t> a((size_t)tp * kI), r((size_t)tp * kI);
-        GDN_HIP(hipMemcpy(a.data(), dy, a.size() * 2, hipMemcpyDeviceToHost));
+        std::vector<uint16_t> &a = first16, r((size_t)tp * kI);
         GDN_HIP(hipMemcpy(r.data(), dr, r.size() * 2, hipMemcpyDeviceToHost));
         for (uint32_t m = 0; m < T; ++m)
             for (uint32_t k = 0; k < (uint32_t)kI; ++k) {
@@ -2891,8 +3001,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
                 std::memcpy(Y_step + (size_t)m * kI + k, &yr, 4);
             }
     } else {
-        std::vector<float> a((size_t)tp * N), r(out_elems);
-        GDN_HIP(hipMemcpy(a.data(), dy, a.size() * 4, hipMemcpyDeviceToHost));
+        std::vector<float> r(out_elems);
         GDN_HIP(hipMemcpy(r.data(), dr, r.size() * 4, hipMemcpyDeviceToHost));
         const int splits = kind == 0 ? 1 : kSplitDown;
         for (uint32_t m = 0; m < T; ++m)
@@ -2900,7 +3009,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
                 const size_t base = (size_t)(m / kMaxB) * kSplitDown * kMaxB * N + (size_t)(m % kMaxB) * N + n;
                 float v = r[base];
                 for (int sp = 1; sp < splits; ++sp) v = v + r[base + (size_t)sp * kMaxB * N];
-                Y[(size_t)m * N + n] = a[(size_t)m * N + n];
+                Y[(size_t)m * N + n] = first[(size_t)m * N + n];
                 Y_step[(size_t)m * N + n] = v;
             }
     }

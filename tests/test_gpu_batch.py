@@ -101,6 +101,43 @@ def test_prefill_gemm_equals_step_gemm(kind, N, T):
     assert same_bits(y, y_step)
 
 
+@pytest.mark.parametrize("kind,N,T", [(0, 256, 257), (0, 128, 1), (1, 128, 63), (1, 128, 257), (2, 256, 129),
+                                      (2, 128, 1), (3, 5632, 193), (3, 5632, 1)])
+def test_prefill_gemm_routes_agree(kind, N, T):
+    """Each kernel that a segment of some length takes for a projection (the
+    step's over token blocks, the split planes, the 128-token tiles) gives the
+    same bits, at a token past and short of their blocks: the call itself
+    fails if two differ, and its result is the step's."""
+    rng = np.random.default_rng(200 + 10 * kind + T)
+    K = 5632 if kind == 2 else 2048
+    shape = (2, N, K) if kind == 3 else (N, K)
+    W = g.bf16_round(rng.normal(0, 0.02, shape).astype(np.float32)).reshape(shape)
+    X = g.bf16_round(rng.normal(0, 1, (T, K)).astype(np.float32)).reshape(T, K)
+    y, y_step = g.prefill_gemm(kind, W, X)
+    assert np.abs(y_step).max() > 0
+    assert same_bits(y, y_step)
+
+
+@pytest.mark.parametrize("n", [192, 193, 256, 257, 1536, 1537, 3073])
+def test_prefill_route_edges_equal_steps(n):
+    """Prompts on both sides of each projection's change of kernel: a layer's
+    state and the next token equal single-stream steps bit for bit."""
+    m = g.Model.synth(num_layers=1, seed=5, std=0.02, bf16=True)
+    prompt = g.synth_tokens(n, 23, 7)
+    pre, ref = g.BatchState(m, 1), g.BatchState(m, 1)
+    try:
+        seed = pre.prefill(0, prompt)
+        am, _, _ = ref.teacher_forced(prompt.reshape(-1, 1), timing=False)
+        assert seed == int(am[-1, 0])
+        for a, b in zip(pre.save_stream_state(0), ref.save_stream_state(0)):
+            assert same_bits(a, b)
+        assert same_bits(pre.logits(0), ref.logits(0))
+    finally:
+        pre.free()
+        ref.free()
+        m.free()
+
+
 def batch1_reference(m, tokens, init=None):
     """Per-stream batch-1 runs (BF16W_FP32S): logits [steps][B][V], tokens,
     final states."""
