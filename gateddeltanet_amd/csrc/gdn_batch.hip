@@ -120,8 +120,10 @@ struct BEpi {
 // added in wave order through LDS; the epilogue then runs on the reduced
 // tile.  Split partial sums (EPI_RAW with S > 1) are added in split order by
 // the consumer.  With EPI_RAW the grid's z dimension is the 64-token block of
-// a prefill segment.
-template <int RT, int KT, int NW, int S, int EPI>
+// a prefill segment.  G: the 16-stream groups that are formed (four, or as
+// many as hold the step's streams); a group's sums do not depend on the
+// others.
+template <int RT, int KT, int NW, int S, int EPI, int G = 4>
 __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                    BEpi ep) {
     constexpr int KTS = KT / S, KTW = KTS / NW, GT = NW * 64;
@@ -129,9 +131,9 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
     static_assert(S == 1 || EPI == EPI_RAW, "split sums leave the GEMM unrounded");
     constexpr int D = KTW < 4 ? KTW : 4;
     constexpr size_t WSTEP = (size_t)NW * RT * 64, XSTEP = (size_t)NW * 4 * 64;
-    __shared__ f32x4 red[NW * RT * 4 * 64];
-    __shared__ float lm_v[RT * 4][64];
-    __shared__ int lm_i[RT * 4][64];
+    __shared__ f32x4 red[NW * RT * G * 64];
+    __shared__ float lm_v[RT * 4][16 * G];
+    __shared__ int lm_i[RT * 4][16 * G];
     __shared__ uint64_t exp2_lds[EPI == EPI_QKVG ? 32 : 1];  // expf's table for the epilogue
     __shared__ f32x4 conv_lds[EPI == EPI_QKVG ? RT * 16 : 1];  // the conv taps of the workgroup's channels
     if constexpr (EPI == EPI_QKVG) fill_exp2_lds_imm(exp2_lds);
@@ -154,8 +156,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
     // channel) and the workgroup's taps (into LDS) are read ahead of the
     // weight stream.
     constexpr int CG = RT * 4;
-    constexpr int QE = (EPI == EPI_QKVG) ? (64 * CG) / GT : 1;
-    static_assert(EPI != EPI_QKVG || (64 * CG) % GT == 0, "whole epilogue tasks per thread");
+    constexpr int QE = (EPI == EPI_QKVG) ? (16 * G * CG + GT - 1) / GT : 1;
     const int which = (rb * 16 * RT) / kH, c0 = rb * 16 * RT - which * kH;  // q, k, v, g section
     uint2 qtl[QE][3];
     if constexpr (EPI == EPI_QKVG) {
@@ -174,18 +175,18 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
         }
     }
 
-    f32x4 acc[RT][4];
+    f32x4 acc[RT][G];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) acc[r][g] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    u32x4 a[D][RT], b[D][4];
+        for (int g = 0; g < G; ++g) acc[r][g] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    u32x4 a[D][RT], b[D][G];
 #pragma unroll
     for (int i = 0; i < D; ++i) {
 #pragma unroll
         for (int r = 0; r < RT; ++r) a[i][r] = wp[i * WSTEP + r * 64];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) b[i][g] = xp[i * XSTEP + g * 64];
+        for (int g = 0; g < G; ++g) b[i][g] = xp[i * XSTEP + g * 64];
     }
     // the scheduler keeps every prefetch where it is issued: D k tiles stay
     // in flight instead of one
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
+            for (int g = 0; g < G; ++g)
                 acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[s][r]),
                                                                     __builtin_bit_cast(bf16x8, b[s][g]),
                                                                     acc[r][g], 0, 0, 0);
@@ -204,31 +205,31 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
 #pragma unroll
             for (int r = 0; r < RT; ++r) a[s][r] = wp[(i + D) * WSTEP + r * 64];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) b[s][g] = xp[(i + D) * XSTEP + g * 64];
+            for (int g = 0; g < G; ++g) b[s][g] = xp[(i + D) * XSTEP + g * 64];
         }
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) red[((w * RT + r) * 4 + g) * 64 + l] = acc[r][g];
+        for (int g = 0; g < G; ++g) red[((w * RT + r) * G + g) * 64 + l] = acc[r][g];
     __syncthreads();
 
     // Task (rt, nq, m): rows rt * 16 + nq * 4 + 0..3 of stream m, held by lane
     // nq * 16 + m % 16 of stream group m / 16 in every wave's D tile.  Every
     // epilogue takes whole tasks (the four rows as one f32x4).
-    auto red_index = [&](int rt, int nq, int m) { return (rt * 4 + (m >> 4)) * 64 + nq * 16 + (m & 15); };
+    auto red_index = [&](int rt, int nq, int m) { return (rt * G + (m >> 4)) * 64 + nq * 16 + (m & 15); };
     auto reduced = [&](int rt, int nq, int m) {
         const int idx = red_index(rt, nq, m);
         f32x4 v = red[idx];
 #pragma unroll
-        for (int ww = 1; ww < NW; ++ww) v = v + red[ww * RT * 4 * 64 + idx];
+        for (int ww = 1; ww < NW; ++ww) v = v + red[ww * RT * G * 64 + idx];
         return v;
     };
     if constexpr (EPI == EPI_RAW || EPI == EPI_STORE || EPI == EPI_LM) {
 #pragma unroll
-        for (int q = t; q < RT * 4 * 64; q += GT) {
-            const int m = q & 63, nq = (q >> 6) & 3, rt = q >> 8;
+        for (int q = t; q < RT * 4 * 16 * G; q += GT) {
+            const int m = q % (16 * G), nq = (q / (16 * G)) & 3, rt = q / (64 * G);
             const f32x4 v = reduced(rt, nq, m);
             const int row = rb * 16 * RT + rt * 16 + nq * 4;
             if constexpr (EPI == EPI_LM) {
@@ -296,7 +297,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
     }
     if constexpr (EPI == EPI_LM) {
         __syncthreads();
-        if (t < 64) {
+        if (t < 16 * G) {
             // row quads in index order: strict '>' keeps the lowest index of
             // equal maxima (NaN never wins)
             float best = lm_v[0][t];
@@ -333,7 +334,7 @@ static_assert(kGuWgs * kGuCh == kI && kGuCh > 16 && kGuCh <= 24 && (kGuCh % 2) =
 // The NW waves split the 64 k tiles as k_bgemm's do (wave w: w, w + NW, ...)
 // and the per-wave sums are added in wave order, so each channel's sums are
 // those of k_bgemm's 16-channel pairing with the same NW.
-template <int NW>
+template <int NW, int G = 4>
 __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                  uint16_t *__restrict__ x_next, int n_streams) {
     // grid y: the 64-token block of a prefill segment of n_streams tokens
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
     static_assert(KT % NW == 0, "whole k tiles per wave");
     constexpr int D = KTW < 4 ? KTW : 4;
     constexpr size_t WSTEP = (size_t)NW * kGuTileU4, XSTEP = (size_t)NW * 4 * 64;
-    __shared__ f32x4 red[NW * RT * 4 * 64];
+    __shared__ f32x4 red[NW * RT * G * 64];
     __shared__ uint64_t exp2_lds[32];  // expf's table for the SwiGLU epilogue
     const int t = threadIdx.x, w = t >> 6, l = t & 63, rb = blockIdx.x;
     fill_exp2_lds_imm(exp2_lds);
@@ -354,19 +355,19 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
     const u32x4 *xp = X + ((size_t)blockIdx.y * KT + w) * (4 * 64) + l;
     const u32x4 zero = {0u, 0u, 0u, 0u};
 
-    f32x4 acc[RT][4];
+    f32x4 acc[RT][G];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) acc[r][g] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    u32x4 a[D][RT], b[D][4];
+        for (int g = 0; g < G; ++g) acc[r][g] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    u32x4 a[D][RT], b[D][G];
 #pragma unroll
     for (int i = 0; i < D; ++i) {
         a[i][0] = wp[i * WSTEP + l];
         a[i][1] = wp[i * WSTEP + 64 + l];
         a[i][2] = wp[i * WSTEP + o2];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) b[i][g] = xp[i * XSTEP + g * 64];
+        for (int g = 0; g < G; ++g) b[i][g] = xp[i * XSTEP + g * 64];
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
+            for (int g = 0; g < G; ++g)
                 acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[s][r]),
                                                                     __builtin_bit_cast(bf16x8, b[s][g]),
                                                                     acc[r][g], 0, 0, 0);
@@ -385,23 +386,23 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
             a[s][1] = wp[(i + D) * WSTEP + 64 + l];
             a[s][2] = wp[(i + D) * WSTEP + o2];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) b[s][g] = xp[(i + D) * XSTEP + g * 64];
+            for (int g = 0; g < G; ++g) b[s][g] = xp[(i + D) * XSTEP + g * 64];
         }
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) red[((w * RT + r) * 4 + g) * 64 + l] = acc[r][g];
+        for (int g = 0; g < G; ++g) red[((w * RT + r) * G + g) * 64 + l] = acc[r][g];
     __syncthreads();
 
     // rows 4 nq .. 4 nq + 3 of tile r for stream m: lane nq * 16 + m % 16 of
     // stream group m / 16 in every wave's tile, the waves added in order
     auto val4 = [&](int r, int nq, int m) {
-        const int idx = (r * 4 + (m >> 4)) * 64 + nq * 16 + (m & 15);
+        const int idx = (r * G + (m >> 4)) * 64 + nq * 16 + (m & 15);
         f32x4 v = red[idx];
 #pragma unroll
-        for (int ww = 1; ww < NW; ++ww) v = v + red[ww * RT * 4 * 64 + idx];
+        for (int ww = 1; ww < NW; ++ww) v = v + red[ww * RT * G * 64 + idx];
         return v;
     };
     // gemv32_store SwiGLU branch, gdn_model.cpp:4751-4767, for one channel
@@ -412,7 +413,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
     static_assert(kGuCh == 22 && GT == 256, "16 + 6 channels; 256 + 192 tasks over four waves");
     // channels 4 nq .. 4 nq + 3 (gate rows of tile 0, up rows of tile 1):
     // task (stream m, nq), thread 4 m + nq
-    {
+    if (t < 64 * G) {
         const int m = t >> 2, nq = t & 3;
         if (mb + m < n_streams) {
             const f32x4 g = val4(0, nq, m), u = val4(1, nq, m);
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgu(const u32x4 *__restrict__ W, co
     }
     // channels 16 + 2 p, 17 + 2 p (gate rows 2 p, 2 p + 1 and up rows
     // 2 p + 6, 2 p + 7 of tile 2): task (stream m, p), thread 64 + 3 m + p
-    if (t >= 64) {
+    if (t >= 64 && t < 64 + 48 * G) {
         const int q = t - 64, m = q / 3, p = q - 3 * m;
         if (mb + m < n_streams) {
             const int rg = 2 * p, ru = 2 * p + 6;
@@ -2018,12 +2019,39 @@ float *b_state(GDNBatchEngine *e, int l) { return e->state + (size_t)l * e->stre
 // allows, else 32; its weights are tiled to match.
 int lm_rt(const GDNBatchEngine *e) { return (e->vocab % 64) == 0 ? 4 : 2; }
 int lm_wgs(const GDNBatchEngine *e) { return e->vocab / (16 * lm_rt(e)); }
-void launch_lm_gemm(GDNBatchEngine *e, const BEpi &ep, const void *x, hipStream_t s) {
+// The step's GEMM on as many 16-stream groups as hold n streams (or prefill
+// tokens).  Every workgroup reads the activations of the groups it forms
+// beside its rows, two bytes for each weight byte at four groups.  Measured
+// with four groups / as many as needed, us per launch: q/k/v/g 13.1 / 10.0 at
+// one stream, 13.1 / 11.5 at 16, 14.1 / 12.8 at 32; gate/up 14.7 / 12.6, 15.6 /
+// 13.6, 16.2 / 14.8; down 8.1 / 5.6, 8.1 / 6.3, 8.5 / 7.1; LM head 29 / 25,
+// 32 / 27, 35 / 31.
+template <int RT, int KT, int NW, int S, int EPI>
+void launch_bgemm(int n, dim3 grid, const u32x4 *w, const void *x, const BEpi &ep, hipStream_t s) {
     const u32x4 *x4 = reinterpret_cast<const u32x4 *>(x);
-    if (lm_rt(e) == 4)
-        hipLaunchKernelGGL((k_bgemm<4, kKtH, 4, 1, EPI_LM>), dim3(lm_wgs(e)), dim3(kT), 0, s, e->w_lm, x4, ep);
+    const dim3 block(NW * 64);
+    if (n <= 16)
+        hipLaunchKernelGGL((k_bgemm<RT, KT, NW, S, EPI, 1>), grid, block, 0, s, w, x4, ep);
+    else if (n <= 32)
+        hipLaunchKernelGGL((k_bgemm<RT, KT, NW, S, EPI, 2>), grid, block, 0, s, w, x4, ep);
+    else if (n <= 48)
+        hipLaunchKernelGGL((k_bgemm<RT, KT, NW, S, EPI, 3>), grid, block, 0, s, w, x4, ep);
     else
-        hipLaunchKernelGGL((k_bgemm<2, kKtH, 4, 1, EPI_LM>), dim3(lm_wgs(e)), dim3(kT), 0, s, e->w_lm, x4, ep);
+        hipLaunchKernelGGL((k_bgemm<RT, KT, NW, S, EPI, 4>), grid, block, 0, s, w, x4, ep);
+}
+void launch_lm_gemm(GDNBatchEngine *e, const BEpi &ep, const void *x, hipStream_t s) {
+    const dim3 grid(lm_wgs(e));
+    if (lm_rt(e) == 4) launch_bgemm<4, kKtH, 4, 1, EPI_LM>(ep.n_streams, grid, e->w_lm, x, ep, s);
+    else launch_bgemm<2, kKtH, 4, 1, EPI_LM>(ep.n_streams, grid, e->w_lm, x, ep, s);
+}
+
+// Gate/up for n streams or tokens in `blocks` blocks of 64.
+void launch_bgu(int n, int blocks, const u32x4 *w, const u32x4 *x, uint16_t *x_next, hipStream_t s) {
+    const dim3 grid(kGuWgs, blocks), block(kGuWaves * 64);
+    if (n <= 16) hipLaunchKernelGGL((k_bgu<kGuWaves, 1>), grid, block, 0, s, w, x, x_next, n);
+    else if (n <= 32) hipLaunchKernelGGL((k_bgu<kGuWaves, 2>), grid, block, 0, s, w, x, x_next, n);
+    else if (n <= 48) hipLaunchKernelGGL((k_bgu<kGuWaves, 3>), grid, block, 0, s, w, x, x_next, n);
+    else hipLaunchKernelGGL((k_bgu<kGuWaves, 4>), grid, block, 0, s, w, x, x_next, n);
 }
 
 int b_check_shape(const GDNWeightHeader *c) {
@@ -2234,8 +2262,7 @@ void launch_qkvg(GDNBatchEngine *e, int l, hipStream_t s) {
     ep.sgate = e->sgate;
     ep.tails = b_tails(e, l);
     ep.conv_w = b_aux(e, l) + kAuxConv;
-    hipLaunchKernelGGL((k_bgemm<2, kKtH, 8, 1, EPI_QKVG>), dim3(4 * kH / 32), dim3(8 * 64), 0, s, e->w_qkvg[l],
-                       reinterpret_cast<const u32x4 *>(e->x_h), ep);
+    launch_bgemm<2, kKtH, 8, 1, EPI_QKVG>(e->streams, dim3(4 * kH / 32), e->w_qkvg[l], e->x_h, ep, s);
 }
 void launch_recur(GDNBatchEngine *e, int l, hipStream_t s) {
     hipLaunchKernelGGL((k_brecur<kRecCols>), dim3(kNH * (kHD / kRecCols), e->streams), dim3(2 * kRecCols), 0, s,
@@ -2251,16 +2278,14 @@ void launch_o(GDNBatchEngine *e, int l, hipStream_t s) {
     ep.n_rows = kH;
     ep.y = e->ypart;
     ep.y_rows = kMaxB;
-    hipLaunchKernelGGL((k_bgemm<kRtO, kKtH, 4, kSplitO, EPI_RAW>), dim3(kH / (16 * kRtO), kSplitO), dim3(kT), 0, s,
-                       e->w_o[l], reinterpret_cast<const u32x4 *>(e->x_o), ep);
+    launch_bgemm<kRtO, kKtH, 4, kSplitO, EPI_RAW>(e->streams, dim3(kH / (16 * kRtO), kSplitO), e->w_o[l], e->x_o, ep, s);
 }
 void launch_mlp_norm(GDNBatchEngine *e, int l, hipStream_t s) {
     const BNorm p = bnorm(e, e->ypart, b_aux(e, l) + kAuxMlpNorm, e->x_h, -1, l, l);
     hipLaunchKernelGGL((k_bnorm<kSplitO, false, false>), dim3(e->streams), dim3(kT), 0, s, p);
 }
 void launch_gu(GDNBatchEngine *e, int l, hipStream_t s) {
-    hipLaunchKernelGGL(k_bgu<kGuWaves>, dim3(kGuWgs), dim3(kGuWaves * 64), 0, s, e->w_gu[l],
-                       reinterpret_cast<const u32x4 *>(e->x_h), e->x_d, e->streams);
+    launch_bgu(e->streams, 1, e->w_gu[l], reinterpret_cast<const u32x4 *>(e->x_h), e->x_d, s);
 }
 void launch_down(GDNBatchEngine *e, int l, hipStream_t s) {
     BEpi ep{};
@@ -2268,8 +2293,8 @@ void launch_down(GDNBatchEngine *e, int l, hipStream_t s) {
     ep.n_rows = kH;
     ep.y = e->ypart;
     ep.y_rows = kMaxB;
-    hipLaunchKernelGGL((k_bgemm<kRtDown, kKtI, 4, kSplitDown, EPI_RAW>), dim3(kH / (16 * kRtDown), kSplitDown),
-                       dim3(kT), 0, s, e->w_down[l], reinterpret_cast<const u32x4 *>(e->x_d), ep);
+    launch_bgemm<kRtDown, kKtI, 4, kSplitDown, EPI_RAW>(e->streams, dim3(kH / (16 * kRtDown), kSplitDown),
+                                                        e->w_down[l], e->x_d, ep, s);
 }
 // After layer l's down projection: h = R(h + y), then the next layer's
 // attention norm with its a/b rows, or the final norm.
@@ -2460,8 +2485,7 @@ int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int ro
         ep.n_rows = rows;
         ep.y = y;
         ep.y_rows = y_rows;
-        hipLaunchKernelGGL((k_bgemm<2, KT, NW, S, EPI_RAW>), dim3(rows / 32, S, blocks), dim3(NW * 64), 0, s, w, x,
-                           ep);
+        launch_bgemm<2, KT, NW, S, EPI_RAW>(n, dim3(rows / 32, S, blocks), w, x, ep, s);
         return S;
     }
     if (route == P_PLANES) {
@@ -2480,8 +2504,7 @@ static_assert(kRtO == 2 && kRtDown == 2, "o_proj and down in 32-row blocks");
 
 void launch_p_gu(PRoute route, const u32x4 *w, const u32x4 *x, uint16_t *x_next, int n, hipStream_t s) {
     if (route == P_STEP)
-        hipLaunchKernelGGL(k_bgu<kGuWaves>, dim3(kGuWgs, (n + kMaxB - 1) / kMaxB), dim3(kGuWaves * 64), 0, s, w, x,
-                           x_next, n);
+        launch_bgu(n, (n + kMaxB - 1) / kMaxB, w, x, x_next, s);
     else
         hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, (n + kPgTok - 1) / kPgTok), dim3(kPgW * 64), 0, s, w, x, x_next, n);
 }
@@ -2982,7 +3005,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
             hipLaunchKernelGGL((k_bgemm<kRtDown, kKtI, 4, kSplitDown, EPI_RAW>), dim3(N / 32, kSplitDown),
                                dim3(kT), 0, 0, w4, xb4, ep);
         if (kind == 3)
-            hipLaunchKernelGGL(k_bgu<kGuWaves>, dim3(kGuWgs), dim3(kGuWaves * 64), 0, 0, w4, xb4,
+            hipLaunchKernelGGL((k_bgu<kGuWaves>), dim3(kGuWgs), dim3(kGuWaves * 64), 0, 0, w4, xb4,
                                static_cast<uint16_t *>(dr) + (size_t)b * kMaxB * kI, kMaxB);
     }
     GDN_HIP(hipGetLastError());

@@ -339,6 +339,29 @@ def test_streams_are_independent(model):
         one.free()
 
 
+@pytest.mark.parametrize("nb", [1, 16, 17, 32, 33, 48, 49])
+def test_stream_counts_at_group_edges(nb):
+    """A step forms only the 16-stream groups that hold its streams: stream
+    counts at the edges of one to four groups, a 2-layer step's tokens, logits
+    and states equal to a 64-stream engine's bit for bit."""
+    m = g.Model.synth(num_layers=2, seed=6, std=0.02, bf16=True)
+    few, full = g.BatchState(m, nb), g.BatchState(m, B)
+    rng = np.random.default_rng(nb)
+    try:
+        for _ in range(2):
+            toks = rng.integers(0, m.config.vocab_size, B).astype(np.int32)
+            a, b = few.step(toks[:nb]), full.step(toks)
+            assert (a == b[:nb]).all()
+        for s in {0, nb // 2, nb - 1}:
+            assert same_bits(few.logits(s), full.logits(s))
+            for x, y in zip(few.save_stream_state(s), full.save_stream_state(s)):
+                assert same_bits(x, y)
+    finally:
+        few.free()
+        full.free()
+        m.free()
+
+
 def test_batch_graph_eager_and_teacher_forced(model):
     nb, steps = 16, 3
     tokens = g.synth_tokens(steps * nb, 24, 0).reshape(steps, nb)
