@@ -517,6 +517,35 @@ struct BNorm {
 // kNH / kAbSplit * j .. (a 32 KB slice of the 128 KB of rows, requested
 // before the norm's first wait on memory); workgroup 0 alone writes the
 // residual, to h_out != h_in, and the X tiles.
+// beta and decay (head_scalars) of TOK tokens x HEADS heads of a workgroup:
+// wave 0's threads form the betas, wave 1's the decays, so the two serial
+// evaluations of the reference's transcendentals run side by side.  The
+// heads' parameters are requested at the kernel's start (read), where they
+// were loaded behind the a/b chains.
+struct HeadParams {
+    float a_log = 0.0f, dt_bias = 0.0f;
+    template <int HEADS>
+    __device__ __forceinline__ void read(int t, int h0, const float *__restrict__ al, const float *__restrict__ dt) {
+        if ((t >> 6) == 1) {
+            const int hd = h0 + (t & 63) % HEADS;
+            a_log = al[hd];
+            dt_bias = dt[hd];
+        }
+    }
+    // abv[token][row]: the a rows, then the b rows; bd[token][16]
+    template <int HEADS, int TOK>
+    __device__ __forceinline__ void write(int t, int h0, int n, const float *abv, int rows, float *__restrict__ bd,
+                                          const Exp2Lds &tab) const {
+        static_assert(HEADS * TOK <= 64, "one wave");
+        const int i = t & 63, m = i / HEADS, hh = i % HEADS;
+        if (i >= HEADS * TOK || m >= n) return;
+        float *out = bd + m * 16 + 2 * (h0 + hh);
+        if ((t >> 6) == 0)
+            out[0] = sigmoid_ref(abv[m * rows + HEADS + hh], tab);
+        else if ((t >> 6) == 1)
+            out[1] = exp_ref(-exp_ref(a_log, tab) * softplus_ref(abv[m * rows + hh] + dt_bias, tab), tab);
+    }
+};
 constexpr int kAbSplit = 4;
 constexpr int kAbHeads = kNH / kAbSplit;  // heads per a/b workgroup
 static_assert(kNH % kAbSplit == 0 && (2 * kAbHeads * kH) % (4 * kT) == 0 && 2 * kAbHeads <= kT,
@@ -529,9 +558,15 @@ __global__ __launch_bounds__(kT) void k_bnorm(BNorm p) {
     __shared__ __attribute__((aligned(16))) float tab[ABR][64][2];
     __shared__ float abv[ABR];
     __shared__ float scale_s;
+    __shared__ uint64_t exp2_lds[AB ? 32 : 1];  // expf's table for beta and decay
     const int m = blockIdx.x, t = threadIdx.x, e0 = 8 * t;
     const int j = AB ? (int)blockIdx.y : 0;
     const bool writer = j == 0;
+    HeadParams hp;
+    if constexpr (AB) {
+        fill_exp2_lds_imm(exp2_lds);
+        hp.read<kAbHeads>(t, kAbHeads * j, p.a_log, p.dt_bias);
+    }
     const f32x4 *w4 = reinterpret_cast<const f32x4 *>(p.w + e0);
     const f32x4 wa = w4[0], wb = w4[1];
     float hv[8];
@@ -665,13 +700,7 @@ __global__ __launch_bounds__(kT) void k_bnorm(BNorm p) {
             abv[t] = rne_bf16(acc);
         }
         __syncthreads();
-        if (t < kAbHeads) {
-            const int hd = kAbHeads * j + t;
-            float beta, decay;
-            head_scalars(abv[t], abv[kAbHeads + t], p.a_log[hd], p.dt_bias[hd], beta, decay);
-            p.bd[m * 16 + 2 * hd] = beta;
-            p.bd[m * 16 + 2 * hd + 1] = decay;
-        }
+        hp.write<kAbHeads, 1>(t, kAbHeads * j, 1, abv, ABR, p.bd + m * 16, Exp2Lds{exp2_lds});
     }
 }
 
@@ -692,6 +721,8 @@ __global__ __launch_bounds__(kT) void k_pab(const float *__restrict__ xn, int n,
     __shared__ uint64_t exp2_lds[32];
     const int j = blockIdx.x, m0 = (int)blockIdx.y * kPabTok, t = threadIdx.x;
     fill_exp2_lds_imm(exp2_lds);
+    HeadParams hp;
+    hp.read<kAbHeads>(t, kAbHeads * j, a_log, dt_bias);
     // local row r: the a row of head kAbHeads j + r (r < kAbHeads), else the
     // b row of head kAbHeads j + r - kAbHeads
     auto ab_row = [&](int r) { return r < kAbHeads ? kAbHeads * j + r : kNH + kAbHeads * j + r - kAbHeads; };
@@ -749,17 +780,7 @@ __global__ __launch_bounds__(kT) void k_pab(const float *__restrict__ xn, int n,
         }
     }
     __syncthreads();
-    if (t < kPabTok * kAbHeads) {
-        const int mt = t / kAbHeads, hh = t % kAbHeads, m = m0 + mt;
-        if (m < n) {
-            const int hd = kAbHeads * j + hh;
-            float beta, decay;
-            head_scalars(abv[mt][hh], abv[mt][kAbHeads + hh], a_log[hd], dt_bias[hd], beta, decay,
-                         Exp2Lds{exp2_lds});
-            bd[m * 16 + 2 * hd] = beta;
-            bd[m * 16 + 2 * hd + 1] = decay;
-        }
-    }
+    hp.write<kAbHeads, kPabTok>(t, kAbHeads * j, n - m0, &abv[0][0], ABR, bd + m0 * 16, Exp2Lds{exp2_lds});
 }
 
 // Per (head, stream): the output RMSNorm times the gate and sigmoid(gate)
@@ -1006,7 +1027,7 @@ __global__ __launch_bounds__(kConvT) void k_pconv(const float *__restrict__ raw,
 }
 
 // Per (head, token): the q/k L2 norms and alpha of the recurrence, in the
-// batch-1 tree order (k_brecur's first phase), for tokens kQkTok y .. +
+// batch-1 tree order, for tokens kQkTok y .. +
 // kQkTok - 1 of n, their loads requested together (a token past n re-reads
 // token n - 1, unused).
 constexpr int kQkTok = 4;
