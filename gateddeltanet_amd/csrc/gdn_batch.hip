@@ -25,7 +25,7 @@
 // Per layer (8 launches):
 //   k_bgemm<QKVG>  q,k,v,g rows; epilogue: BF16 rounding, conv + SiLU with
 //                  each stream's tails, gate and sigmoid(gate)
-//   k_brecur       the recurrence per (head, stream, 128 columns), state in registers
+//   k_brecur       the recurrence per (head, stream, 64 columns), state in registers
 //   k_bonorm       per (head, stream) output RMSNorm * gate -> X
 //   k_bgemm<RAW>   o_proj in 4 K splits -> split sums
 //   k_bnorm        h = R(h + R(y)), MLP RMSNorm -> X
@@ -55,7 +55,7 @@ namespace bt {
 
 constexpr int kMaxB = GDN_MAX_STREAMS;  // streams = the 64 B-operand columns
 static_assert(kMaxB == 64, "four 16-stream groups per MFMA B operand");
-constexpr int kRecCols = 128;  // state columns per multi-stream recurrence workgroup
+constexpr int kRecCols = 64;  // state columns per multi-stream recurrence workgroup
 constexpr int kSplitO = 4;              // K splits of o_proj (16 k tiles each)
 constexpr int kSplitDown = 4;           // K splits of the down projection (44 k tiles each)
 constexpr int kRtO = 2;                 // 16-row tiles per o_proj workgroup
@@ -841,85 +841,84 @@ __global__ __launch_bounds__(kT) void k_bonorm(const float *__restrict__ attn, c
 }
 constexpr int kOnTok = 4;  // prefill tokens per output-norm workgroup
 
-// The recurrence of one (head, stream, CW-column group) per workgroup of
-// 2 CW threads, with the batch-1 arithmetic (gdn_island_prep / read /
-// update, gdn_model.cpp:2376-2933).  Wave w owns state column
-// c0 + 64 (w % (CW / 64)) + lane and rows 128 (w / (CW / 64)) .. + 127,
-// held in registers from load to store: the first half of the waves run
-// the r and p chains over rows 0..127, hand the partial sums to the second
-// half through LDS, which continue over rows 128..255 (the chain order is
-// j = 0..255 as in the reference) and form delta and o; every wave then
-// writes its rows of S' = decay * S + kn (x) delta.  The q/k norms and alpha
-// use the batch-1 tree order; every column group of a head computes them.
-// 128-column groups (256 threads) leave room for three workgroups per CU,
-// so one group's stores overlap another's loads.
-template <int CW>
-__global__ __launch_bounds__(2 * CW) void k_brecur(const float *__restrict__ qkv, const float *__restrict__ bd,
-                                                   float *__restrict__ state, float *__restrict__ attn) {
-    static_assert(CW == 128 || CW == 256, "column groups of 128 or 256");
-    constexpr int RH = kHD / 2;   // rows per wave
-    constexpr int WPR = CW / 64;  // waves per 128-row half
-    __shared__ float qn[kHD], kn[kHD], rpart[CW], ppart[CW], dl[CW];
-    __shared__ float red[8], red2[4];
-    const int cg = blockIdx.x % (kHD / CW), h = blockIdx.x / (kHD / CW), m = blockIdx.y;
-    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-    const int lc = (w % WPR) * 64 + lane, col = cg * CW + lc, r0 = (w / WPR) * RH;
+// The recurrence of one (head, stream, 64-column group) per workgroup of 256
+// threads, with the batch-1 arithmetic (gdn_island_prep / read / update,
+// gdn_model.cpp:2376-2933).  Wave w owns state rows 64 w .. + 63 of the
+// group's columns (a column per lane), held in registers from load to store.
+// Every wave forms its products S[j][i] kn[j] and S[j][i] qn[j] as its rows
+// arrive; only the adds of the chains, in the reference's order j = 0..255,
+// go from wave to wave: in turn s wave s continues the r chain, wave s - 1 the
+// p chain behind it, the partial sums through LDS.  Then every wave forms
+// delta (the last one o) and writes its rows of S' = decay * S + kn (x) delta.
+// The norms and alpha are each wave's own (four values per lane, then the
+// lanes: the batch-1 tree), so nothing waits for a barrier before the chains.
+// What bounds it: at 64 streams the state's read and write (268 MB, 5.5 TB/s);
+// at few streams the latency of load, chains and store.  In 128-column groups
+// whose waves multiplied inside the chains: 10.7 -> 5.3 us at one stream, 17.3
+// -> 13.4 at 16, 55.7 -> 49.2 at 64 (21.4 -> 22.4 at 24, where 768 workgroups
+// fill the 512 places one and a half times).
+__global__ __launch_bounds__(kT, 2) void k_brecur(const float *__restrict__ qkv, const float *__restrict__ bd,
+                                                  float *__restrict__ state, float *__restrict__ attn) {
+    constexpr int RW = kHD / 4;  // rows per wave
+    __shared__ __attribute__((aligned(16))) float kq[4][2][kHD];  // each wave's kn, qn
+    __shared__ float rs[kRecCols], ps[kRecCols];
+    const int cg = blockIdx.x % (kHD / kRecCols), h = blockIdx.x / (kHD / kRecCols), m = blockIdx.y;
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63, col = cg * kRecCols + lane;
     const float *qp = qkv + (size_t)m * 3 * kH + h * kHD;
-    float *S = state + (size_t)m * kLayerState + (size_t)h * kHD * kHD + col;
-    float sv[RH];
+    const f32x4 q4 = *reinterpret_cast<const f32x4 *>(qp + 4 * lane);
+    const f32x4 k4 = *reinterpret_cast<const f32x4 *>(qp + kH + 4 * lane);
+    float *S = state + (size_t)m * kLayerState + (size_t)h * kHD * kHD + (size_t)(RW * w) * kHD + col;
+    float sv[RW];
 #pragma unroll
-    for (int j = 0; j < RH; ++j) sv[j] = S[(size_t)(r0 + j) * kHD];
-    const float beta = bd[m * 16 + 2 * h], decay = bd[m * 16 + 2 * h + 1];
-    float q = 0.0f, k = 0.0f;
-    if (t < kHD) {
-        q = qp[t];
-        k = qp[kH + t];
-        const float qs = wave_tree64(q * q), ks = wave_tree64(k * k);
-        if (lane == 0) {
-            red[w] = qs;
-            red[4 + w] = ks;
+    for (int j = 0; j < RW; ++j) sv[j] = S[(size_t)j * kHD];
+    const float beta = bd[m * 16 + 2 * h], decay = bd[m * 16 + 2 * h + 1], v = qp[2 * kH + col];
+    auto tree = [](f32x4 x, f32x4 y) { return wave_tree64((x.x * y.x + x.y * y.y) + (x.z * y.z + x.w * y.w)); };
+    const float q_inv = 1.0f / __builtin_sqrtf(tree(q4, q4) + 1e-6f);
+    const float k_inv = 1.0f / __builtin_sqrtf(tree(k4, k4) + 1e-6f);
+    const f32x4 qn = {q4.x * q_inv, q4.y * q_inv, q4.z * q_inv, q4.w * q_inv};
+    const f32x4 kn = {k4.x * k_inv, k4.y * k_inv, k4.z * k_inv, k4.w * k_inv};
+    const float alpha = tree(qn, kn);
+    *reinterpret_cast<f32x4 *>(&kq[w][0][4 * lane]) = kn;
+    *reinterpret_cast<f32x4 *>(&kq[w][1][4 * lane]) = qn;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float pr[RW], pp[RW];
+#pragma unroll
+    for (int j = 0; j < RW; j += 4) {
+        const f32x4 kv = *reinterpret_cast<const f32x4 *>(&kq[w][0][RW * w + j]);
+        const f32x4 qv = *reinterpret_cast<const f32x4 *>(&kq[w][1][RW * w + j]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            pr[j + e] = sv[j + e] * kv[e];
+            pp[j + e] = sv[j + e] * qv[e];
+            // formed here, not sunk into the chains' branches
+            asm volatile("" : "+v"(pr[j + e]), "+v"(pp[j + e]));
         }
     }
-    __syncthreads();
-    if (t < kHD) {
-        const float q_sq = (red[0] + red[1]) + (red[2] + red[3]);
-        const float k_sq = (red[4] + red[5]) + (red[6] + red[7]);
-        const float qv = q * (1.0f / __builtin_sqrtf(q_sq + 1e-6f));
-        const float kv = k * (1.0f / __builtin_sqrtf(k_sq + 1e-6f));
-        qn[t] = qv;
-        kn[t] = kv;
-        const float qk = wave_tree64(qv * kv);
-        if (lane == 0) red2[w] = qk;
-    }
-    __syncthreads();
-    if (w < WPR) {
-        float r = 0.0f, p = 0.0f;
 #pragma unroll
-        for (int j = 0; j < RH; ++j) {
-            r = r + sv[j] * kn[j];
-            p = p + sv[j] * qn[j];
+    for (int s = 0; s < 5; ++s) {
+        if (w == s) {
+            float r = s ? rs[lane] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < RW; ++j) r = r + pr[j];
+            rs[lane] = r;
+        } else if (w == s - 1) {
+            float p = s > 1 ? ps[lane] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < RW; ++j) p = p + pp[j];
+            ps[lane] = p;
         }
-        rpart[lc] = r;
-        ppart[lc] = p;
+        if (s < 4) __syncthreads();
     }
-    __syncthreads();
-    if (w >= WPR) {
-        float r = rpart[lc], p = ppart[lc];
+    const float d = beta * (v - decay * rs[lane]);
+    if (w == 3) attn[(size_t)m * kH + h * kHD + col] = rne_bf16(0.0625f * (decay * ps[lane] + alpha * d));
 #pragma unroll
-        for (int j = 0; j < RH; ++j) {
-            r = r + sv[j] * kn[RH + j];
-            p = p + sv[j] * qn[RH + j];
-        }
-        const float alpha = (red2[0] + red2[1]) + (red2[2] + red2[3]);
-        const float delta = beta * (qp[2 * kH + col] - decay * r);
-        const float o = 0.0625f * (decay * p + alpha * delta);
-        dl[lc] = delta;
-        attn[(size_t)m * kH + h * kHD + col] = rne_bf16(o);
+    for (int j = 0; j < RW; j += 4) {
+        const f32x4 kv = *reinterpret_cast<const f32x4 *>(&kq[w][0][RW * w + j]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[(size_t)(j + e) * kHD] = decay * sv[j + e] + kv[e] * d;
     }
-    __syncthreads();
-    const float d = dl[lc];
-#pragma unroll
-    for (int j = 0; j < RH; ++j) S[(size_t)(r0 + j) * kHD] = decay * sv[j] + kn[r0 + j] * d;
 }
 
 // ---------------------------------------------------------------- prefill
@@ -2286,8 +2285,8 @@ void launch_qkvg(GDNBatchEngine *e, int l, hipStream_t s) {
     launch_bgemm<2, kKtH, 8, 1, EPI_QKVG>(e->streams, dim3(4 * kH / 32), e->w_qkvg[l], e->x_h, ep, s);
 }
 void launch_recur(GDNBatchEngine *e, int l, hipStream_t s) {
-    hipLaunchKernelGGL((k_brecur<kRecCols>), dim3(kNH * (kHD / kRecCols), e->streams), dim3(2 * kRecCols), 0, s,
-                       e->qkv, e->bd, b_state(e, l), e->attn);
+    hipLaunchKernelGGL(k_brecur, dim3(kNH * (kHD / kRecCols), e->streams), dim3(kT), 0, s, e->qkv, e->bd,
+                       b_state(e, l), e->attn);
 }
 void launch_onorm(GDNBatchEngine *e, int l, hipStream_t s) {
     hipLaunchKernelGGL(k_bonorm<1>, dim3(kNH, e->streams), dim3(kT), 0, s, e->attn, e->gate, e->sgate,

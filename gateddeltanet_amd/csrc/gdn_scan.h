@@ -28,6 +28,18 @@ __device__ __forceinline__ float chain256(const float (&p)[16]) {
     return acc;
 }
 
+// From the chains' sums in lane 15 of the rows (r in rows 0 and 2, p in the
+// row after it): delta in every lane of the column's two rows, and o in lane
+// 15 of its p row.  (row_newbcast:15 spreads a row's lane 15 over the row,
+// row_bcast:15 over the next row.)
+__device__ __forceinline__ void scan_delta_o(float acc, float beta, float decay, float alpha, float v, float &delta,
+                                             float &o) {
+    const float d = beta * (v - decay * acc);
+    const int dr = __builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x15f, 0xf, 0xf, true);
+    delta = __int_as_float(__builtin_amdgcn_update_dpp(dr, __float_as_int(d), 0x142, 0xa, 0xf, false));
+    o = 0.0625f * (decay * acc + alpha * delta);
+}
+
 // The scan.  A workgroup is four independent waves (one per SIMD), a wave
 // two state columns, and each of the wave's four 16-lane rows one 256-add
 // chain of the reference's order: row 2 c + 0 sums r of column c (S^T k),
@@ -145,14 +157,8 @@ __device__ __forceinline__ void scan_block(const ScanArgs a, const Scal scal, vo
             const float v = lds.v[b][m][lc], beta = scl.x, decay = scl.y, alpha = scl.z;
             read_mul(b, m + 1 < n ? m + 1 : m);
             const float acc = chain256(p);  // lane 15 of the row
-            // delta in lane 15 of the r rows, from there to every lane of
-            // the row (row_newbcast:15) and of the p row after it
-            // (row_bcast:15)
-            const float d = beta * (v - decay * acc);
-            const int dr = __builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x15f, 0xf, 0xf, true);
-            const float delta =
-                __int_as_float(__builtin_amdgcn_update_dpp(dr, __float_as_int(d), 0x142, 0xa, 0xf, false));
-            const float o = 0.0625f * (decay * acc + alpha * delta);
+            float delta, o;
+            scan_delta_o(acc, beta, decay, alpha, v, delta, o);
             // lane m of a p row keeps token m's o
             const float ob = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o), 0x15f, 0xf, 0xf, true));
             oacc = i16 == m ? ob : oacc;
