@@ -131,12 +131,12 @@ __device__ __forceinline__ float log1p_ref(float x) { return gdn_libm::gdn_log1p
 // gdn_sigmoid / gdn_silu / gdn_softplus, gdn_model.cpp:1307-1330.
 template <class Tab = Exp2Const>
 __device__ __forceinline__ float sigmoid_ref(float x, const Tab &tab = Tab()) {
-    if (x >= 0.0f) {
-        const float z = exp_ref(-x, tab);
-        return 1.0f / (1.0f + z);
-    }
-    const float z = exp_ref(x, tab);
-    return z / (1.0f + z);
+    // 1 / (1 + exp(-x)) for x >= 0, exp(x) / (1 + exp(x)) below, as one
+    // exponential and one division with selected operands: as branches, a wave
+    // with both signs ran two of each
+    const bool pos = x >= 0.0f;
+    const float z = exp_ref(pos ? -x : x, tab);
+    return (pos ? 1.0f : z) / (1.0f + z);
 }
 template <class Tab = Exp2Const>
 __device__ __forceinline__ float silu_ref(float x, const Tab &tab = Tab()) { return x * sigmoid_ref(x, tab); }

@@ -93,25 +93,27 @@ GDN_HD inline float gdn_expf_t(float x, const Tab &tab) {
     constexpr double kC0 = 0x1.c6af84b912394p-5 / kN / kN / kN;
     constexpr double kC1 = 0x1.ebfce50fac4f3p-3 / kN / kN;
     constexpr double kC2 = 0x1.62e42ff0c52d6p-1 / kN;
-    const uint32_t abstop = (bits_f(x) >> 20) & 0x7ffu;
-    if (abstop >= (bits_f(88.0f) >> 20)) {  // |x| >= 88, infinities, NaN
-        if (bits_f(x) == 0xff800000u) return 0.0f;
-        if (abstop >= 0x7f8u) return x + x;
-        if (x > 0x1.62e42ep6f) return from_bits_f(0x7f800000u);  // beyond log(2^128)
-        if (x < -0x1.9fe368p6f) return 0.0f;                     // below log(2^-150)
-    }
     const double xd = (double)x;
     double kd = fused(kInvLn2N, xd, kShift);  // k in the low mantissa bits
-    const uint64_t ki = bits_d(kd);
+    const uint32_t ki = (uint32_t)bits_d(kd);
     kd -= kShift;
     const double r = fused(kInvLn2N, xd, -kd);
-    const double s = from_bits_d(tab((int)(ki % 32u)) + (ki << 47));
+    // table entry + (k << 47): the shifted k has nothing below bit 47, so only
+    // the upper word changes
+    const uint64_t t = tab((int)(ki % 32u));
+    const double s = from_bits_d((uint64_t)((uint32_t)(t >> 32) + (ki << 15)) << 32 | (uint32_t)t);
     const double z = fused(kC0, r, kC1);
     const double r2 = r * r;
     double y = fused(kC2, r, 1.0);
     y = fused(z, r2, y);
     y = y * s;
-    return (float)y;
+    // the method's cases of large |x| and of NaN, taken as selects: a branch
+    // around them would split the wave and keep neighbouring evaluations from
+    // overlapping
+    float v = (float)y;
+    v = x > 0x1.62e42ep6f ? from_bits_f(0x7f800000u) : v;  // beyond log(2^128)
+    v = x < -0x1.9fe368p6f ? 0.0f : v;                     // below log(2^-150)
+    return x != x ? x + x : v;
 }
 
 GDN_HD inline float gdn_expf(float x) { return gdn_expf_t(x, Exp2Const{}); }
