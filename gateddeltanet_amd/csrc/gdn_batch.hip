@@ -1630,12 +1630,28 @@ __device__ __forceinline__ int pg_tile(int j) {
 // XCDs round robin in launch order; when the grid allows, the 32 that one
 // XCD runs together cover 4 row tiles x 8 token tiles (a "super tile"), so
 // that XCD's L2 serves each weight tile to 8 of them and each activation
-// tile to 4.  Otherwise the plain (blockIdx.x, blockIdx.y).
+// tile to 4.  The super tiles that are left over when their number is no
+// multiple of 8 are cut in equal parts over the XCDs (or run in order).
+// Otherwise the plain (blockIdx.x, blockIdx.y).
 __device__ __forceinline__ void pg_place(int &rt, int &tt) {
     const int R = gridDim.x, C = gridDim.y, L = blockIdx.x + R * blockIdx.y;
-    if (R % 4 == 0 && C % 8 == 0 && (R * C) % 256 == 0) {
-        const int x = L & 7, s = L >> 3;
-        const int u = 8 * (s >> 5) + x, q = s & 31, gr = R / 4;
+    if (R % 4 == 0 && C % 8 == 0) {
+        const int gr = R / 4, ns = gr * (C / 8), whole = ns & ~7, rem = ns & 7;
+        int u, q;
+        if (L < whole * 32) {
+            u = 8 * ((L >> 3) >> 5) + (L & 7);
+            q = (L >> 3) & 31;
+        } else {
+            const int r = L - whole * 32;
+            if (rem == 1 || rem == 2 || rem == 4) {
+                const int parts = 8 / rem, x = r & 7;
+                u = whole + x / parts;
+                q = (x % parts) * (32 / parts) + (r >> 3);
+            } else {
+                u = whole + (r >> 5);
+                q = r & 31;
+            }
+        }
         rt = 4 * (u % gr) + (q & 3);
         tt = 8 * (u / gr) + (q >> 2);
     } else {
@@ -1778,15 +1794,18 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
 // (pa_fills), where k_pgemm's twice as many workgroups do better.
 constexpr int kPaRows = 32 * kPgW;  // rows per workgroup
 constexpr int kPaD = 2;       // k tiles of operands in flight
-template <int KT, int NW, int S>
-__global__ __launch_bounds__(kPgW * 64) void k_pgemm_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
-                                                       float *__restrict__ y, int n_rows) {
+template <int KT, int NW, int S, bool SWIGLU>
+__device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
+                                              float *__restrict__ y, uint16_t *__restrict__ x_next, int n_rows,
+                                              int n_tok) {
     constexpr int R = kPaRows / 16 / kPgW;  // 16-row tiles per wave
     constexpr int T = kPgTok / 16;          // 16-token groups per wave
     constexpr int GT = kPgW * 64, BU = T * 64, PB = BU / GT;
     constexpr int NB = R * T, KTS = KT / S, KTW = KTS / NW;
     static_assert(R == 2 && BU % GT == 0 && KT % S == 0 && KTS % NW == 0, "row and token tiles per workgroup");
     __shared__ u32x4 stg[2][BU];
+    __shared__ uint64_t exp2_lds[SWIGLU ? 32 : 1];  // expf's table for the SwiGLU epilogue
+    if constexpr (SWIGLU) fill_exp2_lds_imm(exp2_lds);
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
     int rt, tt;
     pg_place(rt, tt);
@@ -1867,7 +1886,7 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm_a(const u32x4 *__restrict__
             part[b] = cls == 0 ? chain[b] : part[b] + chain[b];
             chain[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
         }
-        if (cls == NW - 1) {
+        if (!SWIGLU && cls == NW - 1) {
             const bool first = c < NW;
 #pragma unroll
             for (int f = 0; f < R; ++f)
@@ -1875,7 +1894,57 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm_a(const u32x4 *__restrict__
                 for (int g = 0; g < T; ++g) *out(f, g) = first ? part[T * f + g] : *out(f, g) + part[T * f + g];
         }
     }
+    if constexpr (SWIGLU) {
+        // row tile 0: the gate rows of the wave's 16 channels, tile 1 their
+        // up rows, so a lane holds both of channels 4 (l / 16) .. + 3
+        // (gemv32_store SwiGLU branch, gdn_model.cpp:4751-4767)
+        const int ch = 16 * (kPgW * rt + w) + 4 * (l >> 4);
+        // one token group per trip, the next ones moved down (unrolled, the
+        // eight groups' SiLUs are 50 KB of code)
+#pragma unroll 1
+        for (int g = 0; g < T; ++g) {
+            uint32_t hv[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                hv[e] = bf16_daz_bits(rne_bf16(silu_ref(rne_bf16(part[0][e]), Exp2Lds{exp2_lds}) *
+                                               rne_bf16(part[T][e])));
+            if (m + 16 * g < n_tok)
+                *reinterpret_cast<uint2 *>(x_next + xt_index(m + 16 * g, ch, kI)) =
+                    make_uint2(hv[0] | (hv[1] << 16), hv[2] | (hv[3] << 16));
+#pragma unroll
+            for (int i = 0; i + 1 < T; ++i) {
+                part[i] = part[i + 1];
+                part[T + i] = part[T + i + 1];
+            }
+        }
+    }
 }
+template <int KT, int NW, int S>
+__global__ __launch_bounds__(kPgW * 64) void k_pgemm_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
+                                                       float *__restrict__ y, int n_rows) {
+    pgemm_a_block<KT, NW, S, false>(W, X, y, nullptr, n_rows, 0);
+}
+
+// Gate/up + SwiGLU on the same kernel: W in 32-row blocks of 16 channels'
+// gate rows then their up rows (k_gu_pairs), classes as k_bgu's, so the sums
+// are the step's; the first n_tok tokens are written.  All rows carry
+// weights, where the 44-row groups of k_pgu leave 4 of 48 empty, and a wave
+// reads 8 fragments from LDS per 16 MFMAs where k_pgu's reads 5 per 6.
+__global__ __launch_bounds__(kPgW * 64) void k_pgu_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
+                                                     uint16_t *__restrict__ x_next, int n_tok) {
+    pgemm_a_block<kKtH, kGuWaves, 1, true>(W, X, nullptr, x_next, 2 * kI, n_tok);
+}
+
+// One layer's gate/up weights from the step's 44-row groups (tile_gu) into
+// k_pgu_a's blocks: grid (kI / 16, kKtH), block of 128: entry (tile, lane) of
+// block b and k tile kt.
+__global__ __launch_bounds__(128) void k_gu_pairs(const u32x4 *__restrict__ src, u32x4 *__restrict__ dst) {
+    const int b = blockIdx.x, kt = blockIdx.y, up = threadIdx.x >> 6, l = threadIdx.x & 63;
+    const int ch = 16 * b + (l & 15), g = ch / kGuCh, r = ch % kGuCh, kq = l >> 4;
+    const int at = r < 16 ? 64 * up + 16 * kq + r : 128 + kq * kGuTail2 + (r - 16) + up * (kGuCh - 16);
+    dst[((size_t)b * kKtH + kt) * 128 + threadIdx.x] = src[((size_t)g * kKtH + kt) * kGuTileU4 + at];
+}
+
 
 // Gate/up + SwiGLU for channel groups 2 rt, +1 (k_bgu's layout and sums:
 // four classes of 16 k tiles) and tokens 128 tt .. +127 (pg_place; the
@@ -2019,6 +2088,9 @@ struct GDNBatchEngine {
     // the chunk matrices L and Mq, final hidden; X tiles of three widths)
     int seg_tokens = kSegDefault, seg_cap = 0;
     void *seg_mem = nullptr;
+    // k_pgu_a's copy of the gate/up weights, made at the first prefill
+    void *gu_mem = nullptr;
+    const u32x4 *w_gup[kMaxLayers] = {};
     float *s_h = nullptr, *s_y = nullptr, *s_qkv = nullptr, *s_gate = nullptr, *s_sgate = nullptr, *s_bd = nullptr,
           *s_attn = nullptr, *s_qn = nullptr, *s_kn = nullptr, *s_alpha = nullptr, *s_xn = nullptr;
     WyOps *s_wy = nullptr;
@@ -2434,6 +2506,21 @@ int seg_alloc(GDNBatchEngine *e) {
     return 0;
 }
 
+// k_pgu_a's layout of every layer's gate/up weights (46 MB a layer beside the
+// step's), formed on the device for the first segment that takes it and kept.
+int gu_pairs(GDNBatchEngine *e) {
+    if (e->gu_mem) return 0;
+    const size_t per = (size_t)2 * kI * kH * 2;
+    GDN_HIP(hipMalloc(&e->gu_mem, (size_t)e->layers * per));
+    for (int l = 0; l < e->layers; ++l) {
+        u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(e->gu_mem) + (size_t)l * per);
+        hipLaunchKernelGGL(k_gu_pairs, dim3(kI / 16, kKtH), dim3(128), 0, e->stream, e->w_gu[l], dst);
+        e->w_gup[l] = dst;
+    }
+    GDN_HIP(hipGetLastError());
+    return 0;
+}
+
 // A segment's norm: the residual of layer l's attention block in buffer
 // l & 1 (as in the step), segment-sized.
 BNorm seg_norm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_out, int ab_layer, int l_in,
@@ -2470,14 +2557,14 @@ enum PRoute {
     P_STEP,    // the decode step's kernels, a grid plane per 64-token block
     P_PLANES,  // k_pgemm with a workgroup per split (o_proj, down)
     P_TILE,    // k_pgemm / k_pgu, 128 tokens per workgroup
-    P_WIDE     // k_pgemm_a, once its grid (half of k_pgemm's) fills the CUs
+    P_WIDE     // k_pgemm_a, once its grid (half of k_pgemm's) fills the CUs; k_pgu_a
 };
 // Where the lines lie (us per launch, step / planes / tile at 64, 256, 512,
 // 1024, 2048 tokens):
 //   q/k/v/g  12 / - / 30   28 / - / 30    49 / - / 32    91 / - / 42   174 / - / 79
 //   o_proj    5 / 11 / 34    9 / 11 / 33   15 / 12 / 34   26 / 19 / 36   49 / 38 / 44
 //   down      9 / 20 / 71   18 / 20 / 69   30 / 22 / 70   54 / 37 / 75  103 / 69 / 85
-//   gate/up  15 / - / 30   33 / - / 31    57 / - / 43   107 / - / 83   207 / - / 165
+//   gate/up  15 / - / 30   33 / - / 31    57 / - / 45   107 / - / 83   207 / - / 151
 // The step's kernels re-read the weights per 64 tokens; the tile kernels leave
 // most CUs idle on short segments (16 workgroups for o_proj and down at up to
 // 128 tokens).  Planes cost the norm after them three more reads (12 against
@@ -2490,7 +2577,15 @@ PRoute route_o(int n) { return n <= 256 ? P_STEP : n <= 1536 ? P_PLANES : P_TILE
 PRoute route_down(int rows, int n) {
     return n <= 256 ? P_STEP : n <= 3072 ? P_PLANES : pa_fills(rows, n) ? P_WIDE : P_TILE;
 }
-PRoute route_gu(int n) { return n <= 192 ? P_STEP : P_TILE; }
+// k_pgu_a takes whole rounds of 256 workgroups (one per CU, 44 per 128 tokens),
+// about 39 us each; k_pgu (two per CU) about 8.5 us per 128 tokens and 14.
+// tile / wide: 512 tokens 46 / 44 us, 768 66 / 77, 1536 117 / 114, 2048 151 /
+// 119, 4096 280 / 226.
+bool pgu_a_pays(int n) {
+    const int tiles = (n + kPgTok - 1) / kPgTok, rounds = (2 * kI / kPaRows * tiles + 255) / 256;
+    return 78 * rounds <= 17 * tiles + 18;
+}
+PRoute route_gu(int n) { return n <= 192 ? P_STEP : pgu_a_pays(n) ? P_WIDE : P_TILE; }
 
 // A projection in 32-row blocks of KT k tiles, NW classes and S splits:
 // returns the planes of y (y_rows tokens each) that its consumer adds: S, or
@@ -2522,11 +2617,16 @@ int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int ro
 }
 static_assert(kRtO == 2 && kRtDown == 2, "o_proj and down in 32-row blocks");
 
-void launch_p_gu(PRoute route, const u32x4 *w, const u32x4 *x, uint16_t *x_next, int n, hipStream_t s) {
+// Gate/up on the step's layout w, or (P_WIDE) k_pgu_a's layout wp.
+void launch_p_gu(PRoute route, const u32x4 *w, const u32x4 *wp, const u32x4 *x, uint16_t *x_next, int n,
+                 hipStream_t s) {
+    const int tiles = (n + kPgTok - 1) / kPgTok;
     if (route == P_STEP)
         launch_bgu(n, (n + kMaxB - 1) / kMaxB, w, x, x_next, s);
+    else if (route == P_WIDE)
+        hipLaunchKernelGGL(k_pgu_a, dim3(2 * kI / kPaRows, tiles), dim3(kPgW * 64), 0, s, wp, x, x_next, n);
     else
-        hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, (n + kPgTok - 1) / kPgTok), dim3(kPgW * 64), 0, s, w, x, x_next, n);
+        hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, tiles), dim3(kPgW * 64), 0, s, w, x, x_next, n);
 }
 
 // The residual add and norm after o_proj or down.
@@ -2575,7 +2675,7 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
                            e->s_gate, e->s_sgate, b_aux(e, l) + kAuxONorm, e->eps, e->s_xo, n);
         const int po = launch_p_gemm<kKtH, 4, kSplitO>(route_o(n), e->w_o[l], xo, e->s_y, kH, n, e->seg_cap, s);
         launch_p_norm(seg_norm(e, e->s_y, b_aux(e, l) + kAuxMlpNorm, e->s_xh, -1, l, l), po, n, s);
-        launch_p_gu(route_gu(n), e->w_gu[l], xh, e->s_xd, n, s);
+        launch_p_gu(route_gu(n), e->w_gu[l], e->w_gup[l], xh, e->s_xd, n, s);
         const int pd =
             launch_p_gemm<kKtI, 4, kSplitDown>(route_down(kH, n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
         if (l + 1 < e->layers) {
@@ -2614,6 +2714,7 @@ int b_prefill(GDNBatchEngine *e, int slot, const int32_t *prompt, uint32_t n_tok
     int n = 0;
     for (uint32_t off = 0; off < n_tokens; off += seg) {
         n = (int)std::min<uint32_t>(seg, n_tokens - off);
+        if (route_gu(n) == P_WIDE && gu_pairs(e)) return -1;
         GDN_HIP(hipMemcpyAsync(e->s_tok, prompt + off, (size_t)n * sizeof(int), hipMemcpyHostToDevice, e->stream));
         enqueue_prefill_segment(e, slot, n, off + (uint32_t)n == n_tokens, e->stream);
         GDN_HIP(hipGetLastError());
@@ -2652,6 +2753,7 @@ void b_destroy(GDNBatchEngine *e) {
     (void)hipFree(e->p_logits);
     (void)hipFree(e->p_tok);
     (void)hipFree(e->seg_mem);
+    (void)hipFree(e->gu_mem);
     if (e->tok_host) (void)hipHostFree(e->tok_host);
     delete e;
 }
@@ -2954,7 +3056,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     for (uint32_t b = 0; b < blocks; ++b)
         gdn_tile_bf16(xb.data() + (size_t)b * kMaxB * K, kMaxB, K, 4, xt.data() + (size_t)b * kMaxB * K);
     const size_t out_elems = kind == 3 ? (size_t)tp * kI : (size_t)kSplitDown * tp * N;
-    void *dw = nullptr, *dx = nullptr, *dy = nullptr, *dr = nullptr;
+    void *dw = nullptr, *dx = nullptr, *dy = nullptr, *dr = nullptr, *dp = nullptr;
     GDN_HIP(hipMalloc(&dw, wt.size() * 2));
     GDN_HIP(hipMalloc(&dx, xt.size() * 2));
     GDN_HIP(hipMalloc(&dy, out_elems * 4));
@@ -2963,6 +3065,10 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     GDN_HIP(hipMemcpy(dw, wt.data(), wt.size() * 2, hipMemcpyHostToDevice));
     GDN_HIP(hipMemcpy(dx, xt.data(), xt.size() * 2, hipMemcpyHostToDevice));
     const u32x4 *w4 = static_cast<const u32x4 *>(dw), *x4 = static_cast<const u32x4 *>(dx);
+    if (kind == 3) {
+        GDN_HIP(hipMalloc(&dp, wt.size() * 2));
+        hipLaunchKernelGGL(k_gu_pairs, dim3(kI / 16, kKtH), dim3(128), 0, 0, w4, static_cast<u32x4 *>(dp));
+    }
     // one route into out (floats of a zeroed buffer's planes added in order,
     // or the X tiles' halves)
     const int rows = (int)N, toks = (int)T, pad = (int)tp;
@@ -2973,7 +3079,8 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
         if (kind == 0) planes = launch_p_gemm<kKtH, 8, 1>(route, w4, x4, y, rows, toks, pad, nullptr);
         if (kind == 1) planes = launch_p_gemm<kKtH, 4, kSplitO>(route, w4, x4, y, rows, toks, pad, nullptr);
         if (kind == 2) planes = launch_p_gemm<kKtI, 4, kSplitDown>(route, w4, x4, y, rows, toks, pad, nullptr);
-        if (kind == 3) launch_p_gu(route, w4, x4, static_cast<uint16_t *>(dy), toks, nullptr);
+        if (kind == 3)
+            launch_p_gu(route, w4, static_cast<const u32x4 *>(dp), x4, static_cast<uint16_t *>(dy), toks, nullptr);
         GDN_HIP(hipGetLastError());
         GDN_HIP(hipDeviceSynchronize());
         if (kind == 3) {
@@ -2995,6 +3102,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     // segment of some length runs on has to agree with it bit for bit
     std::vector<PRoute> routes = {kind % 2 == 0 && N % kPaRows == 0 ? P_WIDE : P_TILE, P_STEP, P_TILE};
     if (kind == 1 || kind == 2) routes.push_back(P_PLANES);
+    if (kind == 3) routes.push_back(P_WIDE);
     std::vector<float> first, other;
     std::vector<uint16_t> first16, other16;
     if (run_route(routes[0], first, first16)) return -1;
@@ -3060,6 +3168,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     (void)hipFree(dx);
     (void)hipFree(dy);
     (void)hipFree(dr);
+    (void)hipFree(dp);
     return 0;
 }
 

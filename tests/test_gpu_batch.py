@@ -118,7 +118,7 @@ def test_prefill_gemm_routes_agree(kind, N, T):
     assert same_bits(y, y_step)
 
 
-@pytest.mark.parametrize("n", [192, 193, 256, 257, 1536, 1537, 3073])
+@pytest.mark.parametrize("n", [192, 193, 256, 257, 385, 641, 1025, 1536, 1537, 3073])
 def test_prefill_route_edges_equal_steps(n):
     """Prompts on both sides of each projection's change of kernel: a layer's
     state and the next token equal single-stream steps bit for bit."""
