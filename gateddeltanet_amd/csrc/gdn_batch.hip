@@ -1786,12 +1786,16 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
 // tiles unrolled, the next kPaD tiles' operands in flight across trips):
 // a loop of fixed shape, whose waits on memory the compiler keeps exact,
 // where a loop of kPgD tiles with a data-dependent class close waited for
-// every load in flight at its top.  Same fragments, chains, class order and
-// split order as k_pgemm, so the same sums bit for bit.  Traced in the
-// 4096-token prefill: q/k/v/g 169.5 -> 150.0 us, down 138.9 -> 127.9 us.
-// o_proj (16 k tiles per split) stays on k_pgemm, as it measured no faster
-// in isolation; so does any launch whose grid would not fill the CUs
-// (pa_fills), where k_pgemm's twice as many workgroups do better.
+// every load in flight at its top.  A class starts from a zero operand of its
+// first MFMAs, the first class of a split in the split's sum itself: 64 adds
+// per further class are all that its close costs (with cleared chains and a
+// select of the first class, 4096 tokens' q/k/v/g took 145 us, now 131 (1.05
+// PFLOP/s); gate/up 228, now 221).  Same fragments, chains, class order and
+// split order as k_pgemm, so the same sums bit for bit.  k_pgemm takes 170 us
+// for q/k/v/g and 139 against 123 for down.  o_proj (16 k tiles per split)
+// stays on k_pgemm, as it measured no faster (78 us either way); so does any
+// launch whose grid would not fill the CUs (pa_fills), where k_pgemm's twice
+// as many workgroups do better.
 constexpr int kPaRows = 32 * kPgW;  // rows per workgroup
 constexpr int kPaD = 2;       // k tiles of operands in flight
 template <int KT, int NW, int S, bool SWIGLU>
@@ -1820,11 +1824,7 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
         bp[i] = X + (size_t)(2 * tt + (q >> 8)) * KT * 256 + (q & 255);
     }
     f32x4 chain[NB], part[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        chain[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        part[b] = chain[b];
-    }
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     u32x4 ra[kPaD][R], rb[kPaD][PB];
 #pragma unroll
     for (int d = 0; d < kPaD; ++d) {
@@ -1841,7 +1841,8 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
     auto out = [&](int f, int g) {
         return reinterpret_cast<f32x4 *>(y + (size_t)(m + 16 * g) * n_rows + row + 16 * f);
     };
-    for (int c = 0; c < KT / KTW; ++c) {
+    // the k tiles of class c, chained in acc from zero
+    auto run_class = [&](int c, f32x4(&acc)[NB]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < KTW; ++i) {
             const int j = c * KTW + i, sb = j & 1;
@@ -1874,24 +1875,28 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
             for (int g = 0; g < T; ++g)
 #pragma unroll
                 for (int f = 0; f < R; ++f)
-                    chain[T * f + g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, fa[f]), __builtin_bit_cast(bf16x8, fb[g]), chain[T * f + g], 0, 0,
-                        0);
+                    acc[T * f + g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, fa[f]), __builtin_bit_cast(bf16x8, fb[g]),
+                        i == 0 ? zero : acc[T * f + g], 0, 0, 0);
         }
-        // class c % NW of split c / NW closes: its chain joins the split's
-        // sum, and the last class's sum joins the total in split order
-        const int cls = c % NW;
+    };
+    // a split's first class chains in part itself, the others in chain and
+    // join it; the split's sum joins the total in split order
+#pragma unroll 1
+    for (int s = 0; s < S; ++s) {
+        run_class(s * NW, part);
+#pragma unroll 1
+        for (int c = 1; c < NW; ++c) {
+            run_class(s * NW + c, chain);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            part[b] = cls == 0 ? chain[b] : part[b] + chain[b];
-            chain[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            for (int b = 0; b < NB; ++b) part[b] = part[b] + chain[b];
         }
-        if (!SWIGLU && cls == NW - 1) {
-            const bool first = c < NW;
+        if (!SWIGLU) {
 #pragma unroll
             for (int f = 0; f < R; ++f)
 #pragma unroll
-                for (int g = 0; g < T; ++g) *out(f, g) = first ? part[T * f + g] : *out(f, g) + part[T * f + g];
+                for (int g = 0; g < T; ++g)
+                    *out(f, g) = s == 0 ? part[T * f + g] : *out(f, g) + part[T * f + g];
         }
     }
     if constexpr (SWIGLU) {
