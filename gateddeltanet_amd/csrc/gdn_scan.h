@@ -50,7 +50,7 @@ __device__ __forceinline__ void scan_delta_o(float acc, float beta, float decay,
 // What bounds it: a wave64 FP32 add occupies its SIMD for 4 cycles, so the
 // 256 adds a bit-equal chain needs are 1024 of the token's cycles whatever
 // the layout; 8 heads x 256 columns x 2 chains fill the 1024 SIMDs exactly
-// once at four chains per wave.  A 4096-token launch takes 3.14 ms (0.77 us a
+// once at four chains per wave.  A 4096-token launch takes 3.06 ms (0.75 us a
 // token); with every product written to LDS and four lanes of a wave reading
 // the chains' operands back it took 4.44 ms (1.08 us).
 //
@@ -132,6 +132,10 @@ __device__ __forceinline__ void scan_block(const ScanArgs a, const Scal scal, vo
         else sv[i] = static_cast<const float *>(state)[at];
     }
     store_chunk(0);
+    // the state waited for here: a wait inside the token loop would also wait
+    // for the next chunk's loads, at each chunk's first token
+#pragma unroll
+    for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(sv[i]));
     __syncthreads();
 
     f32x4 mul[4], kn[4];  // the next token's k or q; the current token's k
@@ -151,11 +155,13 @@ __device__ __forceinline__ void scan_block(const ScanArgs a, const Scal scal, vo
             for (int i = 0; i < 16; ++i) p[i] = sv[i] * mul[i >> 2][i & 3];
             // read under the chain: what the rest of this token needs, and
             // the next token's factors
+            const float v = lds.v[b][m][lc];
 #pragma unroll
             for (int i = 0; i < 4; ++i) kn[i] = lds.kq[b][m][0][16 * i + i16];
             const f32x4 scl = lds.sc[b][m];
-            const float v = lds.v[b][m][lc], beta = scl.x, decay = scl.y, alpha = scl.z;
+            const float beta = scl.x, decay = scl.y, alpha = scl.z;
             read_mul(b, m + 1 < n ? m + 1 : m);
+            __builtin_amdgcn_sched_barrier(0);
             const float acc = chain256(p);  // lane 15 of the row
             float delta, o;
             scan_delta_o(acc, beta, decay, alpha, v, delta, o);
@@ -190,6 +196,10 @@ __device__ __forceinline__ void scan_block(const ScanArgs a, const Scal scal, vo
 #pragma unroll
                 for (int i = 0; i < 16; ++i) sv[i] = nv[i];
             }
+            // used here, so that the reads stay ahead of the chain instead of
+            // moving to the next token's products
+#pragma unroll
+            for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(mul[i]));
         }
         if (kind == 1 && i16 < n) a.o[(size_t)(kScanTok * c + i16) * a.ldo + lc] = R<C>(oacc);
         if (c + 1 < chunks) {
