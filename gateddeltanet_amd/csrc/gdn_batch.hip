@@ -2513,10 +2513,17 @@ int seg_alloc(GDNBatchEngine *e) {
 
 // k_pgu_a's layout of every layer's gate/up weights (46 MB a layer beside the
 // step's), formed on the device for the first segment that takes it and kept.
+// Without the memory for it gu_mem stays NULL and the segment takes k_pgu.
 int gu_pairs(GDNBatchEngine *e) {
     if (e->gu_mem) return 0;
     const size_t per = (size_t)2 * kI * kH * 2;
-    GDN_HIP(hipMalloc(&e->gu_mem, (size_t)e->layers * per));
+    const hipError_t rc = hipMalloc(&e->gu_mem, (size_t)e->layers * per);
+    if (rc != hipSuccess) e->gu_mem = nullptr;
+    if (rc == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    GDN_HIP(rc);
     for (int l = 0; l < e->layers; ++l) {
         u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(e->gu_mem) + (size_t)l * per);
         hipLaunchKernelGGL(k_gu_pairs, dim3(kI / 16, kKtH), dim3(128), 0, e->stream, e->w_gu[l], dst);
@@ -2660,6 +2667,7 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
     launch_ab(0);
     const u32x4 *xh = reinterpret_cast<const u32x4 *>(e->s_xh), *xo = reinterpret_cast<const u32x4 *>(e->s_xo),
                 *xd = reinterpret_cast<const u32x4 *>(e->s_xd);
+    const PRoute gu = route_gu(n) == P_WIDE && !e->gu_mem ? P_TILE : route_gu(n);
     for (int l = 0; l < e->layers; ++l) {
         float *st = b_state(e, l) + (size_t)slot * kLayerState;
         uint16_t *tl = b_tails(e, l) + (size_t)slot * kStreamTails;
@@ -2680,7 +2688,7 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
                            e->s_gate, e->s_sgate, b_aux(e, l) + kAuxONorm, e->eps, e->s_xo, n);
         const int po = launch_p_gemm<kKtH, 4, kSplitO>(route_o(n), e->w_o[l], xo, e->s_y, kH, n, e->seg_cap, s);
         launch_p_norm(seg_norm(e, e->s_y, b_aux(e, l) + kAuxMlpNorm, e->s_xh, -1, l, l), po, n, s);
-        launch_p_gu(route_gu(n), e->w_gu[l], e->w_gup[l], xh, e->s_xd, n, s);
+        launch_p_gu(gu, e->w_gu[l], e->w_gup[l], xh, e->s_xd, n, s);
         const int pd =
             launch_p_gemm<kKtI, 4, kSplitDown>(route_down(kH, n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
         if (l + 1 < e->layers) {
