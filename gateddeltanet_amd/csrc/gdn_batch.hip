@@ -1677,13 +1677,10 @@ __device__ __forceinline__ bool pg_close(int j, f32x4 (&chain)[NB], f32x4 (&part
 }
 
 // y[m][row] for rows 128 rt .. +127 and tokens 128 tt .. +127 (pg_place):
-// the sum k_bgemm<2, KT, NW, S, EPI_RAW> forms for the row (S = 1), or the
-// in-order sum of its S split partials.  With splits the running total
-// lives in the output tile itself (each lane rewrites only its own
-// elements, after its own earlier store), so a wave holds only two
-// accumulator sets (the class chain and the split's sum).  W in the 32-row
-// block layout ([row block][k tile][2 tiles][64 lanes]); X in 64-token X
-// tile blocks; y has the padded token count's rows.
+// the sum k_bgemm<2, KT, NW, S, EPI_RAW> forms for the row (S = 1), or one of
+// its S split partials.  W in the 32-row block layout ([row block][k tile][2
+// tiles][64 lanes]); X in 64-token X tile blocks; y has the padded token
+// count's rows.
 // Waves per workgroup: 8 of 64 rows x 32 tokens (about 100 VGPRs, four
 // waves per SIMD) measured 98.4k against 95.9k prefill tokens/s for 4 of
 // 64 x 64 (two per SIMD), with twice the LDS fragment reads.
@@ -1694,13 +1691,14 @@ constexpr int kPgW = GDN_PG_WAVES;
 
 // PLANES: grid z is the split; a workgroup forms one split's sum and writes
 // it to that split's plane of y (y_rows tokens), which the consumer adds in
-// split order, as it adds the step's.  Four times the workgroups of the
-// running total, for segments whose tiles leave CUs idle.
+// split order, as it adds the step's: S times the workgroups of a kernel that
+// adds the splits itself, for segments whose tiles leave CUs idle.
 template <int KT, int NW, int S, bool PLANES>
 __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                      float *__restrict__ y, int n_rows, int y_rows) {
     constexpr int NT = PLANES ? KT / S : KT;  // k tiles of this workgroup
     static_assert(NT % kPgD == 0, "whole groups of kPgD k tiles");
+    static_assert(S == 1 || PLANES, "one split's sum per workgroup");
     const int jb = PLANES ? (int)blockIdx.z * NT : 0;
     if constexpr (PLANES) y += (size_t)blockIdx.z * y_rows * n_rows;
     constexpr int GT = kPgW * 64, AU = 4 * 2 * 64, BU = 2 * 4 * 64, PT = (AU + BU) / GT;
@@ -1768,11 +1766,8 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
                         __builtin_bit_cast(bf16x8, fa[f]), __builtin_bit_cast(bf16x8, fb[g]), chain[TG * f + g], 0,
                         0, 0);
             if (pg_close<KT, NW, S, NB>(j, chain, part)) {
-                // the split's sum joins the total in split order
-                // (one split per workgroup with PLANES)
-                const bool first = PLANES || j < KT / S;
 #pragma unroll
-                for (int b = 0; b < NB; ++b) *out(b) = first ? part[b] : *out(b) + part[b];
+                for (int b = 0; b < NB; ++b) *out(b) = part[b];
             }
         }
     }
@@ -1788,34 +1783,44 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
 // where a loop of kPgD tiles with a data-dependent class close waited for
 // every load in flight at its top.  A class starts from a zero operand of its
 // first MFMAs, the first class of a split in the split's sum itself: 64 adds
-// per further class are all that its close costs (with cleared chains and a
-// select of the first class, 4096 tokens' q/k/v/g took 145 us, now 131 (1.05
-// PFLOP/s); gate/up 228, now 221).  Same fragments, chains, class order and
-// split order as k_pgemm, so the same sums bit for bit.  k_pgemm takes 170 us
-// for q/k/v/g and 139 against 123 for down.  o_proj (16 k tiles per split)
-// stays on k_pgemm, as it measured no faster (78 us either way); so does any
-// launch whose grid would not fill the CUs (pa_fills), where k_pgemm's twice
-// as many workgroups do better.
-constexpr int kPaRows = 32 * kPgW;  // rows per workgroup
-constexpr int kPaD = 2;       // k tiles of operands in flight
-template <int KT, int NW, int S, bool SWIGLU>
+// per further class are all that its close costs (145 -> 131 us for 4096
+// tokens' q/k/v/g against cleared chains and a select of the first class).
+// A tile's fragments are read from LDS under the second half of the tile
+// before it, the barrier in the middle of that tile's products: at 4096
+// tokens gate/up 239 -> 223 us, o_proj 42 -> 41, q/k/v/g 140 and down 90 as
+// they were (4 waves of 64 rows, half the LDS reads at one wave per SIMD: 279,
+// 56, 160, 111).  The total over the splits stays in LDS, each thread's own
+// elements: through the output tile, as k_pgemm's splits once had it, o_proj
+// at 4096 tokens took 84 us (now 41, 0.84 PFLOP/s) and down 123 (now 90, 1.05).
+// What bounds it: the LDS reads of the tokens' fragments (64 KB per k tile and
+// CU), as long as the products themselves, and one barrier per k tile.
+// Same fragments, chains, class order and split order as the step's kernels,
+// so the same sums bit for bit.  PLANES: as k_pgemm's.
+constexpr int kPaW = 8;             // waves per workgroup
+constexpr int kPaRows = 32 * kPaW;  // rows per workgroup
+constexpr int kPaD = 2;             // k tiles of operands in flight
+template <int KT, int NW, int S, bool SWIGLU, bool PLANES>
 __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                               float *__restrict__ y, uint16_t *__restrict__ x_next, int n_rows,
                                               int n_tok) {
-    constexpr int R = kPaRows / 16 / kPgW;  // 16-row tiles per wave
+    constexpr bool TOTAL = S > 1 && !PLANES;  // the splits are added here
+    constexpr int R = kPaRows / 16 / kPaW;  // 16-row tiles per wave
     constexpr int T = kPgTok / 16;          // 16-token groups per wave
-    constexpr int GT = kPgW * 64, BU = T * 64, PB = BU / GT;
+    constexpr int GT = kPaW * 64, BU = T * 64, PB = BU / GT;
     constexpr int NB = R * T, KTS = KT / S, KTW = KTS / NW;
     static_assert(R == 2 && BU % GT == 0 && KT % S == 0 && KTS % NW == 0, "row and token tiles per workgroup");
     __shared__ u32x4 stg[2][BU];
+    __shared__ f32x4 tot[TOTAL ? NB : 1][TOTAL ? GT : 1];  // each thread's own sums
     __shared__ uint64_t exp2_lds[SWIGLU ? 32 : 1];  // expf's table for the SwiGLU epilogue
+    // the first k tile in class order, and the one past the last
+    const int jb = PLANES ? (int)blockIdx.z * KTS : 0, je = PLANES ? jb + KTS : KT;
     if constexpr (SWIGLU) fill_exp2_lds_imm(exp2_lds);
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
     int rt, tt;
     pg_place(rt, tt);
-    // wave w's rows: 32-row block kPgW rt + w of the weight layout (its two
+    // wave w's rows: 32-row block kPaW rt + w of the weight layout (its two
     // tiles at entries 0..63 and 64..127 of each k tile)
-    const u32x4 *ap = W + (size_t)(kPgW * rt + w) * KT * 128 + l;
+    const u32x4 *ap = W + (size_t)(kPaW * rt + w) * KT * 128 + l;
     // B entry q of a k tile: token group q / 64 (of 8), lane q % 64
     const u32x4 *bp[PB];
 #pragma unroll
@@ -1825,14 +1830,31 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
     }
     f32x4 chain[NB], part[NB];
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    u32x4 ra[kPaD][R], rb[kPaD][PB];
+    // ra[d]: the weights of tile j + d; rb[d]: the tokens of tile j + 1 + d
+    u32x4 ra[kPaD + 1][R], rb[kPaD][PB], fb[T];
+    auto load_a = [&](u32x4(&r)[R], int j) __attribute__((always_inline)) {
+        const int kt = pg_tile<KT, NW, S>(j < je ? j : je - 1);
 #pragma unroll
-    for (int d = 0; d < kPaD; ++d) {
-        const int kt = pg_tile<KT, NW, S>(d);
+        for (int f = 0; f < R; ++f) r[f] = ap[(size_t)kt * 128 + 64 * f];
+    };
+    auto load_b = [&](u32x4(&r)[PB], int j) __attribute__((always_inline)) {
+        const int kt = pg_tile<KT, NW, S>(j < je ? j : je - 1);
 #pragma unroll
-        for (int f = 0; f < R; ++f) ra[d][f] = ap[(size_t)kt * 128 + 64 * f];
+        for (int i = 0; i < PB; ++i) r[i] = bp[i][(size_t)kt * 256];
+    };
+    {
+        u32x4 r0[PB];
+        load_b(r0, jb);
 #pragma unroll
-        for (int i = 0; i < PB; ++i) rb[d][i] = bp[i][(size_t)kt * 256];
+        for (int d = 0; d < kPaD; ++d) {
+            load_a(ra[d], jb + d);
+            load_b(rb[d], jb + 1 + d);
+        }
+#pragma unroll
+        for (int q = 0; q < PB; ++q) stg[jb & 1][t + GT * q] = r0[q];
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < T; ++g) fb[g] = stg[jb & 1][64 * g + l];
     }
     // row tile f: rows kPaRows rt + 32 w + 16 f + 4 (l / 16) .. +3; token group
     // g: token 128 tt + 16 g + l % 16
@@ -1845,45 +1867,48 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
     auto run_class = [&](int c, f32x4(&acc)[NB]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < KTW; ++i) {
-            const int j = c * KTW + i, sb = j & 1;
-            u32x4 fa[R];
-#pragma unroll
-            for (int f = 0; f < R; ++f) fa[f] = ra[0][f];
+            const int j = c * KTW + i, sb = (j + 1) & 1;
+            u32x4 fn[T];
+            // issued on every tile (the last ones re-read the final tile,
+            // unused), so the loop's shape stays fixed
+            load_a(ra[kPaD], j + kPaD);
+            // the buffer's fragments of tile j - 1 were read before the
+            // barrier of tile j - 1
 #pragma unroll
             for (int q = 0; q < PB; ++q) stg[sb][t + GT * q] = rb[0][q];
 #pragma unroll
-            for (int d = 0; d + 1 < kPaD; ++d) {
-#pragma unroll
-                for (int f = 0; f < R; ++f) ra[d][f] = ra[d + 1][f];
+            for (int d = 0; d + 1 < kPaD; ++d)
 #pragma unroll
                 for (int q = 0; q < PB; ++q) rb[d][q] = rb[d + 1][q];
-            }
-            {
-                // issued on every tile (the last ones re-read the final tile,
-                // unused), so the loop's shape stays fixed
-                const int kt = pg_tile<KT, NW, S>(j + kPaD < KT ? j + kPaD : KT - 1);
-#pragma unroll
-                for (int f = 0; f < R; ++f) ra[kPaD - 1][f] = ap[(size_t)kt * 128 + 64 * f];
-#pragma unroll
-                for (int q = 0; q < PB; ++q) rb[kPaD - 1][q] = bp[q][(size_t)kt * 256];
-            }
-            __syncthreads();
-            u32x4 fb[T];
-#pragma unroll
-            for (int g = 0; g < T; ++g) fb[g] = stg[sb][64 * g + l];
-#pragma unroll
-            for (int g = 0; g < T; ++g)
+            load_b(rb[kPaD - 1], j + 1 + kPaD);
+            auto mm = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
                 for (int f = 0; f < R; ++f)
                     acc[T * f + g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, fa[f]), __builtin_bit_cast(bf16x8, fb[g]),
+                        __builtin_bit_cast(bf16x8, ra[0][f]), __builtin_bit_cast(bf16x8, fb[g]),
                         i == 0 ? zero : acc[T * f + g], 0, 0, 0);
+            };
+#pragma unroll
+            for (int g = 0; g < T / 2; ++g) mm(g);
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+#pragma unroll
+            for (int g = 0; g < T; ++g) fn[g] = stg[sb][64 * g + l];
+#pragma unroll
+            for (int g = T / 2; g < T; ++g) mm(g);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < T; ++g) fb[g] = fn[g];
+#pragma unroll
+            for (int d = 0; d < kPaD; ++d)
+#pragma unroll
+                for (int f = 0; f < R; ++f) ra[d][f] = ra[d + 1][f];
         }
     };
     // a split's first class chains in part itself, the others in chain and
     // join it; the split's sum joins the total in split order
 #pragma unroll 1
-    for (int s = 0; s < S; ++s) {
+    for (int s = PLANES ? (int)blockIdx.z : 0, se = PLANES ? s + 1 : S; s < se; ++s) {
         run_class(s * NW, part);
 #pragma unroll 1
         for (int c = 1; c < NW; ++c) {
@@ -1891,19 +1916,24 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
 #pragma unroll
             for (int b = 0; b < NB; ++b) part[b] = part[b] + chain[b];
         }
-        if (!SWIGLU) {
+        if constexpr (TOTAL) {
 #pragma unroll
-            for (int f = 0; f < R; ++f)
-#pragma unroll
-                for (int g = 0; g < T; ++g)
-                    *out(f, g) = s == 0 ? part[T * f + g] : *out(f, g) + part[T * f + g];
+            for (int b = 0; b < NB; ++b) {
+                if (s) part[b] = tot[b][t] + part[b];
+                if (s + 1 < S) tot[b][t] = part[b];
+            }
         }
     }
-    if constexpr (SWIGLU) {
+    if constexpr (!SWIGLU) {
+#pragma unroll
+        for (int f = 0; f < R; ++f)
+#pragma unroll
+            for (int g = 0; g < T; ++g) *out(f, g) = part[T * f + g];
+    } else {
         // row tile 0: the gate rows of the wave's 16 channels, tile 1 their
         // up rows, so a lane holds both of channels 4 (l / 16) .. + 3
         // (gemv32_store SwiGLU branch, gdn_model.cpp:4751-4767)
-        const int ch = 16 * (kPgW * rt + w) + 4 * (l >> 4);
+        const int ch = 16 * (kPaW * rt + w) + 4 * (l >> 4);
         // one token group per trip, the next ones moved down (unrolled, the
         // eight groups' SiLUs are 50 KB of code)
 #pragma unroll 1
@@ -1924,10 +1954,11 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
         }
     }
 }
-template <int KT, int NW, int S>
-__global__ __launch_bounds__(kPgW * 64) void k_pgemm_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
-                                                       float *__restrict__ y, int n_rows) {
-    pgemm_a_block<KT, NW, S, false>(W, X, y, nullptr, n_rows, 0);
+template <int KT, int NW, int S, bool PLANES>
+__global__ __launch_bounds__(kPaW * 64) void k_pgemm_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
+                                                       float *__restrict__ y, int n_rows, int y_rows) {
+    if constexpr (PLANES) y += (size_t)blockIdx.z * y_rows * n_rows;
+    pgemm_a_block<KT, NW, S, false, PLANES>(W, X, y, nullptr, n_rows, 0);
 }
 
 // Gate/up + SwiGLU on the same kernel: W in 32-row blocks of 16 channels'
@@ -1935,9 +1966,9 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm_a(const u32x4 *__restrict__
 // are the step's; the first n_tok tokens are written.  All rows carry
 // weights, where the 44-row groups of k_pgu leave 4 of 48 empty, and a wave
 // reads 8 fragments from LDS per 16 MFMAs where k_pgu's reads 5 per 6.
-__global__ __launch_bounds__(kPgW * 64) void k_pgu_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
+__global__ __launch_bounds__(kPaW * 64) void k_pgu_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                      uint16_t *__restrict__ x_next, int n_tok) {
-    pgemm_a_block<kKtH, kGuWaves, 1, true>(W, X, nullptr, x_next, 2 * kI, n_tok);
+    pgemm_a_block<kKtH, kGuWaves, 1, true, false>(W, X, nullptr, x_next, 2 * kI, n_tok);
 }
 
 // One layer's gate/up weights from the step's 44-row groups (tile_gu) into
@@ -2566,36 +2597,47 @@ BNorm seg_norm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_ou
 // to whole 128-token tiles), on the kernel that is fastest at that size; every
 // choice forms the same sums.
 enum PRoute {
-    P_STEP,    // the decode step's kernels, a grid plane per 64-token block
-    P_PLANES,  // k_pgemm with a workgroup per split (o_proj, down)
-    P_TILE,    // k_pgemm / k_pgu, 128 tokens per workgroup
-    P_WIDE     // k_pgemm_a, once its grid (half of k_pgemm's) fills the CUs; k_pgu_a
+    P_STEP,        // the decode step's kernels, a grid plane per 64-token block
+    P_TILE,        // k_pgemm / k_pgu, 128 tokens per workgroup (q/k/v/g, gate/up)
+    P_PLANES,      // k_pgemm with a workgroup per split (o_proj, down)
+    P_WIDE,        // k_pgemm_a / k_pgu_a, 256 rows x 128 tokens per workgroup
+    P_WIDE_PLANES  // k_pgemm_a with a workgroup per split (down)
 };
-// Where the lines lie (us per launch, step / planes / tile at 64, 256, 512,
-// 1024, 2048 tokens):
-//   q/k/v/g  12 / - / 30   28 / - / 30    49 / - / 32    91 / - / 42   174 / - / 79
-//   o_proj    5 / 11 / 34    9 / 11 / 33   15 / 12 / 34   26 / 19 / 36   49 / 38 / 44
-//   down      9 / 20 / 71   18 / 20 / 69   30 / 22 / 70   54 / 37 / 75  103 / 69 / 85
-//   gate/up  15 / - / 30   33 / - / 31    57 / - / 45   107 / - / 83   207 / - / 151
-// The step's kernels re-read the weights per 64 tokens; the tile kernels leave
-// most CUs idle on short segments (16 workgroups for o_proj and down at up to
-// 128 tokens).  Planes cost the norm after them three more reads (12 against
-// 9 us at 1024 tokens, 46 against 32 at 4096), which moves their upper line
-// down: at 4096 tokens o_proj, down and their norms take 114 + 177 against
-// 114 + 161 us.
-bool pa_fills(int rows, int n) { return rows % kPaRows == 0 && (rows / kPaRows) * ((n + kPgTok - 1) / kPgTok) >= 256; }
+// Where the lines lie, us per launch (the step's kernels re-read the weights
+// per 64 tokens; the others leave CUs idle on short segments):
+//   tokens                   64  256  512  768 1024 1536 2048 2560 3072 4096
+//   q/k/v/g  step            12   28   49    -   91    -  174    -    -    -
+//            tile            30   30   32   42   42    -   79    -    -    -
+//            wide             -    -    -    -   39   62   75   96  106  140
+//   o_proj   step             5    9   15    -   26    -   49    -    -    -
+//            planes          11   11   13   18   20   29   38   46   54   69
+//            wide             -    -   33   33   34   35   37   38   39   41
+//   down     step             9   18   30    -   54    -  103    -    -    -
+//            planes          20   20   23   34   38   55   71   87  102  135
+//            wide planes      -    -   26   26   33   54   58   77   82  113
+//            wide             -    -   78   77   80   80   84   85   85   90
+//   gate/up  step            15   33   57    -  107    -  207    -    -    -
+//            tile            30   31   45   63   81  120  151    -    -  280
+//            wide             -    -   42    -    -    -  114  151  183  223
+// and the norm that reads four planes in place of one sum costs more: 8.3
+// against 6.8 at 512 tokens, 12.6 / 9.7 at 1024, 19 / 13 at 1536, 25 / 18 at
+// 2048, 30 / 21 at 2560, 37 / 24 at 3072.
+int p_tiles(int n) { return (n + kPgTok - 1) / kPgTok; }
+bool pa_fills(int rows, int n) { return rows % kPaRows == 0 && (rows / kPaRows) * p_tiles(n) >= 256; }
 PRoute route_qkvg(int rows, int n) { return n <= 256 ? P_STEP : pa_fills(rows, n) ? P_WIDE : P_TILE; }
-PRoute route_o(int n) { return n <= 256 ? P_STEP : n <= 1536 ? P_PLANES : P_TILE; }
-PRoute route_down(int rows, int n) {
-    return n <= 256 ? P_STEP : n <= 3072 ? P_PLANES : pa_fills(rows, n) ? P_WIDE : P_TILE;
+PRoute route_o(int n) { return n <= 256 ? P_STEP : n <= 1536 ? P_PLANES : P_WIDE; }
+// down's wide planes take whole rounds of 256 workgroups (eight tiles, about
+// 26 us), its planes about 4.4 us a tile and 4.
+PRoute route_down(int n) {
+    if (n <= 256) return P_STEP;
+    if (n > 2560) return P_WIDE;
+    return 65 * ((p_tiles(n) + 7) / 8) <= 11 * p_tiles(n) + 10 ? P_WIDE_PLANES : P_PLANES;
 }
 // k_pgu_a takes whole rounds of 256 workgroups (one per CU, 44 per 128 tokens),
-// about 39 us each; k_pgu (two per CU) about 8.5 us per 128 tokens and 14.
-// tile / wide: 512 tokens 46 / 44 us, 768 66 / 77, 1536 117 / 114, 2048 151 /
-// 119, 4096 280 / 226.
+// about 38 us each; k_pgu (two per CU) about 8.5 us per 128 tokens and 14.
 bool pgu_a_pays(int n) {
-    const int tiles = (n + kPgTok - 1) / kPgTok, rounds = (2 * kI / kPaRows * tiles + 255) / 256;
-    return 78 * rounds <= 17 * tiles + 18;
+    const int rounds = (2 * kI / kPaRows * p_tiles(n) + 255) / 256;
+    return 76 * rounds <= 17 * p_tiles(n) + 22;
 }
 PRoute route_gu(int n) { return n <= 192 ? P_STEP : pgu_a_pays(n) ? P_WIDE : P_TILE; }
 
@@ -2605,7 +2647,7 @@ PRoute route_gu(int n) { return n <= 192 ? P_STEP : pgu_a_pays(n) ? P_WIDE : P_T
 template <int KT, int NW, int S>
 int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int rows, int n, int y_rows,
                   hipStream_t s) {
-    const int blocks = (n + kMaxB - 1) / kMaxB, tiles = (n + kPgTok - 1) / kPgTok;
+    const int blocks = (n + kMaxB - 1) / kMaxB, tiles = p_tiles(n);
     if (route == P_STEP) {
         BEpi ep{};
         ep.n_streams = kMaxB;
@@ -2615,17 +2657,24 @@ int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int ro
         launch_bgemm<2, KT, NW, S, EPI_RAW>(n, dim3(rows / 32, S, blocks), w, x, ep, s);
         return S;
     }
-    if (route == P_PLANES) {
-        hipLaunchKernelGGL((k_pgemm<KT, NW, S, true>), dim3(rows / 128, tiles, S), dim3(kPgW * 64), 0, s, w, x, y,
-                           rows, y_rows);
-        return S;
+    if (route == P_WIDE) {
+        hipLaunchKernelGGL((k_pgemm_a<KT, NW, S, false>), dim3(rows / kPaRows, tiles), dim3(kPaW * 64), 0, s, w, x, y,
+                           rows, 0);
+        return 1;
     }
-    if (route == P_WIDE)
-        hipLaunchKernelGGL((k_pgemm_a<KT, NW, S>), dim3(rows / kPaRows, tiles), dim3(kPgW * 64), 0, s, w, x, y, rows);
-    else
-        hipLaunchKernelGGL((k_pgemm<KT, NW, S, false>), dim3(rows / 128, tiles), dim3(kPgW * 64), 0, s, w, x, y, rows,
+    if constexpr (S > 1) {
+        if (route == P_WIDE_PLANES)
+            hipLaunchKernelGGL((k_pgemm_a<KT, NW, S, true>), dim3(rows / kPaRows, tiles, S), dim3(kPaW * 64), 0, s, w,
+                               x, y, rows, y_rows);
+        else
+            hipLaunchKernelGGL((k_pgemm<KT, NW, S, true>), dim3(rows / 128, tiles, S), dim3(kPgW * 64), 0, s, w, x, y,
+                               rows, y_rows);
+        return S;
+    } else {
+        hipLaunchKernelGGL((k_pgemm<KT, NW, 1, false>), dim3(rows / 128, tiles), dim3(kPgW * 64), 0, s, w, x, y, rows,
                            0);
-    return 1;
+        return 1;
+    }
 }
 static_assert(kRtO == 2 && kRtDown == 2, "o_proj and down in 32-row blocks");
 
@@ -2636,7 +2685,7 @@ void launch_p_gu(PRoute route, const u32x4 *w, const u32x4 *wp, const u32x4 *x, 
     if (route == P_STEP)
         launch_bgu(n, (n + kMaxB - 1) / kMaxB, w, x, x_next, s);
     else if (route == P_WIDE)
-        hipLaunchKernelGGL(k_pgu_a, dim3(2 * kI / kPaRows, tiles), dim3(kPgW * 64), 0, s, wp, x, x_next, n);
+        hipLaunchKernelGGL(k_pgu_a, dim3(2 * kI / kPaRows, tiles), dim3(kPaW * 64), 0, s, wp, x, x_next, n);
     else
         hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, tiles), dim3(kPgW * 64), 0, s, w, x, x_next, n);
 }
@@ -2690,7 +2739,7 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
         launch_p_norm(seg_norm(e, e->s_y, b_aux(e, l) + kAuxMlpNorm, e->s_xh, -1, l, l), po, n, s);
         launch_p_gu(gu, e->w_gu[l], e->w_gup[l], xh, e->s_xd, n, s);
         const int pd =
-            launch_p_gemm<kKtI, 4, kSplitDown>(route_down(kH, n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
+            launch_p_gemm<kKtI, 4, kSplitDown>(route_down(n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
         if (l + 1 < e->layers) {
             BNorm pa = seg_norm(e, e->s_y, b_aux(e, l + 1) + kAuxAttnNorm, e->s_xh, -1, l, l + 1);
             pa.xn_out = e->s_xn;
@@ -3113,9 +3162,11 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     };
     // the 128-token kernels give the result; every other kernel that a
     // segment of some length runs on has to agree with it bit for bit
-    std::vector<PRoute> routes = {kind % 2 == 0 && N % kPaRows == 0 ? P_WIDE : P_TILE, P_STEP, P_TILE};
-    if (kind == 1 || kind == 2) routes.push_back(P_PLANES);
-    if (kind == 3) routes.push_back(P_WIDE);
+    std::vector<PRoute> routes = {P_STEP, kind == 1 || kind == 2 ? P_PLANES : P_TILE};
+    const bool wide = kind == 3 || N % kPaRows == 0;
+    if (wide) routes.insert(routes.begin(), P_WIDE);
+    else std::swap(routes[0], routes[1]);
+    if (wide && (kind == 1 || kind == 2)) routes.push_back(P_WIDE_PLANES);
     std::vector<float> first, other;
     std::vector<uint16_t> first16, other16;
     if (run_route(routes[0], first, first16)) return -1;

@@ -101,11 +101,13 @@ def test_prefill_gemm_equals_step_gemm(kind, N, T):
     assert same_bits(y, y_step)
 
 
-@pytest.mark.parametrize("kind,N,T", [(0, 256, 257), (0, 128, 1), (1, 128, 63), (1, 128, 257), (2, 256, 129),
-                                      (2, 128, 1), (3, 5632, 193), (3, 5632, 1)])
+@pytest.mark.parametrize("kind,N,T", [(0, 256, 257), (0, 128, 1), (1, 128, 63), (1, 128, 257), (1, 256, 129),
+                                      (1, 512, 1), (2, 256, 129), (2, 512, 257), (2, 128, 1), (3, 5632, 193),
+                                      (3, 5632, 1)])
 def test_prefill_gemm_routes_agree(kind, N, T):
     """Each kernel that a segment of some length takes for a projection (the
-    step's over token blocks, the split planes, the 128-token tiles) gives the
+    step's over token blocks, the split planes, the 128-token tiles, 256 rows a
+    workgroup with the splits added or in planes) gives the
     same bits, at a token past and short of their blocks: the call itself
     fails if two differ, and its result is the step's."""
     rng = np.random.default_rng(200 + 10 * kind + T)
@@ -118,7 +120,7 @@ def test_prefill_gemm_routes_agree(kind, N, T):
     assert same_bits(y, y_step)
 
 
-@pytest.mark.parametrize("n", [192, 193, 256, 257, 385, 641, 1025, 1536, 1537, 3073])
+@pytest.mark.parametrize("n", [192, 193, 256, 257, 385, 512, 513, 641, 1024, 1025, 1536, 1537, 2560, 2561, 3073])
 def test_prefill_route_edges_equal_steps(n):
     """Prompts on both sides of each projection's change of kernel: a layer's
     state and the next token equal single-stream steps bit for bit."""
