@@ -510,8 +510,8 @@ struct BNorm {
 // tiny a/b rows and beta/decay (gdn_gemv_tiny_ab :1501-1536, :2461-2465).
 // Thread t holds elements 8t..8t+7; a 16-element chunk is the sequential sum
 // of thread 2c's eight squares continued by thread 2c + 1.  SPLITS partial
-// sums of the preceding projection are added in split order (0: no residual
-// add; EMBED: the embedding row instead).  Without AB one workgroup per
+// sums of the preceding projection are added in split order (1: its rounded
+// sums as BF16 bits; 0: no residual add; EMBED: the embedding row instead).  Without AB one workgroup per
 // stream updates the residual in place.  With AB, grid (streams, kAbSplit):
 // workgroup j repeats the norm and runs the a/b rows of heads
 // kNH / kAbSplit * j .. (a 32 KB slice of the 128 KB of rows, requested
@@ -583,7 +583,17 @@ __global__ __launch_bounds__(kT) void k_bnorm(BNorm p) {
         const f32x4 a0 = h4[0], a1 = h4[1];
         hv[0] = a0.x; hv[1] = a0.y; hv[2] = a0.z; hv[3] = a0.w;
         hv[4] = a1.x; hv[5] = a1.y; hv[6] = a1.z; hv[7] = a1.w;
-        if constexpr (SPLITS > 0) {
+        if constexpr (SPLITS == 1) {
+            // the projection's sums, rounded by its kernel
+            const u32x4 y = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint16_t *>(p.y) +
+                                                             (size_t)m * kH + e0);
+            const uint32_t yw[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                hv[2 * i] = rne_bf16(hv[2 * i] + u2f(yw[i] << 16));
+                hv[2 * i + 1] = rne_bf16(hv[2 * i + 1] + u2f(yw[i] & 0xffff0000u));
+            }
+        } else if constexpr (SPLITS > 0) {
             // the projection's split sums in split order, then its rounding
             f32x4 yp[SPLITS][2];
 #pragma unroll
@@ -787,9 +797,12 @@ __global__ __launch_bounds__(kT) void k_pab(const float *__restrict__ xn, int n,
 // (gdn_output_norm_and_gate, gdn_model.cpp:3226-3349) into X tiles, for
 // streams (or prefill tokens) PT y .. PT y + PT - 1 of n: every input of
 // the workgroup's PT streams is requested at its start (a stream past n
-// re-reads stream n - 1, unused), so they share one memory latency.
-template <int PT>
-__global__ __launch_bounds__(kT) void k_bonorm(const float *__restrict__ attn, const float *__restrict__ gate,
+// re-reads stream n - 1, unused), so they share one memory latency.  RAW: gate
+// is the g section of the projection's rounded sums ([token][4 kH] BF16 bits)
+// and the sigmoid is formed here: 4 bytes less to read a value, and 8 less
+// for the conv kernel to write.
+template <int PT, bool RAW>
+__global__ __launch_bounds__(kT) void k_bonorm(const float *__restrict__ attn, const void *__restrict__ gate,
                                                const float *__restrict__ sgate, const float *__restrict__ w,
                                                float eps, uint16_t *__restrict__ x_out, int n) {
     static_assert(PT * (kHD / 8) <= kT && kT == kHD, "a thread per channel; one X store task per thread");
@@ -797,19 +810,29 @@ __global__ __launch_bounds__(kT) void k_bonorm(const float *__restrict__ attn, c
     __shared__ float cs[PT][kHD / 16];
     __shared__ float xs[PT][kHD];
     __shared__ float scale_s[PT];
+    __shared__ uint64_t exp2_lds[RAW ? 32 : 1];  // expf's table for the sigmoid
+    if constexpr (RAW) fill_exp2_lds_imm(exp2_lds);
     const int h = blockIdx.x, m0 = (int)blockIdx.y * PT, t = threadIdx.x, c = h * kHD + t;
     float a[PT], gt[PT], sg[PT];
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-        const size_t o = (size_t)(m0 + i < n ? m0 + i : n - 1) * kH + c;
-        a[i] = attn[o];
-        gt[i] = gate[o];
-        sg[i] = sgate[o];
+        const size_t m = m0 + i < n ? m0 + i : n - 1;
+        a[i] = attn[m * kH + c];
+        if constexpr (RAW) {
+            gt[i] = bf16_bits_to_f32(static_cast<const uint16_t *>(gate)[m * 4 * kH + 3 * kH + c]);
+        } else {
+            gt[i] = static_cast<const float *>(gate)[m * kH + c];
+            sg[i] = sgate[m * kH + c];
+        }
     }
     const float wt = w[t];
 #pragma unroll
     for (int i = 0; i < PT; ++i) as[i][t] = a[i];
     __syncthreads();
+    if constexpr (RAW) {
+#pragma unroll
+        for (int i = 0; i < PT; ++i) sg[i] = sigmoid_ref(gt[i], Exp2Lds{exp2_lds});
+    }
     if (t < PT * (kHD / 16)) {
         const int i = t / (kHD / 16), r = t % (kHD / 16);
         float s = 0.0f;
@@ -932,17 +955,19 @@ __global__ __launch_bounds__(kT, 2) void k_brecur(const float *__restrict__ qkv,
 // multi-stream step, so a prefill of n tokens equals n steps bit for bit.
 
 // The causal conv of one 64-channel block over 64 tokens of a segment of n:
-// grid (4 kH / 64, ceil(n / 64)), thread 16 r + j on channels 4 j .. 4 j + 3
+// grid (4 kH / 64, ceil(n / 64)), with B16 (3 kH / 64, ..), the gate left to
+// k_bonorm; thread 16 r + j on channels 4 j .. 4 j + 3
 // of the block and tokens r, r + 16, r + 32, r + 48 (16-byte loads and
-// stores; the four loads in flight together).  raw is [n][4 kH] (the
-// unrounded q, k, v, g sums); the tails are the prefilled stream's for this
+// stores; the four loads in flight together).  raw is [n][4 kH]: the
+// unrounded q, k, v, g sums, or (B16) their roundings R(raw); the tails are the prefilled stream's for this
 // layer, [q,k,v][3 oldest..newest][kH].  Token m's window is (s[m], s[m+1],
 // s[m+2]) and its input s[m+3] in the sequence s = tails ++ R(raw[0..n));
 // the new tails are s[n], s[n+1], s[n+2].  Only the first token block reads
 // the old tails, and it writes the new ones after that read.
 constexpr int kConvT = 256;                  // threads per conv workgroup
 constexpr int kConvR = 16 * kMaxB / kConvT;  // tokens per thread
-__global__ __launch_bounds__(kConvT) void k_pconv(const float *__restrict__ raw, int n, uint16_t *__restrict__ tails,
+template <bool B16>
+__global__ __launch_bounds__(kConvT) void k_pconv(const void *__restrict__ raw, int n, uint16_t *__restrict__ tails,
                                                   const float *__restrict__ conv_w, float *__restrict__ qkv,
                                                   float *__restrict__ gate, float *__restrict__ sgate) {
     static_assert(kConvR * kConvT == 16 * kMaxB && kConvT >= 64, "16 lanes of 4 channels x kMaxB tokens");
@@ -957,14 +982,25 @@ __global__ __launch_bounds__(kConvT) void k_pconv(const float *__restrict__ raw,
     // tokens m0 + mr + MS i: raw sums of channels cb + c4 .. + 3.  Tokens
     // past the segment load its last token (in bounds, unused), so every
     // load is unconditional and all are in flight at once.
+    auto one = [&](int m) {  // R(raw) of token m, channel row0 + t
+        const size_t o = (size_t)m * 4 * kH + row0 + t;
+        if constexpr (B16) return bf16_bits_to_f32(static_cast<const uint16_t *>(raw)[o]);
+        else return rne_bf16(static_cast<const float *>(raw)[o]);
+    };
     f32x4 rr[kConvR];
 #pragma unroll
     for (int i = 0; i < kConvR; ++i) {
         const int m = mr + MS * i < nb ? mr + MS * i : nb - 1;
-        const f32x4 r = *reinterpret_cast<const f32x4 *>(raw + (size_t)(m0 + m) * 4 * kH + row0 + c4);
-        rr[i] = (f32x4){rne_bf16(r.x), rne_bf16(r.y), rne_bf16(r.z), rne_bf16(r.w)};
+        const size_t o = (size_t)(m0 + m) * 4 * kH + row0 + c4;
+        if constexpr (B16) {
+            const u32x2 r = *reinterpret_cast<const u32x2 *>(static_cast<const uint16_t *>(raw) + o);
+            rr[i] = (f32x4){u2f(r.x << 16), u2f(r.x & 0xffff0000u), u2f(r.y << 16), u2f(r.y & 0xffff0000u)};
+        } else {
+            const f32x4 r = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(raw) + o);
+            rr[i] = (f32x4){rne_bf16(r.x), rne_bf16(r.y), rne_bf16(r.z), rne_bf16(r.w)};
+        }
     }
-    if (which < 3) {
+    if (B16 || which < 3) {
         uint16_t *tl = tails + (size_t)which * 3 * kH + cb;
         const f32x4 *cw4 = reinterpret_cast<const f32x4 *>(conv_w + ((size_t)which * kH + cb + c4) * 4);
         const f32x4 cw[4] = {cw4[0], cw4[1], cw4[2], cw4[3]};
@@ -975,7 +1011,7 @@ __global__ __launch_bounds__(kConvT) void k_pconv(const float *__restrict__ raw,
                 xs[2][t] = bf16_bits_to_f32(tl[2 * kH + t]);
             } else {
 #pragma unroll
-                for (int i = 0; i < 3; ++i) xs[i][t] = rne_bf16(raw[(size_t)(m0 - 3 + i) * 4 * kH + row0 + t]);
+                for (int i = 0; i < 3; ++i) xs[i][t] = one(m0 - 3 + i);
             }
         }
 #pragma unroll
@@ -1006,8 +1042,7 @@ __global__ __launch_bounds__(kConvT) void k_pconv(const float *__restrict__ raw,
                 tl[2 * kH + t] = bf16_hi(xs[n + 2][t]);
             } else {
 #pragma unroll
-                for (int i = 0; i < 3; ++i)
-                    tl[i * kH + t] = bf16_hi(rne_bf16(raw[(size_t)(n - 3 + i) * 4 * kH + row0 + t]));
+                for (int i = 0; i < 3; ++i) tl[i * kH + t] = bf16_hi(one(n - 3 + i));
             }
         }
     } else {
@@ -1693,7 +1728,16 @@ constexpr int kPgW = GDN_PG_WAVES;
 // it to that split's plane of y (y_rows tokens), which the consumer adds in
 // split order, as it adds the step's: S times the workgroups of a kernel that
 // adds the splits itself, for segments whose tiles leave CUs idle.
-template <int KT, int NW, int S, bool PLANES>
+// B16: the sums are written rounded, as BF16 bits (the step rounds them before
+// anything else reads them), half the bytes for this kernel and its reader.
+__device__ __forceinline__ void pg_store(float *y, size_t o, const f32x4 v, bool b16) {
+    if (b16)
+        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(y) + o) =
+            make_uint2((f2u(rne_bf16(v.x)) >> 16) | f2u(rne_bf16(v.y)), (f2u(rne_bf16(v.z)) >> 16) | f2u(rne_bf16(v.w)));
+    else
+        *reinterpret_cast<f32x4 *>(y + o) = v;
+}
+template <int KT, int NW, int S, bool PLANES, bool B16>
 __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                      float *__restrict__ y, int n_rows, int y_rows) {
     constexpr int NT = PLANES ? KT / S : KT;  // k tiles of this workgroup
@@ -1736,9 +1780,6 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
     // group g of the wave: token 128 tt + 16 (TG wt + g) + l % 16
     const int row = 128 * rt + 64 * wr + 4 * (l >> 4);
     const int m = kPgTok * tt + 16 * TG * wt + (l & 15);
-    auto out = [&](int b) {
-        return reinterpret_cast<f32x4 *>(y + (size_t)(m + 16 * (b % TG)) * n_rows + row + 16 * (b / TG));
-    };
     u32x4 rg[kPgD][PT];
 #pragma unroll
     for (int d = 0; d < kPgD; ++d) fetch(rg[d], pg_tile<KT, NW, S>(jb + d));
@@ -1767,7 +1808,8 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
                         0, 0);
             if (pg_close<KT, NW, S, NB>(j, chain, part)) {
 #pragma unroll
-                for (int b = 0; b < NB; ++b) *out(b) = part[b];
+                for (int b = 0; b < NB; ++b)
+                    pg_store(y, (size_t)(m + 16 * (b % TG)) * n_rows + row + 16 * (b / TG), part[b], B16);
             }
         }
     }
@@ -1799,7 +1841,7 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
 constexpr int kPaW = 8;             // waves per workgroup
 constexpr int kPaRows = 32 * kPaW;  // rows per workgroup
 constexpr int kPaD = 2;             // k tiles of operands in flight
-template <int KT, int NW, int S, bool SWIGLU, bool PLANES>
+template <int KT, int NW, int S, bool SWIGLU, bool PLANES, bool B16>
 __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                               float *__restrict__ y, uint16_t *__restrict__ x_next, int n_rows,
                                               int n_tok) {
@@ -1860,9 +1902,6 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
     // g: token 128 tt + 16 g + l % 16
     const int row = kPaRows * rt + 32 * w + 4 * (l >> 4);
     const int m = kPgTok * tt + (l & 15);
-    auto out = [&](int f, int g) {
-        return reinterpret_cast<f32x4 *>(y + (size_t)(m + 16 * g) * n_rows + row + 16 * f);
-    };
     // the k tiles of class c, chained in acc from zero
     auto run_class = [&](int c, f32x4(&acc)[NB]) __attribute__((always_inline)) {
 #pragma unroll
@@ -1928,7 +1967,8 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
 #pragma unroll
         for (int f = 0; f < R; ++f)
 #pragma unroll
-            for (int g = 0; g < T; ++g) *out(f, g) = part[T * f + g];
+            for (int g = 0; g < T; ++g)
+                pg_store(y, (size_t)(m + 16 * g) * n_rows + row + 16 * f, part[T * f + g], B16);
     } else {
         // row tile 0: the gate rows of the wave's 16 channels, tile 1 their
         // up rows, so a lane holds both of channels 4 (l / 16) .. + 3
@@ -1954,11 +1994,11 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
         }
     }
 }
-template <int KT, int NW, int S, bool PLANES>
+template <int KT, int NW, int S, bool PLANES, bool B16>
 __global__ __launch_bounds__(kPaW * 64) void k_pgemm_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                        float *__restrict__ y, int n_rows, int y_rows) {
     if constexpr (PLANES) y += (size_t)blockIdx.z * y_rows * n_rows;
-    pgemm_a_block<KT, NW, S, false, PLANES>(W, X, y, nullptr, n_rows, 0);
+    pgemm_a_block<KT, NW, S, false, PLANES, B16>(W, X, y, nullptr, n_rows, 0);
 }
 
 // Gate/up + SwiGLU on the same kernel: W in 32-row blocks of 16 channels'
@@ -1968,7 +2008,7 @@ __global__ __launch_bounds__(kPaW * 64) void k_pgemm_a(const u32x4 *__restrict__
 // reads 8 fragments from LDS per 16 MFMAs where k_pgu's reads 5 per 6.
 __global__ __launch_bounds__(kPaW * 64) void k_pgu_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                      uint16_t *__restrict__ x_next, int n_tok) {
-    pgemm_a_block<kKtH, kGuWaves, 1, true, false>(W, X, nullptr, x_next, 2 * kI, n_tok);
+    pgemm_a_block<kKtH, kGuWaves, 1, true, false, false>(W, X, nullptr, x_next, 2 * kI, n_tok);
 }
 
 // One layer's gate/up weights from the step's 44-row groups (tile_gu) into
@@ -2397,7 +2437,7 @@ void launch_recur(GDNBatchEngine *e, int l, hipStream_t s) {
                        b_state(e, l), e->attn);
 }
 void launch_onorm(GDNBatchEngine *e, int l, hipStream_t s) {
-    hipLaunchKernelGGL(k_bonorm<1>, dim3(kNH, e->streams), dim3(kT), 0, s, e->attn, e->gate, e->sgate,
+    hipLaunchKernelGGL((k_bonorm<1, false>), dim3(kNH, e->streams), dim3(kT), 0, s, e->attn, e->gate, e->sgate,
                        b_aux(e, l) + kAuxONorm, e->eps, e->x_o, e->streams);
 }
 void launch_o(GDNBatchEngine *e, int l, hipStream_t s) {
@@ -2608,7 +2648,7 @@ enum PRoute {
 //   tokens                   64  256  512  768 1024 1536 2048 2560 3072 4096
 //   q/k/v/g  step            12   28   49    -   91    -  174    -    -    -
 //            tile            30   30   32   42   42    -   79    -    -    -
-//            wide             -    -    -    -   39   62   75   96  106  140
+//            wide             -    -    -    -   34   56   66   89   96  128
 //   o_proj   step             5    9   15    -   26    -   49    -    -    -
 //            planes          11   11   13   18   20   29   38   46   54   69
 //            wide             -    -   33   33   34   35   37   38   39   41
@@ -2618,7 +2658,7 @@ enum PRoute {
 //            wide             -    -   78   77   80   80   84   85   85   90
 //   gate/up  step            15   33   57    -  107    -  207    -    -    -
 //            tile            30   31   45   63   81  120  151    -    -  280
-//            wide             -    -   42    -    -    -  114  151  183  223
+//            wide             -    -   42    -   73    -  109  144  179  219
 // and the norm that reads four planes in place of one sum costs more: 8.3
 // against 6.8 at 512 tokens, 12.6 / 9.7 at 1024, 19 / 13 at 1536, 25 / 18 at
 // 2048, 30 / 21 at 2560, 37 / 24 at 3072.
@@ -2634,7 +2674,7 @@ PRoute route_down(int n) {
     return 65 * ((p_tiles(n) + 7) / 8) <= 11 * p_tiles(n) + 10 ? P_WIDE_PLANES : P_PLANES;
 }
 // k_pgu_a takes whole rounds of 256 workgroups (one per CU, 44 per 128 tokens),
-// about 38 us each; k_pgu (two per CU) about 8.5 us per 128 tokens and 14.
+// about 37 us each; k_pgu (two per CU) about 8.5 us per 128 tokens and 14.
 bool pgu_a_pays(int n) {
     const int rounds = (2 * kI / kPaRows * p_tiles(n) + 255) / 256;
     return 76 * rounds <= 17 * p_tiles(n) + 22;
@@ -2643,8 +2683,9 @@ PRoute route_gu(int n) { return n <= 192 ? P_STEP : pgu_a_pays(n) ? P_WIDE : P_T
 
 // A projection in 32-row blocks of KT k tiles, NW classes and S splits:
 // returns the planes of y (y_rows tokens each) that its consumer adds: S, or
-// 1 (the total).
-template <int KT, int NW, int S>
+// 1 (the total).  P_WIDE and P_TILE write rounded sums as BF16 bits with B16
+// (without, the test of the sums reads them whole); the others FP32.
+template <int KT, int NW, int S, bool B16>
 int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int rows, int n, int y_rows,
                   hipStream_t s) {
     const int blocks = (n + kMaxB - 1) / kMaxB, tiles = p_tiles(n);
@@ -2658,20 +2699,23 @@ int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int ro
         return S;
     }
     if (route == P_WIDE) {
-        hipLaunchKernelGGL((k_pgemm_a<KT, NW, S, false>), dim3(rows / kPaRows, tiles), dim3(kPaW * 64), 0, s, w, x, y,
+        hipLaunchKernelGGL((k_pgemm_a<KT, NW, S, false, B16>), dim3(rows / kPaRows, tiles), dim3(kPaW * 64), 0, s, w, x, y,
                            rows, 0);
         return 1;
     }
     if constexpr (S > 1) {
-        if (route == P_WIDE_PLANES)
-            hipLaunchKernelGGL((k_pgemm_a<KT, NW, S, true>), dim3(rows / kPaRows, tiles, S), dim3(kPaW * 64), 0, s, w,
-                               x, y, rows, y_rows);
-        else
-            hipLaunchKernelGGL((k_pgemm<KT, NW, S, true>), dim3(rows / 128, tiles, S), dim3(kPgW * 64), 0, s, w, x, y,
-                               rows, y_rows);
+        if constexpr (KT == kKtI) {
+            if (route == P_WIDE_PLANES) {
+                hipLaunchKernelGGL((k_pgemm_a<KT, NW, S, true, false>), dim3(rows / kPaRows, tiles, S),
+                                   dim3(kPaW * 64), 0, s, w, x, y, rows, y_rows);
+                return S;
+            }
+        }
+        hipLaunchKernelGGL((k_pgemm<KT, NW, S, true, false>), dim3(rows / 128, tiles, S), dim3(kPgW * 64), 0, s, w, x,
+                           y, rows, y_rows);
         return S;
     } else {
-        hipLaunchKernelGGL((k_pgemm<KT, NW, 1, false>), dim3(rows / 128, tiles), dim3(kPgW * 64), 0, s, w, x, y, rows,
+        hipLaunchKernelGGL((k_pgemm<KT, NW, 1, false, B16>), dim3(rows / 128, tiles), dim3(kPgW * 64), 0, s, w, x, y, rows,
                            0);
         return 1;
     }
@@ -2716,13 +2760,14 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
     launch_ab(0);
     const u32x4 *xh = reinterpret_cast<const u32x4 *>(e->s_xh), *xo = reinterpret_cast<const u32x4 *>(e->s_xo),
                 *xd = reinterpret_cast<const u32x4 *>(e->s_xd);
+    const PRoute r_qkvg = route_qkvg(4 * kH, n);
     const PRoute gu = route_gu(n) == P_WIDE && !e->gu_mem ? P_TILE : route_gu(n);
     for (int l = 0; l < e->layers; ++l) {
         float *st = b_state(e, l) + (size_t)slot * kLayerState;
         uint16_t *tl = b_tails(e, l) + (size_t)slot * kStreamTails;
-        launch_p_gemm<kKtH, 8, 1>(route_qkvg(4 * kH, n), e->w_qkvg[l], xh, e->s_y, 4 * kH, n, e->seg_cap, s);
-        hipLaunchKernelGGL(k_pconv, dim3(4 * kH / 64, blocks), dim3(kConvT), 0, s, e->s_y, n, tl,
-                           b_aux(e, l) + kAuxConv, e->s_qkv, e->s_gate, e->s_sgate);
+        launch_p_gemm<kKtH, 8, 1, true>(r_qkvg, e->w_qkvg[l], xh, e->s_y, 4 * kH, n, e->seg_cap, s);
+        hipLaunchKernelGGL(r_qkvg == P_STEP ? k_pconv<false> : k_pconv<true>,
+                           dim3((r_qkvg == P_STEP ? 4 : 3) * kH / 64, blocks), dim3(kConvT), 0, s, e->s_y, n, tl, b_aux(e, l) + kAuxConv, e->s_qkv, e->s_gate, e->s_sgate);
         if (e->prefill_mode == GDN_PREFILL_CHUNKED) {
             hipLaunchKernelGGL(k_wy_prep, dim3(kNH, blocks), dim3(kT), 0, s, e->s_qkv, e->s_bd, n, e->s_wy);
             hipLaunchKernelGGL(k_wy_seq, dim3(kNH * (kHD / kWyCols)), dim3(kWyWaves * 64), 0, s, e->s_qkv, e->s_wy, n, st,
@@ -2733,13 +2778,15 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
             hipLaunchKernelGGL(k_pscan, dim3(kHD / kScanWgCols, kNH), dim3(kT), 0, s, e->s_qkv, e->s_qn, e->s_kn,
                                e->s_alpha, e->s_bd, n, st, e->s_attn);
         }
-        hipLaunchKernelGGL(k_bonorm<kOnTok>, dim3(kNH, (n + kOnTok - 1) / kOnTok), dim3(kT), 0, s, e->s_attn,
-                           e->s_gate, e->s_sgate, b_aux(e, l) + kAuxONorm, e->eps, e->s_xo, n);
-        const int po = launch_p_gemm<kKtH, 4, kSplitO>(route_o(n), e->w_o[l], xo, e->s_y, kH, n, e->seg_cap, s);
+        const bool raw = r_qkvg != P_STEP;
+        hipLaunchKernelGGL((raw ? k_bonorm<kOnTok, true> : k_bonorm<kOnTok, false>),
+                           dim3(kNH, (n + kOnTok - 1) / kOnTok), dim3(kT), 0, s, e->s_attn,
+                           raw ? e->s_y : e->s_gate, e->s_sgate, b_aux(e, l) + kAuxONorm, e->eps, e->s_xo, n);
+        const int po = launch_p_gemm<kKtH, 4, kSplitO, true>(route_o(n), e->w_o[l], xo, e->s_y, kH, n, e->seg_cap, s);
         launch_p_norm(seg_norm(e, e->s_y, b_aux(e, l) + kAuxMlpNorm, e->s_xh, -1, l, l), po, n, s);
         launch_p_gu(gu, e->w_gu[l], e->w_gup[l], xh, e->s_xd, n, s);
         const int pd =
-            launch_p_gemm<kKtI, 4, kSplitDown>(route_down(n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
+            launch_p_gemm<kKtI, 4, kSplitDown, true>(route_down(n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
         if (l + 1 < e->layers) {
             BNorm pa = seg_norm(e, e->s_y, b_aux(e, l + 1) + kAuxAttnNorm, e->s_xh, -1, l, l + 1);
             pa.xn_out = e->s_xn;
@@ -3138,9 +3185,9 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
         GDN_HIP(hipMemset(dy, 0, out_elems * 4));
         int planes = 1;
         float *y = static_cast<float *>(dy);
-        if (kind == 0) planes = launch_p_gemm<kKtH, 8, 1>(route, w4, x4, y, rows, toks, pad, nullptr);
-        if (kind == 1) planes = launch_p_gemm<kKtH, 4, kSplitO>(route, w4, x4, y, rows, toks, pad, nullptr);
-        if (kind == 2) planes = launch_p_gemm<kKtI, 4, kSplitDown>(route, w4, x4, y, rows, toks, pad, nullptr);
+        if (kind == 0) planes = launch_p_gemm<kKtH, 8, 1, false>(route, w4, x4, y, rows, toks, pad, nullptr);
+        if (kind == 1) planes = launch_p_gemm<kKtH, 4, kSplitO, false>(route, w4, x4, y, rows, toks, pad, nullptr);
+        if (kind == 2) planes = launch_p_gemm<kKtI, 4, kSplitDown, false>(route, w4, x4, y, rows, toks, pad, nullptr);
         if (kind == 3)
             launch_p_gu(route, w4, static_cast<const u32x4 *>(dp), x4, static_cast<uint16_t *>(dy), toks, nullptr);
         GDN_HIP(hipGetLastError());
@@ -3166,7 +3213,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     const bool wide = kind == 3 || N % kPaRows == 0;
     if (wide) routes.insert(routes.begin(), P_WIDE);
     else std::swap(routes[0], routes[1]);
-    if (wide && (kind == 1 || kind == 2)) routes.push_back(P_WIDE_PLANES);
+    if (wide && kind == 2) routes.push_back(P_WIDE_PLANES);
     std::vector<float> first, other;
     std::vector<uint16_t> first16, other16;
     if (run_route(routes[0], first, first16)) return -1;
