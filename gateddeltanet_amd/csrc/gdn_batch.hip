@@ -1855,6 +1855,19 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
 constexpr int kPaW = 8;             // waves per workgroup
 constexpr int kPaRows = 32 * kPaW;  // rows per workgroup
 constexpr int kPaD = 2;             // k tiles of operands in flight
+
+// The i-th of the 16 channels of k_pgu_a's block b: eight of 11 blocks are the
+// first 16 channels of a 22-channel group (whole tiles of its weights), three
+// the last six of those eight groups.  Channels i and i + 1 (i even) are
+// neighbours.
+__device__ __forceinline__ int gu_channel(int b, int i) {
+    constexpr int kTail = kGuCh - 16;
+    static_assert(8 * kTail == 3 * 16 && kGuWgs % 8 == 0 && kTail % 2 == 0, "three blocks of tails per eight groups");
+    const int g0 = 8 * (b / 11), q = b % 11;
+    if (q < 8) return (g0 + q) * kGuCh + i;
+    const int t = 16 * (q - 8) + i;
+    return (g0 + t / kTail) * kGuCh + 16 + t % kTail;
+}
 template <int KT, int NW, int S, bool SWIGLU, bool PLANES, bool B16>
 __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                               float *__restrict__ y, uint16_t *__restrict__ x_next, int n_rows,
@@ -1875,8 +1888,20 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
     int rt, tt;
     pg_place(rt, tt);
     // wave w's rows: 32-row block kPaW rt + w of the weight layout (its two
-    // tiles at entries 0..63 and 64..127 of each k tile)
-    const u32x4 *ap = W + (size_t)(kPaW * rt + w) * KT * 128 + l;
+    // tiles at entries 0..63 and 64..127 of each k tile), or the gate and up
+    // rows of the 16 channels gu_channel names, in k_bgu's 44-row groups
+    constexpr int AS = SWIGLU ? kGuTileU4 : 128;  // entries per k tile
+    const u32x4 *ap[R];
+#pragma unroll
+    for (int f = 0; f < R; ++f) {
+        if constexpr (SWIGLU) {
+            const int c = gu_channel(kPaW * rt + w, l & 15), g = c / kGuCh, r = c % kGuCh;
+            ap[f] = W + (size_t)g * KT * AS +
+                    (r < 16 ? 64 * f + l : 128 + (l >> 4) * kGuTail2 + (r - 16) + f * (kGuCh - 16));
+        } else {
+            ap[f] = W + (size_t)(kPaW * rt + w) * KT * AS + 64 * f + l;
+        }
+    }
     // B entry q of a k tile: token group q / 64 (of 8), lane q % 64
     const u32x4 *bp[PB];
 #pragma unroll
@@ -1891,7 +1916,7 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
     auto load_a = [&](u32x4(&r)[R], int j) __attribute__((always_inline)) {
         const int kt = pg_tile<KT, NW, S>(j < je ? j : je - 1);
 #pragma unroll
-        for (int f = 0; f < R; ++f) r[f] = ap[(size_t)kt * 128 + 64 * f];
+        for (int f = 0; f < R; ++f) r[f] = ap[f][(size_t)kt * AS];
     };
     auto load_b = [&](u32x4(&r)[PB], int j) __attribute__((always_inline)) {
         const int kt = pg_tile<KT, NW, S>(j < je ? j : je - 1);
@@ -1985,9 +2010,10 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
                 pg_store(y, (size_t)(m + 16 * g) * n_rows + row + 16 * f, part[T * f + g], B16);
     } else {
         // row tile 0: the gate rows of the wave's 16 channels, tile 1 their
-        // up rows, so a lane holds both of channels 4 (l / 16) .. + 3
+        // up rows, so a lane holds both of the wave's channels 4 (l / 16) .. + 3
         // (gemv32_store SwiGLU branch, gdn_model.cpp:4751-4767)
-        const int ch = 16 * (kPaW * rt + w) + 4 * (l >> 4);
+        // channels of a pair are neighbours, pairs need not be (gu_channel)
+        const int k0 = gu_channel(kPaW * rt + w, 4 * (l >> 4)), k2 = gu_channel(kPaW * rt + w, 4 * (l >> 4) + 2);
         // one token group per trip, the next ones moved down (unrolled, the
         // eight groups' SiLUs are 50 KB of code)
 #pragma unroll 1
@@ -1997,9 +2023,10 @@ __device__ __forceinline__ void pgemm_a_block(const u32x4 *__restrict__ W, const
             for (int e = 0; e < 4; ++e)
                 hv[e] = bf16_daz_bits(rne_bf16(silu_ref(rne_bf16(part[0][e]), Exp2Lds{exp2_lds}) *
                                                rne_bf16(part[T][e])));
-            if (m + 16 * g < n_tok)
-                *reinterpret_cast<uint2 *>(x_next + xt_index(m + 16 * g, ch, kI)) =
-                    make_uint2(hv[0] | (hv[1] << 16), hv[2] | (hv[3] << 16));
+            if (m + 16 * g < n_tok) {
+                *reinterpret_cast<uint32_t *>(x_next + xt_index(m + 16 * g, k0, kI)) = hv[0] | (hv[1] << 16);
+                *reinterpret_cast<uint32_t *>(x_next + xt_index(m + 16 * g, k2, kI)) = hv[2] | (hv[3] << 16);
+            }
 #pragma unroll
             for (int i = 0; i + 1 < T; ++i) {
                 part[i] = part[i + 1];
@@ -2015,26 +2042,19 @@ __global__ __launch_bounds__(kPaW * 64) void k_pgemm_a(const u32x4 *__restrict__
     pgemm_a_block<KT, NW, S, false, PLANES, B16>(W, X, y, nullptr, n_rows, 0);
 }
 
-// Gate/up + SwiGLU on the same kernel: W in 32-row blocks of 16 channels'
-// gate rows then their up rows (k_gu_pairs), classes as k_bgu's, so the sums
-// are the step's; the first n_tok tokens are written.  All rows carry
-// weights, where the 44-row groups of k_pgu leave 4 of 48 empty, and a wave
-// reads 8 fragments from LDS per 16 MFMAs where k_pgu's reads 5 per 6.
+// Gate/up + SwiGLU on the same kernel, over the step's weights: a wave takes
+// 16 channels' gate rows and their up rows out of k_bgu's 44-row groups, classes
+// as k_bgu's, so the sums are the step's; the first n_tok tokens are written.
+// All rows carry weights, where the 44-row groups of k_pgu leave 4 of 48 empty,
+// and a wave reads 8 fragments from LDS per 16 MFMAs where k_pgu's reads 5 per 6.
+// A copy of the weights in 32-row blocks of 16 channels in order (46 MB a layer)
+// took 205-208 us at 4096 tokens and 73 at 1000 where this takes 212-214 and 75,
+// and 42 at 400 to 640 tokens where this takes 40; channels in order out of the
+// groups, 224, 76 and 41.
 __global__ __launch_bounds__(kPaW * 64) void k_pgu_a(const u32x4 *__restrict__ W, const u32x4 *__restrict__ X,
                                                      uint16_t *__restrict__ x_next, int n_tok) {
     pgemm_a_block<kKtH, kGuWaves, 1, true, false, false>(W, X, nullptr, x_next, 2 * kI, n_tok);
 }
-
-// One layer's gate/up weights from the step's 44-row groups (tile_gu) into
-// k_pgu_a's blocks: grid (kI / 16, kKtH), block of 128: entry (tile, lane) of
-// block b and k tile kt.
-__global__ __launch_bounds__(128) void k_gu_pairs(const u32x4 *__restrict__ src, u32x4 *__restrict__ dst) {
-    const int b = blockIdx.x, kt = blockIdx.y, up = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int ch = 16 * b + (l & 15), g = ch / kGuCh, r = ch % kGuCh, kq = l >> 4;
-    const int at = r < 16 ? 64 * up + 16 * kq + r : 128 + kq * kGuTail2 + (r - 16) + up * (kGuCh - 16);
-    dst[((size_t)b * kKtH + kt) * 128 + threadIdx.x] = src[((size_t)g * kKtH + kt) * kGuTileU4 + at];
-}
-
 
 // Gate/up + SwiGLU for channel groups 2 rt, +1 (k_bgu's layout and sums:
 // four classes of 16 k tiles) and tokens 128 tt .. +127 (pg_place; the
@@ -2178,9 +2198,6 @@ struct GDNBatchEngine {
     // the chunk matrices L and Mq, final hidden; X tiles of three widths)
     int seg_tokens = kSegDefault, seg_cap = 0;
     void *seg_mem = nullptr;
-    // k_pgu_a's copy of the gate/up weights, made at the first prefill
-    void *gu_mem = nullptr;
-    const u32x4 *w_gup[kMaxLayers] = {};
     float *s_h = nullptr, *s_y = nullptr, *s_qkv = nullptr, *s_gate = nullptr, *s_sgate = nullptr, *s_bd = nullptr,
           *s_attn = nullptr, *s_qn = nullptr, *s_kn = nullptr, *s_alpha = nullptr, *s_xn = nullptr;
     WyOps *s_wy = nullptr;
@@ -2596,28 +2613,6 @@ int seg_alloc(GDNBatchEngine *e) {
     return 0;
 }
 
-// k_pgu_a's layout of every layer's gate/up weights (46 MB a layer beside the
-// step's), formed on the device for the first segment that takes it and kept.
-// Without the memory for it gu_mem stays NULL and the segment takes k_pgu.
-int gu_pairs(GDNBatchEngine *e) {
-    if (e->gu_mem) return 0;
-    const size_t per = (size_t)2 * kI * kH * 2;
-    const hipError_t rc = hipMalloc(&e->gu_mem, (size_t)e->layers * per);
-    if (rc != hipSuccess) e->gu_mem = nullptr;
-    if (rc == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    GDN_HIP(rc);
-    for (int l = 0; l < e->layers; ++l) {
-        u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(e->gu_mem) + (size_t)l * per);
-        hipLaunchKernelGGL(k_gu_pairs, dim3(kI / 16, kKtH), dim3(128), 0, e->stream, e->w_gu[l], dst);
-        e->w_gup[l] = dst;
-    }
-    GDN_HIP(hipGetLastError());
-    return 0;
-}
-
 // A segment's norm: the residual of layer l's attention block in buffer
 // l & 1 (as in the step), segment-sized.
 BNorm seg_norm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_out, int ab_layer, int l_in,
@@ -2736,14 +2731,13 @@ int launch_p_gemm(PRoute route, const u32x4 *w, const u32x4 *x, float *y, int ro
 }
 static_assert(kRtO == 2 && kRtDown == 2, "o_proj and down in 32-row blocks");
 
-// Gate/up on the step's layout w, or (P_WIDE) k_pgu_a's layout wp.
-void launch_p_gu(PRoute route, const u32x4 *w, const u32x4 *wp, const u32x4 *x, uint16_t *x_next, int n,
-                 hipStream_t s) {
+// Gate/up on the step's layout.
+void launch_p_gu(PRoute route, const u32x4 *w, const u32x4 *x, uint16_t *x_next, int n, hipStream_t s) {
     const int tiles = (n + kPgTok - 1) / kPgTok;
     if (route == P_STEP)
         launch_bgu(n, (n + kMaxB - 1) / kMaxB, w, x, x_next, s);
     else if (route == P_WIDE)
-        hipLaunchKernelGGL(k_pgu_a, dim3(2 * kI / kPaRows, tiles), dim3(kPaW * 64), 0, s, wp, x, x_next, n);
+        hipLaunchKernelGGL(k_pgu_a, dim3(2 * kI / kPaRows, tiles), dim3(kPaW * 64), 0, s, w, x, x_next, n);
     else
         hipLaunchKernelGGL(k_pgu, dim3(kGuWgs / 2, tiles), dim3(kPgW * 64), 0, s, w, x, x_next, n);
 }
@@ -2775,7 +2769,6 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
     const u32x4 *xh = reinterpret_cast<const u32x4 *>(e->s_xh), *xo = reinterpret_cast<const u32x4 *>(e->s_xo),
                 *xd = reinterpret_cast<const u32x4 *>(e->s_xd);
     const PRoute r_qkvg = route_qkvg(4 * kH, n);
-    const PRoute gu = route_gu(n) == P_WIDE && !e->gu_mem ? P_TILE : route_gu(n);
     for (int l = 0; l < e->layers; ++l) {
         float *st = b_state(e, l) + (size_t)slot * kLayerState;
         uint16_t *tl = b_tails(e, l) + (size_t)slot * kStreamTails;
@@ -2798,7 +2791,7 @@ void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipS
                            raw ? e->s_y : e->s_gate, e->s_sgate, b_aux(e, l) + kAuxONorm, e->eps, e->s_xo, n);
         const int po = launch_p_gemm<kKtH, 4, kSplitO, true>(route_o(n), e->w_o[l], xo, e->s_y, kH, n, e->seg_cap, s);
         launch_p_norm(seg_norm(e, e->s_y, b_aux(e, l) + kAuxMlpNorm, e->s_xh, -1, l, l), po, n, s);
-        launch_p_gu(gu, e->w_gu[l], e->w_gup[l], xh, e->s_xd, n, s);
+        launch_p_gu(route_gu(n), e->w_gu[l], xh, e->s_xd, n, s);
         const int pd =
             launch_p_gemm<kKtI, 4, kSplitDown, true>(route_down(n), e->w_down[l], xd, e->s_y, kH, n, e->seg_cap, s);
         if (l + 1 < e->layers) {
@@ -2837,7 +2830,6 @@ int b_prefill(GDNBatchEngine *e, int slot, const int32_t *prompt, uint32_t n_tok
     int n = 0;
     for (uint32_t off = 0; off < n_tokens; off += seg) {
         n = (int)std::min<uint32_t>(seg, n_tokens - off);
-        if (route_gu(n) == P_WIDE && gu_pairs(e)) return -1;
         GDN_HIP(hipMemcpyAsync(e->s_tok, prompt + off, (size_t)n * sizeof(int), hipMemcpyHostToDevice, e->stream));
         enqueue_prefill_segment(e, slot, n, off + (uint32_t)n == n_tokens, e->stream);
         GDN_HIP(hipGetLastError());
@@ -2876,7 +2868,6 @@ void b_destroy(GDNBatchEngine *e) {
     (void)hipFree(e->p_logits);
     (void)hipFree(e->p_tok);
     (void)hipFree(e->seg_mem);
-    (void)hipFree(e->gu_mem);
     if (e->tok_host) (void)hipHostFree(e->tok_host);
     delete e;
 }
@@ -3179,7 +3170,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     for (uint32_t b = 0; b < blocks; ++b)
         gdn_tile_bf16(xb.data() + (size_t)b * kMaxB * K, kMaxB, K, 4, xt.data() + (size_t)b * kMaxB * K);
     const size_t out_elems = kind == 3 ? (size_t)tp * kI : (size_t)kSplitDown * tp * N;
-    void *dw = nullptr, *dx = nullptr, *dy = nullptr, *dr = nullptr, *dp = nullptr;
+    void *dw = nullptr, *dx = nullptr, *dy = nullptr, *dr = nullptr;
     GDN_HIP(hipMalloc(&dw, wt.size() * 2));
     GDN_HIP(hipMalloc(&dx, xt.size() * 2));
     GDN_HIP(hipMalloc(&dy, out_elems * 4));
@@ -3188,10 +3179,6 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     GDN_HIP(hipMemcpy(dw, wt.data(), wt.size() * 2, hipMemcpyHostToDevice));
     GDN_HIP(hipMemcpy(dx, xt.data(), xt.size() * 2, hipMemcpyHostToDevice));
     const u32x4 *w4 = static_cast<const u32x4 *>(dw), *x4 = static_cast<const u32x4 *>(dx);
-    if (kind == 3) {
-        GDN_HIP(hipMalloc(&dp, wt.size() * 2));
-        hipLaunchKernelGGL(k_gu_pairs, dim3(kI / 16, kKtH), dim3(128), 0, 0, w4, static_cast<u32x4 *>(dp));
-    }
     // one route into out (floats of a zeroed buffer's planes added in order,
     // or the X tiles' halves)
     const int rows = (int)N, toks = (int)T, pad = (int)tp;
@@ -3203,7 +3190,7 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
         if (kind == 1) planes = launch_p_gemm<kKtH, 4, kSplitO, false>(route, w4, x4, y, rows, toks, pad, nullptr);
         if (kind == 2) planes = launch_p_gemm<kKtI, 4, kSplitDown, false>(route, w4, x4, y, rows, toks, pad, nullptr);
         if (kind == 3)
-            launch_p_gu(route, w4, static_cast<const u32x4 *>(dp), x4, static_cast<uint16_t *>(dy), toks, nullptr);
+            launch_p_gu(route, w4, x4, static_cast<uint16_t *>(dy), toks, nullptr);
         GDN_HIP(hipGetLastError());
         GDN_HIP(hipDeviceSynchronize());
         if (kind == 3) {
@@ -3293,7 +3280,6 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     (void)hipFree(dx);
     (void)hipFree(dy);
     (void)hipFree(dr);
-    (void)hipFree(dp);
     return 0;
 }
 

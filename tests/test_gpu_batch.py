@@ -530,6 +530,33 @@ def test_prefill_chunked_edges(n):
     assert diff < 5e-7
 
 
+def test_prefill_holds_no_second_copy_of_the_weights():
+    """The segment buffers are all that a prefill keeps: once they are there, a
+    512-token prompt (every projection on a 128-token kernel) leaves the free
+    device memory as it was, to 8 MB for the runtime's own (a layer's gate/up
+    weights are 46 MB)."""
+    import ctypes
+
+    from test_zz_no_alloc import _hip
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    m = g.Model.synth(num_layers=1, seed=5, std=0.02, bf16=True)
+    bs = g.BatchState(m, 1)
+    try:
+        bs.set_prefill_segment(512)
+        bs.prefill(0, g.synth_tokens(64, 23, 7))
+        before = free_bytes()
+        bs.prefill(0, g.synth_tokens(512, 23, 8))
+        assert before - free_bytes() < 8 << 20
+    finally:
+        bs.free()
+        m.free()
+
+
 def test_prefill_continues_a_decoded_stream(model):
     """A prefill on a stream that has already decoded tokens continues from
     its state and conv tails: 5 steps then a 70-token prefill equal 75
