@@ -1666,6 +1666,7 @@ constexpr int kPgD = GDN_PG_DEPTH;  // k tiles of operand loads in flight per th
 constexpr int kPgTok = 128;  // tokens per workgroup (2 X tile blocks)
 constexpr int kSegDefault = 4096;  // prefill tokens per segment by default
 constexpr int kSegMax = 32768;     // largest segment (k_pqk's grid.y holds it)
+constexpr int kStepTok = 256;      // longest segment whose q/k/v/g take the step's kernel (and gate buffers)
 
 // The j-th k tile in class order: split s, class c, i-th tile of the class.
 template <int KT, int NW, int S>
@@ -2579,9 +2580,10 @@ int seg_alloc(GDNBatchEngine *e) {
     e->seg_mem = nullptr;
     e->seg_cap = 0;
     const size_t T = (size_t)e->seg_tokens, chunks = T / kMaxB;
+    const size_t TG = std::min(T, (size_t)kStepTok);  // longer ones leave the gate in s_y
     // normalised q and k (scan) or k_wy_seq's operands (chunked)
     const size_t qk = std::max(T * 2 * kH, chunks * kNH * sizeof(WyOps) / sizeof(float));
-    const size_t floats = T * (2 * kH + 4 * kH + 3 * kH + kH + kH + 16 + kH + kNH + kH) + qk;
+    const size_t floats = T * (2 * kH + 4 * kH + 3 * kH + 16 + kH + kNH + kH) + TG * 2 * kH + qk;
     const size_t halves = T * (kH + kH + kI);
     const size_t bytes = floats * 4 + halves * 2 + T * sizeof(int);
     GDN_HIP(hipMalloc(&e->seg_mem, bytes));
@@ -2594,8 +2596,8 @@ int seg_alloc(GDNBatchEngine *e) {
     e->s_h = p; p += 2 * T * kH;
     e->s_y = p; p += 4 * T * kH;
     e->s_qkv = p; p += 3 * T * kH;
-    e->s_gate = p; p += T * kH;
-    e->s_sgate = p; p += T * kH;
+    e->s_gate = p; p += TG * kH;
+    e->s_sgate = p; p += TG * kH;
     e->s_bd = p; p += T * 16;
     e->s_attn = p; p += T * kH;
     e->s_qn = p;
@@ -2673,7 +2675,7 @@ enum PRoute {
 // 2048, 30 / 21 at 2560, 37 / 24 at 3072.
 int p_tiles(int n) { return (n + kPgTok - 1) / kPgTok; }
 bool pa_fills(int rows, int n) { return rows % kPaRows == 0 && (rows / kPaRows) * p_tiles(n) >= 256; }
-PRoute route_qkvg(int rows, int n) { return n <= 256 ? P_STEP : pa_fills(rows, n) ? P_WIDE : P_TILE; }
+PRoute route_qkvg(int rows, int n) { return n <= kStepTok ? P_STEP : pa_fills(rows, n) ? P_WIDE : P_TILE; }
 PRoute route_o(int n) { return n <= 256 ? P_STEP : n <= 1536 ? P_PLANES : P_WIDE; }
 // down's wide planes take whole rounds of 256 workgroups (eight tiles, about
 // 26 us), its planes about 4.4 us a tile and 4.

@@ -538,7 +538,7 @@ int gdn_batch_save_stream_state(const GDNBatchState *state, uint32_t stream, flo
  * receives the argmax of the last position; that position's logits and final
  * hidden vector become the stream's readable ones.  Other streams' states
  * are untouched.  The first prefill allocates the segment's buffers (about
- * 150 KB per segment token, 0.6 GB at 4096), kept until the engine is freed
+ * 128 KB per segment token, 0.53 GB at 4096), kept until the engine is freed
  * or the segment length changes. */
 #define GDN_PREFILL_SCAN 0
 #define GDN_PREFILL_CHUNKED 1

@@ -25,10 +25,13 @@ arithmetic; it is 3-4e-2 from the BF16W arm after one layer):
   * 24 layers against the batch-1 engine: the measured gap is reported and
     bounded loosely (the random-init model amplifies rounding differences).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 import gateddeltanet_amd as g
+from test_zz_no_alloc import _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -530,28 +533,43 @@ def test_prefill_chunked_edges(n):
     assert diff < 5e-7
 
 
+def free_device_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_prefill_segment_memory():
+    """The buffers of a 4096-token segment: 525 MB for the tokens (128,230 B
+    each) and 4 MB for the gate of the segments of at most 256 tokens that
+    keep one, to 8 MB for the runtime's own."""
+    m = g.Model.synth(num_layers=1, seed=5, std=0.02, bf16=True)
+    bs = g.BatchState(m, 1)
+    try:
+        bs.step([1])
+        before = free_device_bytes()
+        bs.prefill(0, g.synth_tokens(64, 23, 7))
+        used = before - free_device_bytes()
+        print(f"4096-token segment: {used} bytes")
+        assert used < 4096 * 128_230 + (4 << 20) + (8 << 20)
+    finally:
+        bs.free()
+        m.free()
+
+
 def test_prefill_holds_no_second_copy_of_the_weights():
     """The segment buffers are all that a prefill keeps: once they are there, a
     512-token prompt (every projection on a 128-token kernel) leaves the free
     device memory as it was, to 8 MB for the runtime's own (a layer's gate/up
     weights are 46 MB)."""
-    import ctypes
-
-    from test_zz_no_alloc import _hip
-
-    def free_bytes():
-        free, total = ctypes.c_size_t(), ctypes.c_size_t()
-        assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-        return free.value
-
     m = g.Model.synth(num_layers=1, seed=5, std=0.02, bf16=True)
     bs = g.BatchState(m, 1)
     try:
         bs.set_prefill_segment(512)
         bs.prefill(0, g.synth_tokens(64, 23, 7))
-        before = free_bytes()
+        before = free_device_bytes()
         bs.prefill(0, g.synth_tokens(512, 23, 8))
-        assert before - free_bytes() < 8 << 20
+        assert before - free_device_bytes() < 8 << 20
     finally:
         bs.free()
         m.free()
