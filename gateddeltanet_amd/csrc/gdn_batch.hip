@@ -1173,13 +1173,19 @@ __device__ __forceinline__ f32x4 mfma_bf16(u32x4 a, u32x4 b, f32x4 c) {
 }
 
 // x as three BF16 terms: p[0] + p[1] + p[2] = x (each rounded to nearest, the
-// differences exact), four values packed in two words.
+// differences exact), four values packed in two words.  The first term is
+// held to the largest finite BF16 value, so every finite x of 2^-110 and more
+// is its terms' sum (rounded up to an infinity, that term would leave
+// infinity - infinity behind); below, the last terms are BF16 subnormals.  An
+// infinite or NaN x has a NaN term.
 __device__ __forceinline__ void split3(const f32x4 x, u32x2 (&p)[3]) {
+    constexpr float kMax = 0x1.fep127f;
+    auto held = [](float v) { return __builtin_amdgcn_fmed3f(v, -kMax, kMax); };
     f32x4 r = x;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-        p[i].x = cvt_pk(r.x, r.y);
-        p[i].y = cvt_pk(r.z, r.w);
+        p[i].x = i == 0 ? cvt_pk(held(r.x), held(r.y)) : cvt_pk(r.x, r.y);
+        p[i].y = i == 0 ? cvt_pk(held(r.z), held(r.w)) : cvt_pk(r.z, r.w);
         if (i < 2) {
             r.x = r.x - u2f(p[i].x << 16);
             r.y = r.y - u2f(p[i].x & 0xffff0000u);

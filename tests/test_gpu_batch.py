@@ -533,6 +533,32 @@ def test_prefill_chunked_edges(n):
     assert diff < 5e-7
 
 
+@pytest.mark.parametrize("n", [1, 20, 70])
+def test_prefill_chunked_largest_state(n):
+    """State elements above the largest finite BF16 value (3.39e38), one a
+    column, stay finite and as near the scan's as any others: the chunked
+    recurrence takes the state as a sum of BF16 terms, of which the first
+    would round to infinity.  1e-6: a few roundings of 2^-24 on the way to
+    each element, on either side."""
+    m = g.Model.synth(num_layers=1, seed=4, std=0.02, bf16=True)
+    rng = np.random.default_rng(n)
+    S = rng.standard_normal((8, 256, 256), dtype=np.float32)
+    S[:, rng.integers(0, 256, 256), np.arange(256)] = rng.choice([-1, 1], 256) * np.float32(3.4e38)
+    tails = np.zeros(9 * 2048, np.float32)
+    states = []
+    for mode in (g.PREFILL_SCAN, g.PREFILL_CHUNKED):
+        bs = g.BatchState(m, 1)
+        bs.set_prefill_mode(mode)
+        bs.load_stream_state(0, S.reshape(-1), tails)
+        bs.prefill(0, g.synth_tokens(n, 22, 6))
+        states.append(bs.save_stream_state(0)[0].astype(np.float64))
+        bs.free()
+    m.free()
+    scan, chunked = states
+    assert np.isfinite(scan).all() and np.isfinite(chunked).all()
+    assert np.linalg.norm(scan - chunked) < 1e-6 * np.linalg.norm(scan)
+
+
 def free_device_bytes():
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
     assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
