@@ -43,6 +43,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "gdn_amd.h"
@@ -3190,14 +3191,19 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
     // one route into out (floats of a zeroed buffer's planes added in order,
     // or the X tiles' halves)
     const int rows = (int)N, toks = (int)T, pad = (int)tp;
+    auto launch_route = [&](PRoute route, auto b16) {
+        constexpr bool B16 = decltype(b16)::value;
+        float *y = static_cast<float *>(dy);
+        if (kind == 0) return launch_p_gemm<kKtH, 8, 1, B16>(route, w4, x4, y, rows, toks, pad, nullptr);
+        if (kind == 1) return launch_p_gemm<kKtH, 4, kSplitO, B16>(route, w4, x4, y, rows, toks, pad, nullptr);
+        return launch_p_gemm<kKtI, 4, kSplitDown, B16>(route, w4, x4, y, rows, toks, pad, nullptr);
+    };
     auto run_route = [&](PRoute route, std::vector<float> &out, std::vector<uint16_t> &tiles16) -> int {
         GDN_HIP(hipMemset(dy, 0, out_elems * 4));
         int planes = 1;
-        float *y = static_cast<float *>(dy);
-        if (kind == 0) planes = launch_p_gemm<kKtH, 8, 1, false>(route, w4, x4, y, rows, toks, pad, nullptr);
-        if (kind == 1) planes = launch_p_gemm<kKtH, 4, kSplitO, false>(route, w4, x4, y, rows, toks, pad, nullptr);
-        if (kind == 2) planes = launch_p_gemm<kKtI, 4, kSplitDown, false>(route, w4, x4, y, rows, toks, pad, nullptr);
-        if (kind == 3)
+        if (kind < 3)
+            planes = launch_route(route, std::false_type{});
+        else
             launch_p_gu(route, w4, x4, static_cast<uint16_t *>(dy), toks, nullptr);
         GDN_HIP(hipGetLastError());
         GDN_HIP(hipDeviceSynchronize());
@@ -3234,6 +3240,26 @@ int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, 
             std::fprintf(stderr, "gdn_test_prefill_gemm: kind %d, route %d differs from route %d\n", kind,
                          (int)routes[r], (int)routes[0]);
             return -1;
+        }
+    }
+    // the stores of rounded sums, as the engine launches these routes: the
+    // rounding of the whole sums
+    for (PRoute route : {P_WIDE, P_TILE}) {
+        if (kind == 3 || (route == P_WIDE && !wide) || (route == P_TILE && kind != 0)) continue;
+        GDN_HIP(hipMemset(dy, 0, out_elems * 4));
+        launch_route(route, std::true_type{});
+        GDN_HIP(hipGetLastError());
+        GDN_HIP(hipDeviceSynchronize());
+        std::vector<uint16_t> half((size_t)T * N);
+        GDN_HIP(hipMemcpy(half.data(), dy, half.size() * 2, hipMemcpyDeviceToHost));
+        for (size_t i = 0; i < half.size(); ++i) {
+            uint32_t u;
+            std::memcpy(&u, &first[i], 4);
+            if (half[i] != (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16)) {
+                std::fprintf(stderr, "gdn_test_prefill_gemm: kind %d, route %d: a rounded sum differs\n", kind,
+                             (int)route);
+                return -1;
+            }
         }
     }
     // the step's kernels, one 64-token block at a time

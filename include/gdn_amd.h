@@ -578,8 +578,9 @@ int gdn_test_batch_gemm(const float *W, const float *X, uint32_t N, uint32_t K, 
  * (K 2048, 4 splits); 2: down's (K 5632, 4 splits); 3: gate/up + SwiGLU
  * (W = gate [5632][2048] then up rows, N = 5632; Y the BF16 SwiGLU values).
  * N a multiple of 128 for kinds 0-2; W and X BF16-exact.  Every kernel that
- * a prefill of some length takes for the kind is run; -1 when two of them
- * differ in a bit. */
+ * a prefill of some length takes for the kind is run (those of 256 rows a
+ * workgroup where N is a multiple of 256); -1 when two of them differ in a
+ * bit, or a kernel's store of rounded sums from its sums' rounding. */
 int gdn_test_prefill_gemm(int kind, const float *W, const float *X, uint32_t N, uint32_t T, float *Y,
                           float *Y_step);
 

@@ -110,9 +110,10 @@ def test_prefill_gemm_equals_step_gemm(kind, N, T):
 def test_prefill_gemm_routes_agree(kind, N, T):
     """Each kernel that a segment of some length takes for a projection (the
     step's over token blocks, the split planes, the 128-token tiles, 256 rows a
-    workgroup with the splits added or in planes) gives the
-    same bits, at a token past and short of their blocks: the call itself
-    fails if two differ, and its result is the step's."""
+    workgroup with the splits added or in planes; the 256-row ones where N is
+    a multiple of 256) gives the same bits, at a token past and short of their
+    blocks, and those that store rounded sums store these sums' rounding: the
+    call itself fails where that does not hold, and its result is the step's."""
     rng = np.random.default_rng(200 + 10 * kind + T)
     K = 5632 if kind == 2 else 2048
     shape = (2, N, K) if kind == 3 else (N, K)
