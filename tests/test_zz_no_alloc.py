@@ -116,11 +116,13 @@ def test_noalloc_recurrence_matches_allocating_entry_point(contract):
 
 
 # Step counts and head counts on both sides of the choice between one scan and
-# a launch per step (2 steps: 8 heads; 3: 96; 4), of the scan's 16-token
-# staging and of a scratch fill that leaves a chunk of one step (4 x 4097).
+# a launch per step (2 steps: 8 heads; 3: 96; 4) and of the scan's 16-token
+# staging; a scan fill followed by a fill of one step, which reuses the scratch
+# array in the per-step kernel's layout (192 heads: 85 + 1 steps); and fills of
+# three steps and of one, both per step (4097 heads).
 @pytest.mark.parametrize("contract", [g.CONTRACT_BF16W_FP32S, g.CONTRACT_REF, g.CONTRACT_FP32])
 @pytest.mark.parametrize("heads,steps", [(1, 1), (8, 2), (9, 2), (96, 3), (97, 3), (97, 4), (3, 15), (3, 16), (3, 17),
-                                         (1, 33), (4097, 4)])
+                                         (1, 33), (192, 86), (4097, 4)])
 def test_noalloc_recurrence_routes(contract, heads, steps):
     q, k, v, a, b, al, dt, S = _inputs(7 * heads + steps, steps, heads, contract)
     o_ref, S_ref = g.recurrence(contract, q, k, v, a, b, al, dt, S)
