@@ -124,7 +124,8 @@ def test_prefill_gemm_routes_agree(kind, N, T):
     assert same_bits(y, y_step)
 
 
-@pytest.mark.parametrize("n", [192, 193, 256, 257, 385, 512, 513, 641, 1024, 1025, 1536, 1537, 2560, 2561, 3073])
+@pytest.mark.parametrize("n", [192, 193, 256, 257, 384, 385, 512, 513, 640, 641, 896, 897, 1024, 1025, 1280, 1281, 1408,
+                               1409, 1536, 1537, 2560, 2561, 3073])
 def test_prefill_route_edges_equal_steps(n):
     """Prompts on both sides of each projection's change of kernel: a layer's
     state and the next token equal single-stream steps bit for bit."""
@@ -436,9 +437,9 @@ def stepped_reference(m, prompt):
 
 @pytest.mark.parametrize("n", [1, 2, 64, 65, 128, 150])
 def test_prefill_equals_steps(model, n):
-    """Prefill of n tokens (chunks of 64; n < 3 exercises the conv tails
-    alone, 64 / 65 / 128 the chunk edges) equals n single-stream steps bit
-    for bit, and leaves the other streams' states alone."""
+    """Prefill of n tokens (n < 3 exercises the conv tails alone, 64 / 65 /
+    128 the edges of the 64-token blocks) equals n single-stream steps bit for
+    bit, and leaves the other streams' states alone."""
     prompt = g.synth_tokens(n, 40 + n, 0)
     seed_ref, logits_ref, hidden_ref, (rec_ref, conv_ref) = stepped_reference(model, prompt)
     bs = g.BatchState(model, 3)
@@ -467,11 +468,10 @@ def test_prefill_equals_steps(model, n):
 
 @pytest.mark.parametrize("n", [4096, 4200])
 def test_prefill_long_segment_equals_steps(n):
-    """A 4096-token segment, where the engine runs the q/k/v/g and down
-    projections on k_pgemm_a (its grid fills the CUs only from 1024 and 4096
-    tokens), equals n single-stream steps bit for bit (2 layers); at 4200
-    the 104-token second segment runs them on k_pgemm, from the first
-    segment's state."""
+    """A 4096-token segment, whose projections all run on the kernels of 256
+    rows a workgroup, equals n single-stream steps bit for bit (2 layers); at
+    4200 a 104-token second segment, on the step's kernels, continues from the
+    first segment's state and conv tails."""
     m = g.Model.synth(num_layers=2, seed=4, std=0.02, bf16=True)
     try:
         prompt = g.synth_tokens(n, 44, 0)
