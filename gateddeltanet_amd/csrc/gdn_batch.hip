@@ -68,7 +68,7 @@ constexpr size_t kStreamTails = (size_t)3 * 3 * kH;      // floats per (layer, s
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-enum { EPI_RAW = 0, EPI_STORE = 1, EPI_QKVG = 2, EPI_LM = 4 };
+enum { EPI_RAW = 0, EPI_QKVG = 2, EPI_LM = 4 };
 
 // BF16 bits of a value already at a BF16 rounding point, subnormals flushed
 // to a signed zero (the reference's products treat them as zero).
@@ -102,7 +102,7 @@ __device__ __forceinline__ void store_x8(uint16_t *x, int m, int k, const float 
 struct BEpi {
     int n_streams;
     int n_rows;          // N: row stride of y / logits
-    float *y;            // EPI_RAW / EPI_STORE: [splits][y_rows][N]
+    float *y;            // EPI_RAW: [splits][y_rows][N]
     int y_rows;          // rows of one split's plane (64 in a step)
     float *qkv;          // EPI_QKVG: [64][3][kH] after conv + SiLU
     float *gate;         // [64][kH] R(g)
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
         for (int ww = 1; ww < NW; ++ww) v = v + red[ww * RT * G * 64 + idx];
         return v;
     };
-    if constexpr (EPI == EPI_RAW || EPI == EPI_STORE || EPI == EPI_LM) {
+    if constexpr (EPI == EPI_RAW || EPI == EPI_LM) {
 #pragma unroll
         for (int q = t; q < RT * 4 * 16 * G; q += GT) {
             const int m = q % (16 * G), nq = (q / (16 * G)) & 3, rt = q / (64 * G);
@@ -246,14 +246,7 @@ __global__ __launch_bounds__(NW * 64) void k_bgemm(const u32x4 *__restrict__ W, 
                 lm_v[rt * 4 + nq][m] = best;
                 lm_i[rt * 4 + nq][m] = idx;
             } else {
-                f32x4 o = v;
-                if constexpr (EPI == EPI_STORE) {
-                    o.x = rne_bf16(v.x);
-                    o.y = rne_bf16(v.y);
-                    o.z = rne_bf16(v.z);
-                    o.w = rne_bf16(v.w);
-                }
-                *reinterpret_cast<f32x4 *>(ep.y + ((size_t)sp * ep.y_rows + zb * 64 + m) * ep.n_rows + row) = o;
+                *reinterpret_cast<f32x4 *>(ep.y + ((size_t)sp * ep.y_rows + zb * 64 + m) * ep.n_rows + row) = v;
             }
         }
     } else if constexpr (EPI == EPI_QKVG) {
@@ -1666,10 +1659,7 @@ __global__ __launch_bounds__(kWyWaves * 64) void k_wy_seq(const float *__restric
 // its waves' sums; and the splits' sums added in split order, as the
 // step's norm adds k_bgemm's split partials.  A prefill therefore still
 // equals the steps bit for bit.
-#ifndef GDN_PG_DEPTH
-#define GDN_PG_DEPTH 2
-#endif
-constexpr int kPgD = GDN_PG_DEPTH;  // k tiles of operand loads in flight per thread
+constexpr int kPgD = 2;      // k tiles of operand loads in flight per thread
 constexpr int kPgTok = 128;  // tokens per workgroup (2 X tile blocks)
 constexpr int kSegDefault = 4096;  // prefill tokens per segment by default
 constexpr int kSegMax = 32768;     // largest segment (k_pqk's grid.y holds it)
@@ -1741,10 +1731,7 @@ __device__ __forceinline__ bool pg_close(int j, f32x4 (&chain)[NB], f32x4 (&part
 // Waves per workgroup: 8 of 64 rows x 32 tokens (about 100 VGPRs, four
 // waves per SIMD) measured 98.4k against 95.9k prefill tokens/s for 4 of
 // 64 x 64 (two per SIMD), with twice the LDS fragment reads.
-#ifndef GDN_PG_WAVES
-#define GDN_PG_WAVES 8
-#endif
-constexpr int kPgW = GDN_PG_WAVES;
+constexpr int kPgW = 8;
 
 // PLANES: grid z is the split; a workgroup forms one split's sum and writes
 // it to that split's plane of y (y_rows tokens), which the consumer adds in
@@ -1768,9 +1755,8 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgemm(const u32x4 *__restrict__ W
     const int jb = PLANES ? (int)blockIdx.z * NT : 0;
     if constexpr (PLANES) y += (size_t)blockIdx.z * y_rows * n_rows;
     constexpr int GT = kPgW * 64, AU = 4 * 2 * 64, BU = 2 * 4 * 64, PT = (AU + BU) / GT;
-    constexpr int TG = kPgW == 4 ? 4 : 2;  // 16-token groups per wave
+    constexpr int TG = 2;                 // 16-token groups per wave
     constexpr int NB = 4 * TG;            // 16 x 16 blocks per wave
-    static_assert(kPgW == 4 || kPgW == 8, "four or eight waves");
     static_assert(KT % kPgD == 0 && kPgD % 2 == 0, "whole groups of kPgD k tiles");
     __shared__ u32x4 stg[2][AU + BU];
     const int t = threadIdx.x, w = t >> 6, l = t & 63, wr = w & 1, wt = w >> 1;
@@ -2071,9 +2057,8 @@ __global__ __launch_bounds__(kPgW * 64) void k_pgu(const u32x4 *__restrict__ W, 
                                                    uint16_t *__restrict__ x_next, int n_tok) {
     constexpr int KT = kKtH, NW = kGuWaves, GT = kPgW * 64;
     constexpr int AU = 2 * kGuTileU4, BU = 2 * 4 * 64, PT = (AU + BU + GT - 1) / GT;
-    constexpr int TG = kPgW == 4 ? 4 : 2;  // 16-token groups per wave
+    constexpr int TG = 2;                 // 16-token groups per wave
     constexpr int NB = 3 * TG;            // 16 x 16 blocks per wave
-    static_assert(kPgW == 4 || kPgW == 8, "four or eight waves");
     static_assert(KT % kPgD == 0 && kPgD % 2 == 0, "whole groups of kPgD k tiles");
     __shared__ u32x4 stg[2][AU + BU];
     __shared__ f32x4 red[kPgW][NB * 64];
