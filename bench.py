@@ -521,8 +521,8 @@ def run_streams(B, steps, warm, eager, profile_rounds, cpu_tokens):
 def main_prefill(args):
     """The prompt pass: an N-token uniform prompt through one stream's state
     (gdn_batch_prefill: the prompt as one segment of up to 4096 tokens, run
-    layer by layer -- projections as matrix-core GEMMs, the recurrence over
-    64-token chunks in token order or in the WY form), timed against the same
+    layer by layer -- projections as matrix-core GEMMs, the recurrence in
+    token order or over 64-token chunks in the WY form), timed against the same
     prompt as N batch-1 decode steps (BF16W_FP32S); `value` is prefill
     tokens/s.  The warm-up prefill also allocates the segment buffers."""
     print(json.dumps(run_prefill(args.prefill, args.prefill_mode, args.eager)), flush=True)
@@ -569,7 +569,8 @@ def run_prefill(n, mode, eager, decode_steps=True):
         "dtype": "bf16",
         "data": "synthetic (seeded random-init weights, uniform random prompt)",
         "config": {"workload": f"{n}-token prompt through one stream, 24 layers, FP32 state, "
-                                f"segments of 4096 tokens layer by layer, recurrence chunks of 64",
+                                f"segments of 4096 tokens layer by layer, recurrence "
+                                + ("over 64-token chunks" if chunked else "in token order"),
                    "prefill_mode": mode,
                    "arithmetic": ("the multi-stream step's, with the recurrence in the chunk-parallel (WY) form "
                                   "(FP32 re-association)" if chunked else "the multi-stream step's, bit for bit")},

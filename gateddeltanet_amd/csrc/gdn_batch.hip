@@ -498,19 +498,6 @@ struct BNorm {
     float eps;
 };
 
-// Per stream: the residual add (or embedding import), the RMSNorm in chunk
-// order (gdn_rmsnorm_rows_bf16 / gdn_residual_rmsnorm_bf16,
-// gdn_model.cpp:1394-1474, :3351-3450) and, before an attention block, the
-// tiny a/b rows and beta/decay (gdn_gemv_tiny_ab :1501-1536, :2461-2465).
-// Thread t holds elements 8t..8t+7; a 16-element chunk is the sequential sum
-// of thread 2c's eight squares continued by thread 2c + 1.  SPLITS partial
-// sums of the preceding projection are added in split order (1: its rounded
-// sums as BF16 bits; 0: no residual add; EMBED: the embedding row instead).  Without AB one workgroup per
-// stream updates the residual in place.  With AB, grid (streams, kAbSplit):
-// workgroup j repeats the norm and runs the a/b rows of heads
-// kNH / kAbSplit * j .. (a 32 KB slice of the 128 KB of rows, requested
-// before the norm's first wait on memory); workgroup 0 alone writes the
-// residual, to h_out != h_in, and the X tiles.
 // beta and decay (head_scalars) of TOK tokens x HEADS heads of a workgroup:
 // wave 0's threads form the betas, wave 1's the decays, so the two serial
 // evaluations of the reference's transcendentals run side by side.  The
@@ -544,6 +531,19 @@ constexpr int kAbSplit = 4;
 constexpr int kAbHeads = kNH / kAbSplit;  // heads per a/b workgroup
 static_assert(kNH % kAbSplit == 0 && (2 * kAbHeads * kH) % (4 * kT) == 0 && 2 * kAbHeads <= kT,
               "whole heads per a/b workgroup, whole 16-byte row pieces per thread");
+// Per stream: the residual add (or embedding import), the RMSNorm in chunk
+// order (gdn_rmsnorm_rows_bf16 / gdn_residual_rmsnorm_bf16,
+// gdn_model.cpp:1394-1474, :3351-3450) and, before an attention block, the
+// tiny a/b rows and beta/decay (gdn_gemv_tiny_ab :1501-1536, :2461-2465).
+// Thread t holds elements 8t..8t+7; a 16-element chunk is the sequential sum
+// of thread 2c's eight squares continued by thread 2c + 1.  SPLITS partial
+// sums of the preceding projection are added in split order (1: its rounded
+// sums as BF16 bits; 0: no residual add; EMBED: the embedding row instead).
+// Without AB one workgroup per stream updates the residual in place.  With AB, grid (streams, kAbSplit):
+// workgroup j repeats the norm and runs the a/b rows of heads
+// kNH / kAbSplit * j .. (a 32 KB slice of the 128 KB of rows, requested
+// before the norm's first wait on memory); workgroup 0 alone writes the
+// residual, to h_out != h_in, and the X tiles.
 template <int SPLITS, bool EMBED, bool AB>
 __global__ __launch_bounds__(kT) void k_bnorm(BNorm p) {
     constexpr int ABR = 2 * kAbHeads;  // a/b rows per workgroup: a rows, then b rows
@@ -944,21 +944,22 @@ __global__ __launch_bounds__(kT, 2) void k_brecur(const float *__restrict__ qkv,
 
 // ---------------------------------------------------------------- prefill
 //
-// A prompt runs through one stream's state in chunks of up to 64 tokens, the
+// A prompt runs through one stream's state in segments, layer by layer, the
 // tokens taking the place of the streams: each layer's projections take the
-// whole chunk (the same GEMMs and reduction order as the step), the causal
-// conv reads its taps from the neighbouring tokens of the chunk, and one
-// workgroup per head runs the recurrence over the chunk's tokens in order
-// with the state held in registers.  Every token sees the arithmetic of a
-// multi-stream step, so a prefill of n tokens equals n steps bit for bit.
+// whole segment (the step's sums in the step's order, see "prefill
+// projections"), the causal conv reads its taps from the neighbouring tokens,
+// and the recurrence runs over the segment's tokens in one launch, in order
+// with the state in registers (k_pscan) or in the chunked form (k_wy_seq).  In
+// order, every token sees the arithmetic of a multi-stream step, so a prefill
+// of n tokens equals n steps bit for bit.
 
 // The causal conv of one 64-channel block over 64 tokens of a segment of n:
 // grid (4 kH / 64, ceil(n / 64)), with B16 (3 kH / 64, ..), the gate left to
-// k_bonorm; thread 16 r + j on channels 4 j .. 4 j + 3
-// of the block and tokens r, r + 16, r + 32, r + 48 (16-byte loads and
-// stores; the four loads in flight together).  raw is [n][4 kH]: the
-// unrounded q, k, v, g sums, or (B16) their roundings R(raw); the tails are the prefilled stream's for this
-// layer, [q,k,v][3 oldest..newest][kH].  Token m's window is (s[m], s[m+1],
+// k_bonorm; thread 16 r + j on channels 4 j .. 4 j + 3 of the block and tokens
+// r, r + 16, r + 32, r + 48 (16-byte loads and stores; the four loads in
+// flight together).  raw is [n][4 kH]: the unrounded q, k, v, g sums, or (B16)
+// their roundings R(raw); the tails are the prefilled stream's for this layer,
+// [q,k,v][3 oldest..newest][kH].  Token m's window is (s[m], s[m+1],
 // s[m+2]) and its input s[m+3] in the sequence s = tails ++ R(raw[0..n));
 // the new tails are s[n], s[n+1], s[n+2].  Only the first token block reads
 // the old tails, and it writes the new ones after that read.
@@ -1059,9 +1060,8 @@ __global__ __launch_bounds__(kConvT) void k_pconv(const void *__restrict__ raw, 
 }
 
 // Per (head, token): the q/k L2 norms and alpha of the recurrence, in the
-// batch-1 tree order, for tokens kQkTok y .. +
-// kQkTok - 1 of n, their loads requested together (a token past n re-reads
-// token n - 1, unused).
+// batch-1 tree order, for tokens kQkTok y .. + kQkTok - 1 of n, their loads
+// requested together (a token past n re-reads token n - 1, unused).
 constexpr int kQkTok = 4;
 __global__ __launch_bounds__(kT) void k_pqk(const float *__restrict__ qkv, int n, float *__restrict__ qn_out,
                                             float *__restrict__ kn_out, float *__restrict__ alpha_out) {
@@ -1443,9 +1443,10 @@ __global__ __launch_bounds__(kT) void k_wy_prep(const float *__restrict__ qkv_se
 // 4200 cycles a chunk), and the issue of the operand loads (about 1700: 128 KB
 // per CU and chunk against a SIMD's limit of some 16 loads in flight); with
 // the Q products, or two thirds of the state products, left out it ran only
-// 10 % shorter.  At 4096 tokens a launch takes 180 us (2.8 us a chunk), 192
-// with the o path on the same four waves, and 520 (8.0) in FP32 MFMAs with the
-// state and operands through LDS and seven barriers a chunk.
+// 10 % shorter.  At 4096 tokens a launch takes 180 to 190 us on different
+// boxes (2.8 to 3.0 us a chunk); where it took 180, the o path on the same four
+// waves took 192, and FP32 MFMAs with the state and operands through LDS and
+// seven barriers a chunk 520 (8.0 a chunk).
 constexpr int kWyCols = 16;
 constexpr int kWyTok = kMaxB + 8;  // padded token stride of b and delta (BF16)
 constexpr int kWyWaves = 8;
@@ -2186,9 +2187,11 @@ struct GDNBatchEngine {
     int *p_tok = nullptr;
     int prefill_mode = GDN_PREFILL_SCAN;
     // prefill segment buffers, allocated at the first prefill for seg_cap
-    // tokens (per token: residual ping-pong, projection sums, q/k/v, gate,
-    // sigmoid(gate), beta/decay, attention output, normalised q/k, alpha,
-    // the chunk matrices L and Mq, final hidden; X tiles of three widths)
+    // tokens (per token: residual ping-pong, projection sums, q/k/v,
+    // beta/decay, attention output, alpha, the norms' copy; X tiles of three
+    // widths; gate and sigmoid(gate) for kStepTok tokens).  s_wy, the chunked
+    // mode's operands, shares its memory with s_qn and s_kn, the scan's
+    // normalised q and k
     int seg_tokens = kSegDefault, seg_cap = 0;
     void *seg_mem = nullptr;
     float *s_h = nullptr, *s_y = nullptr, *s_qkv = nullptr, *s_gate = nullptr, *s_sgate = nullptr, *s_bd = nullptr,
@@ -2629,16 +2632,8 @@ BNorm seg_norm(GDNBatchEngine *e, const float *y, const float *w, uint16_t *x_ou
     return p;
 }
 
-// One prefill segment of n tokens (already in s_tok[0..n)) through stream
-// `slot`'s state, layer by layer: the step's kernels with the tokens as the
-// streams (k_pgemm / k_pgu in place of the step's GEMMs, k_bnorm + k_pab in
-// place of the split a/b norm; same sums), the conv across the segment
-// (k_pconv), and the recurrence chunk by chunk of 64 tokens, in token order
-// (k_pqk, k_pscan) or in the WY form (k_wy_prep over every chunk at once,
-// then k_wy_seq over the chunks in order).
 // The prefill's projections over n tokens (X in 64-token tile blocks, padded
-// to whole 128-token tiles), on the kernel that is fastest at that size; every
-// choice forms the same sums.
+// to whole 128-token tiles), by a rule on n; every choice forms the same sums.
 enum PRoute {
     P_STEP,        // the decode step's kernels, a grid plane per 64-token block
     P_TILE,        // k_pgemm / k_pgu, 128 tokens per workgroup (q/k/v/g, gate/up)
@@ -2646,25 +2641,29 @@ enum PRoute {
     P_WIDE,        // k_pgemm_a / k_pgu_a, 256 rows x 128 tokens per workgroup
     P_WIDE_PLANES  // k_pgemm_a with a workgroup per split (down)
 };
-// Where the lines lie, us per launch (the step's kernels re-read the weights
-// per 64 tokens; the others leave CUs idle on short segments):
-//   tokens                   64  256  512  768 1024 1536 2048 2560 3072 4096
-//   q/k/v/g  step            12   28   49    -   91    -  174    -    -    -
-//            tile            30   30   32   42   42    -   79    -    -    -
-//            wide             -    -    -    -   34   56   66   89   96  128
-//   o_proj   step             5    9   15    -   26    -   49    -    -    -
-//            planes          11   11   13   18   20   29   38   46   54   69
-//            wide             -    -   33   33   34   35   37   38   39   41
-//   down     step             9   18   30    -   54    -  103    -    -    -
-//            planes          20   20   23   34   38   55   71   87  102  135
-//            wide planes      -    -   26   26   33   54   58   77   82  113
-//            wide             -    -   78   77   80   80   84   85   85   90
-//   gate/up  step            15   33   57    -  107    -  207    -    -    -
-//            tile            30   31   45   63   81  120  151    -    -  280
-//            wide             -    -   42    -   73    -  109  144  179  219
-// and the norm that reads four planes in place of one sum costs more: 8.3
-// against 6.8 at 512 tokens, 12.6 / 9.7 at 1024, 19 / 13 at 1536, 25 / 18 at
-// 2048, 30 / 21 at 2560, 37 / 24 at 3072.
+// Where the lines lie, us per launch with the weights in cache, the stores as
+// the engine takes them (the step's kernels re-read the weights per 64 tokens;
+// the others leave CUs idle on short segments).  At 64 tokens, in a prefill:
+// q/k/v/g step 12, tile 30; o_proj 5 / planes 11; down 9 / 20; gate/up 15 / 30.
+//   tokens         256 384 512 640 768 896 1024 1152 1280 1408 1536 2048 2560 3072 4096
+//   q/k/v/g  step   27  39  51  62  74  84   96  107  118  129  141  186    -    -    -
+//            tile   25  27  28  43  44  45   47   63   64   66   67   87  110  131  173
+//            wide   27  28  31  31  33  34   35   57   56   59   60   65   92   98  141
+//   o_proj   step    9  12  15  19  22  25   28   32   35   37   40   53    -    -    -
+//            planes 11  12  14  18  19  19   20   26   27   27   28   35   43   49   63
+//            wide   30  31  31  32  32  32   32   33   34   34   34   36   37   39   41
+//   down     step   17  24  31  36  43  50   57   62   69   76   83  110    -    -    -
+//            planes 21  23  25  34  35  36   38   51   52   54   55   68   85   98  127
+//       wide planes 21  23  25  26  27  28   29   45   46   47   49   53   75   77   97
+//            wide   67  67  68  69  70  70   70   71   72   72   73   76   79   82   88
+//   gate/up  step   29  41  54  66  78  91  103  116  128  140  152  202    -    -    -
+//            tile   31  44  46  64  68  83   86  102  105  121  124  162  199  237  313
+//            wide   40  40  41  42  70  75   78   76   78   79  108  115  150  182  222
+// The lines were drawn from fewer sizes than these; what the table would move
+// (wide for q/k/v/g from 640 tokens and gate/up at 896, wide planes for down at
+// 1025 to 1280) is 5 to 12 us a launch.  A norm behind four planes costs more
+// than behind one sum: 8.3 against 6.8 us at 512 tokens, 12.6 / 9.7 at 1024,
+// 19 / 13 at 1536, 25 / 18 at 2048, 30 / 21 at 2560, 37 / 24 at 3072.
 int p_tiles(int n) { return (n + kPgTok - 1) / kPgTok; }
 bool pa_fills(int rows, int n) { return rows % kPaRows == 0 && (rows / kPaRows) * p_tiles(n) >= 256; }
 PRoute route_qkvg(int rows, int n) { return n <= kStepTok ? P_STEP : pa_fills(rows, n) ? P_WIDE : P_TILE; }
@@ -2745,6 +2744,13 @@ void launch_p_norm(const BNorm &p, int planes, int n, hipStream_t s) {
         hipLaunchKernelGGL((k_bnorm<kSplitO, false, false>), dim3(n), dim3(kT), 0, s, p);
 }
 
+// One prefill segment of n tokens (already in s_tok[0..n)) through stream
+// `slot`'s state, layer by layer: the step's kernels with the tokens as the
+// streams (the projections by route, k_bnorm + k_pab in place of the split
+// a/b norm; same sums), the conv across the segment (k_pconv), and the
+// recurrence over all its tokens: in token order (k_pqk, k_pscan) or in the WY
+// form (k_wy_prep over every 64-token chunk at once, then k_wy_seq over the
+// chunks in order).
 void enqueue_prefill_segment(GDNBatchEngine *e, int slot, int n, bool last, hipStream_t s) {
     const int blocks = (n + kMaxB - 1) / kMaxB;
     const int pab_blocks = (n + kPabTok - 1) / kPabTok;

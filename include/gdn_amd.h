@@ -530,11 +530,11 @@ int gdn_batch_save_stream_state(const GDNBatchState *state, uint32_t stream, flo
  * :325-330),
  * in segments of up to 4096 tokens (gdn_batch_set_prefill_segment), each
  * layer by layer: token-parallel projections as GEMMs on the matrix cores,
- * the causal conv across the segment, and the recurrence over chunks of 64
- * tokens -- by default in token order with the state held on chip, so
- * results equal the steps bit for bit; in GDN_PREFILL_CHUNKED mode in the
- * chunk-parallel (WY) form of the gated delta rule (chunk.py:616-686), equal
- * to the steps within FP32 re-association.  *seed_token (may be NULL)
+ * the causal conv across the segment, and the recurrence over its tokens --
+ * by default in token order with the state held on chip, so results equal
+ * the steps bit for bit; in GDN_PREFILL_CHUNKED mode over chunks of 64 tokens
+ * in the chunk-parallel (WY) form of the gated delta rule (chunk.py:616-686),
+ * equal to the steps within FP32 re-association.  *seed_token (may be NULL)
  * receives the argmax of the last position; that position's logits and final
  * hidden vector become the stream's readable ones.  Other streams' states
  * are untouched.  The first prefill allocates the segment's buffers (about
